@@ -55,6 +55,17 @@ __device__ __forceinline__ uint16_t f32_to_bf16_out(float f) {
     return static_cast<uint16_t>((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 
+// Two output elements at once, as packed BF16 codes (low half first): the same codes as
+// f32_to_bf16_out.  v_cvt_pk_bf16_f32 rounds to nearest even; a NaN of either sign is then
+// replaced by 0xffc0.
+__device__ __forceinline__ uint32_t f32x2_to_bf16_out(float lo, float hi) {
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    typedef __bf16 b16x2_t __attribute__((ext_vector_type(2)));
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, b16x2_t));
+    const uint32_t wl = lo != lo ? 0xffc0u : (w & 0xffffu);
+    return hi != hi ? (wl | 0xffc00000u) : (wl | (w & 0xffff0000u));
+}
+
 // double -> f32 (RNE) -> BF16 (RNE): the reference's f32_to_bf16 path
 // (pyfiles/gqa_reference.py:15-19).
 __device__ __forceinline__ uint16_t f64_to_bf16_via_f32(double d) {

@@ -190,6 +190,15 @@ __device__ __forceinline__ uint32_t pk_f16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, h);
 }
 
+// A double rounded to fp32, opaque to the compiler: it merges the conversion with a following
+// one to fp16 into a double -> fp16 conversion, which gfx950 does not have and which it
+// expands to about 40 instructions (one v_cvt_f32_f64 and half a v_cvt_pk_f16_f32 here).
+__device__ __forceinline__ float f32_of(double x) {
+    float f = static_cast<float>(x);
+    asm("" : "+v"(f));
+    return f;
+}
+
 __device__ __forceinline__ float f16_lo(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2_t, w)[0]); }
 __device__ __forceinline__ float f16_hi(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2_t, w)[1]); }
 
@@ -831,28 +840,6 @@ __device__ __forceinline__ bool pf_flag_row(const PrefillArgs& a, int b, int kvh
     const uint4 q3 = *reinterpret_cast<const uint4*>(qrow + kPairs + 32 + 8 * g);
     const uint32_t k0 = max(a.rs_kc[ec * 8 + g], a.rs_kpre[er * 8 + g]);
     const uint32_t k1 = max(a.rs_kc[ec * 8 + 4 + g], a.rs_kpre[er * 8 + 4 + g]);
-    double ss = 0.0, mn2 = INFINITY;
-    float mnx = INFINITY;
-    bool bad = forced, vinf = false;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-        const uint4 dc = *reinterpret_cast<const uint4*>(a.rs_dc + ec * kD + 16 * dt + 4 * g);
-        const uint2 dp = *reinterpret_cast<const uint2*>(a.rs_dpre + er * kD + 16 * dt + 4 * g);
-        const uint32_t d[4] = {max(dc.x, dp.x & 0xffffu), max(dc.y, dp.x >> 16), max(dc.z, dp.y & 0xffffu),
-                               max(dc.w, dp.y >> 16)};
-        const uint32_t xs[4] = {pk[dt].x << 16, pk[dt].x & 0xffff0000u, pk[dt].y << 16, pk[dt].y & 0xffff0000u};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float x = __uint_as_float(xs[i]);
-            const float dv = __uint_as_float(d[i] << 16);
-            const double y = dv > 0.f ? static_cast<double>(x) * __builtin_amdgcn_rcp(static_cast<double>(dv)) : 0.0;
-            ss = fma(y, y, ss);
-            if (dv > 0.f) mn2 = fmin(mn2, y * y);
-            mnx = fminf(mnx, fabsf(x));
-            bad |= !__builtin_isfinite(x);
-            vinf |= !(dv <= 3.4028235e38f);         // an infinite or NaN V among the row's keys
-        }
-    }
     float qq0 = 0.f, qq1 = 0.f;
     {
         const uint32_t w0[8] = {q0.x, q0.y, q0.z, q0.w, q2.x, q2.y, q2.z, q2.w};
@@ -864,41 +851,92 @@ __device__ __forceinline__ bool pf_flag_row(const PrefillArgs& a, int b, int kvh
         }
     }
     float e = sqrtf(qq0) * sqrtf(__uint_as_float(k0)) + sqrtf(qq1) * sqrtf(__uint_as_float(k1));
+    // Element magnitudes as packed codes: the largest (infinity and NaN above every finite
+    // one) and the smallest; and the D_j, the largest of them likewise.
+    uint32_t d[8][4], d_max = 0u, x_max = 0u, x_min = 0x7fff7fffu;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+        const uint4 dc = *reinterpret_cast<const uint4*>(a.rs_dc + ec * kD + 16 * dt + 4 * g);
+        const uint2 dp = *reinterpret_cast<const uint2*>(a.rs_dpre + er * kD + 16 * dt + 4 * g);
+        d[dt][0] = max(dc.x, dp.x & 0xffffu);
+        d[dt][1] = max(dc.y, dp.x >> 16);
+        d[dt][2] = max(dc.z, dp.y & 0xffffu);
+        d[dt][3] = max(dc.w, dp.y >> 16);
+        d_max = max(d_max, max(max(d[dt][0], d[dt][1]), max(d[dt][2], d[dt][3])));
+        const uint32_t m0 = pk[dt].x & 0x7fff7fffu, m1 = pk[dt].y & 0x7fff7fffu;
+        x_max = pk_max_u16(x_max, pk_max_u16(m0, m1));
+        x_min = pk_min_u16(x_min, pk_min_u16(m0, m1));
+    }
+    auto elem = [&](int dt, int i) {
+        const uint32_t w = i < 2 ? pk[dt].x : pk[dt].y;
+        return __uint_as_float((i & 1) ? w & 0xffff0000u : w << 16);
+    };
+    // A first decision in fp32: y and its squares lose range there (an element 2^63 below its
+    // D_j squares to zero, a subnormal D_j has no reciprocal), but only towards "cannot tell"
+    // -- a zero minimum, an infinite or NaN sum -- and its relative error is far below the 1 %
+    // margin, so a row it clears is clear.  About 1 % of the N(0,1) waves hold a row that it
+    // does not clear and form the decision in double below.  (The double version for every
+    // wave cost about 2 us at the end of each workgroup.)
+    float ss32 = 0.f, mn32 = INFINITY;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float y = elem(dt, i) * __builtin_amdgcn_rcpf(__uint_as_float(d[dt][i] << 16));
+            ss32 = fmaf(y, y, ss32);
+            mn32 = fminf(mn32, y * y);
+        }
     // the row's four lanes: n, n + 16, n + 32, n + 48
-    ss += __shfl_xor(ss, 16);
-    ss += __shfl_xor(ss, 32);
     e += __shfl_xor(e, 16);
     e += __shfl_xor(e, 32);
-    mn2 = fmin(mn2, __shfl_xor(mn2, 16));
-    mn2 = fmin(mn2, __shfl_xor(mn2, 32));
-    mnx = fminf(mnx, __shfl_xor(mnx, 16));
-    mnx = fminf(mnx, __shfl_xor(mnx, 32));
-    bad |= static_cast<double>(mnx) < 8.0 * ul;
-    bad = (__shfl_xor(static_cast<int>(bad), 16) | __shfl_xor(static_cast<int>(bad), 32) |
-           __shfl_xor(static_cast<int>(bad), 48) | static_cast<int>(bad)) != 0;
-    vinf = (__shfl_xor(static_cast<int>(vinf), 16) | __shfl_xor(static_cast<int>(vinf), 32) |
-            __shfl_xor(static_cast<int>(vinf), 48) | static_cast<int>(vinf)) != 0;
-    if (vinf && (lane >> 4) == 0) atomicOr(a.rs_hdr + 2, 1u);   // the row is flagged: y = 0 there
-    return bad || rs_flag_decide(mn2, ss, static_cast<double>(m), static_cast<double>(e) * fabs(a.qk_scale_log2));
+    ss32 += __shfl_xor(ss32, 16);
+    ss32 += __shfl_xor(ss32, 32);
+    mn32 = swap32_max(swap16_max(-mn32));
+    x_max = pk_max_u16(x_max, static_cast<uint32_t>(__shfl_xor(static_cast<int>(x_max), 16)));
+    x_max = pk_max_u16(x_max, static_cast<uint32_t>(__shfl_xor(static_cast<int>(x_max), 32)));
+    x_min = pk_min_u16(x_min, static_cast<uint32_t>(__shfl_xor(static_cast<int>(x_min), 16)));
+    x_min = pk_min_u16(x_min, static_cast<uint32_t>(__shfl_xor(static_cast<int>(x_min), 32)));
+    d_max = max(d_max, static_cast<uint32_t>(__shfl_xor(static_cast<int>(d_max), 16)));
+    d_max = max(d_max, static_cast<uint32_t>(__shfl_xor(static_cast<int>(d_max), 32)));
+    const float mnx = __uint_as_float(min(x_min & 0xffffu, x_min >> 16) << 16);
+    const bool bad = forced || max(x_max & 0xffffu, x_max >> 16) >= 0x7f80u ||
+                     static_cast<double>(mnx) < 8.0 * ul;
+    // an infinite or NaN V among the row's keys (its y is 0: the row is flagged)
+    if (d_max >= 0x7f80u && (lane >> 4) == 0) atomicOr(a.rs_hdr + 2, 1u);
+    const double ed = static_cast<double>(e) * fabs(a.qk_scale_log2);
+    const double md = static_cast<double>(m);
+    bool flagged = bad || rs_flag_decide(-static_cast<double>(mn32), 1.01 * static_cast<double>(ss32), md, ed);
+    if (__ballot(flagged && !bad)) {
+        double ss = 0.0, mn2 = INFINITY;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float dv = __uint_as_float(d[dt][i] << 16);
+                const double y =
+                    dv > 0.f ? static_cast<double>(elem(dt, i)) * __builtin_amdgcn_rcp(static_cast<double>(dv)) : 0.0;
+                ss = fma(y, y, ss);
+                if (dv > 0.f) mn2 = fmin(mn2, y * y);
+            }
+        ss += __shfl_xor(ss, 16);
+        ss += __shfl_xor(ss, 32);
+        mn2 = fmin(mn2, __shfl_xor(mn2, 16));
+        mn2 = fmin(mn2, __shfl_xor(mn2, 32));
+        flagged = bad || rs_flag_decide(mn2, ss, md, ed);
+    }
+    return flagged;
 }
 
 __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsB];
 
     // Workgroup -> (sequence, KV head, query block).  Workgroups are dealt to the 8 XCDs
-    // round-robin; when the (sequence, KV head) pairs divide evenly, all query blocks of
-    // a pair go to one XCD so that its K/V blocks are shared in that XCD's L2.
-    const int n_pairs = a.batch * kHkv;
-    const int id = blockIdx.x;
-    int pair, qb;
-    if (n_pairs % 8 == 0) {
-        const int k = id >> 3;
-        qb = k % a.n_qblk;
-        pair = (k / a.n_qblk) * 8 + (id & 7);
-    } else {
-        pair = id / a.n_qblk;
-        qb = id % a.n_qblk;
-    }
+    // round-robin; all query blocks of a pair (8 per sequence) go to one XCD so that its K/V
+    // blocks are shared in that XCD's L2.  A pair's query blocks are dealt last first: the
+    // last ones see the most keys, and the short ones then fill the CUs that finish early.
+    const int k_id = blockIdx.x >> 3;
+    const int qb = a.n_qblk - 1 - k_id % a.n_qblk;
+    const int pair = (k_id / a.n_qblk) * 8 + (blockIdx.x & 7);
     const int b = pair / kHkv;
     const int kvh = pair % kHkv;
     const int tid = threadIdx.x;
@@ -959,6 +997,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
                                          (lds_void_t*)(lds + kOffSw + 4 * (first & (kSwRing - 1))), 4, 0, 0);
     };
     issue_sw(64 * wave);
+    // The first scale words again, for their maximum below (requested with the rest).
+    constexpr int kSwAhead = 3;
+    uint32_t sw_ahead[kSwAhead];
+#pragma unroll
+    for (int i = 0; i < kSwAhead; ++i) sw_ahead[i] = sw[min(i * kWave + lane, nblk_stg - 1)];
     auto sw_at = [&](int blk) {
         return __builtin_amdgcn_readfirstlane(
             *reinterpret_cast<const uint32_t*>(lds + kOffSw + 4 * (blk & (kSwRing - 1))));
@@ -970,37 +1013,50 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     float cq;                               // 2^-sq
     bool q_bad = false;
     {
-        const uint16_t* qrow = a.q + ((static_cast<int64_t>(b) * T + tq_c) * kHq + hq) * kD;
-        // Every load first (the rotation below branches inside sincos, and each branch would
-        // otherwise wait for all memory in flight, the K/V copies included).
-        uint16_t qx[2][8], qy[2][8];
-        double fr[2][8];
+        const int64_t tok = static_cast<int64_t>(b) * T + tq_c;
+        const char* qrow = reinterpret_cast<const char*>(a.q + (tok * kHq + hq) * kD) + 16 * g;
+        // The token's (cos, sin) row, from the append kernel: rotating here (16 double sincos
+        // per lane) took about 20 us at the start of every workgroup.
+        const double2* csr = a.rs_cs + tok * kPairs + 8 * g;
+        uint4 qw[4];
+        double2 cs[2][8];
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < 4; ++kb) qw[kb] = *reinterpret_cast<const uint4*>(qrow + 64 * kb);
+        if (a.flags & 1u) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int d = 32 * kb + 8 * g + j;
-                qx[kb][j] = qrow[d];
-                qy[kb][j] = qrow[d + kPairs];
-                fr[kb][j] = a.rope.inv_freq[d];
-            }
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) cs[kb][j] = csr[32 * kb + j];
+        }
+        float qf[4][8];
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) unpack8(qw[kb], qf[kb]);
         double qv[4][8];
         double mx = 0.0;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const double x = bf16_to_f32(qx[kb][j]);
-                const double y = bf16_to_f32(qy[kb][j]);
+                const double x = qf[kb][j];
+                const double y = qf[kb + 2][j];
                 double xr = x, yr = y;
-                if (a.flags & 1u) rope_pair(x, y, pos_n, fr[kb][j], xr, yr);
+                if (a.flags & 1u) {
+                    xr = x * cs[kb][j].x - y * cs[kb][j].y;
+                    yr = x * cs[kb][j].y + y * cs[kb][j].x;
+                }
                 qv[kb][j] = xr * a.qk_scale_log2;
                 qv[kb + 2][j] = yr * a.qk_scale_log2;
-                // NaN fails both comparisons
-                if (!(fabs(qv[kb][j]) <= 1e300) || !(fabs(qv[kb + 2][j]) <= 1e300)) q_bad = true;
                 mx = fmax(mx, fmax(fabs(qv[kb][j]), fabs(qv[kb + 2][j])));
             }
         }
+        // Out of range: an element that is not finite as given, or a rotated and scaled one
+        // past 1e300 (finite elements rotate and scale without a NaN).
+        uint32_t qm = 0u;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+            qm = pk_max_u16(qm, pk_max_u16(pk_max_u16(qw[kb].x & 0x7fff7fffu, qw[kb].y & 0x7fff7fffu),
+                                           pk_max_u16(qw[kb].z & 0x7fff7fffu, qw[kb].w & 0x7fff7fffu)));
+        if (max(qm & 0xffffu, qm >> 16) >= 0x7f80u || !(mx <= 1e300)) q_bad = true;
         mx = fmax(mx, __shfl_xor(mx, 16));
         mx = fmax(mx, __shfl_xor(mx, 32));
         int e = 0;
@@ -1017,14 +1073,9 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const double x0 = ldexp(qv[kb][2 * j], sq), x1 = ldexp(qv[kb][2 * j + 1], sq);
-                const _Float16 h0 = static_cast<_Float16>(static_cast<float>(x0));
-                const _Float16 h1 = static_cast<_Float16>(static_cast<float>(x1));
-                f16x2_t hh;
-                hh[0] = h0;
-                hh[1] = h1;
-                w0[j] = __builtin_bit_cast(uint32_t, hh);
-                w1[j] = pk_f16(static_cast<float>(x0 - static_cast<double>(h0)),
-                               static_cast<float>(x1 - static_cast<double>(h1)));
+                w0[j] = pk_f16(f32_of(x0), f32_of(x1));
+                w1[j] = pk_f16(f32_of(x0 - static_cast<double>(f16_lo(w0[j]))),
+                               f32_of(x1 - static_cast<double>(f16_hi(w0[j]))));
             }
             // Pin the operands: without this the compiler re-derives them from the double
             // rows inside the block loop to save registers.
@@ -1052,11 +1103,12 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     tl.u = 0.f;
     // The open group: blocks summed into tl.acc so far and their V scale exponent.  A block
     // whose V scale differs from the group's by more than 3 (its P would leave fp16's range
-    // or its precision) closes the group first.  A block holding chunk keys is summed alone:
-    // its scales depend on rows that later tokens see and this token does not, and within a
-    // group a different scale would change how the other blocks' terms round, so this
-    // token's output would depend on keys its mask hides.  Alone, its sum only scales by a
-    // power of two.
+    // or its precision) closes the group first.  A block with keys past the wave's first
+    // query is summed alone: its scales depend on rows that later tokens see and this token
+    // does not, and within a group a different scale would change how the other blocks'
+    // terms round, so this token's output would depend on keys its mask hides.  Alone, its
+    // sum only scales by a power of two.  (Blocks of chunk keys that every query of the wave
+    // sees join groups like cached ones.)
     int grp_n = 0, grp_sv = 0;
 
     // Raw scores carry 2^(sq + sk): mult = 2^-sq * 2^-sk(block) turns them into log2 units.
@@ -1068,7 +1120,10 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     auto blk_sv = [&](uint32_t w) { return static_cast<int>(static_cast<int8_t>((w >> 8) & 0xffu)); };
     // The largest V scale exponent among this workgroup's blocks (the smallest-V block's).
     int sv_hi = -128;
-    for (int j = lane; j < n_blk; j += kWave) sv_hi = max(sv_hi, blk_sv(sw[j]));
+#pragma unroll
+    for (int i = 0; i < kSwAhead; ++i)
+        if (i * kWave + lane < n_blk) sv_hi = max(sv_hi, blk_sv(sw_ahead[i]));
+    for (int j = kSwAhead * kWave + lane; j < n_blk; j += kWave) sv_hi = max(sv_hi, blk_sv(sw[j]));
 #pragma unroll
     for (int sh = 1; sh < kWave; sh <<= 1) sv_hi = max(sv_hi, __shfl_xor(sv_hi, sh));
     sv_hi = __builtin_amdgcn_readfirstlane(sv_hi);
@@ -1103,7 +1158,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
         unsafe |= w_next;
 
         const int sv = blk_sv(w_cur);
-        const bool solo = blk_new(blk);
+        const bool solo = blk_diag(blk);
         if (grp_n == kPfGroup || (grp_n > 0 && (solo || abs(grp_sv - sv) > 3))) {
             pf_flush(tl, static_cast<double>(pow2f(-grp_sv)));
             grp_n = 0;
@@ -1170,21 +1225,20 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     u += __shfl_xor(u, 32);
     const double ul = static_cast<double>(u) / l;     // bound on that error in the row's elements
     // The row of query n: lanes n, n+16, n+32, n+48 hold dims 16dt + 4g ..
+    const double inv_l = 1.0 / l;
     double x[8][4];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[dt][i] = tl.o64[dt][i] / l;
+        for (int i = 0; i < 4; ++i) x[dt][i] = tl.o64[dt][i] * inv_l;
     const bool q_bad_row = __shfl_xor(static_cast<int>(q_bad), 16) | __shfl_xor(static_cast<int>(q_bad), 32) |
                            __shfl_xor(static_cast<int>(q_bad), 48) | static_cast<int>(q_bad);
     const int64_t row = (static_cast<int64_t>(b) * T + tq_c) * kHq + hq;
     uint2 pk[8];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
-        pk[dt].x = f32_to_bf16_out(static_cast<float>(x[dt][0])) |
-                   (static_cast<uint32_t>(f32_to_bf16_out(static_cast<float>(x[dt][1]))) << 16);
-        pk[dt].y = f32_to_bf16_out(static_cast<float>(x[dt][2])) |
-                   (static_cast<uint32_t>(f32_to_bf16_out(static_cast<float>(x[dt][3]))) << 16);
+        pk[dt].x = f32x2_to_bf16_out(static_cast<float>(x[dt][0]), static_cast<float>(x[dt][1]));
+        pk[dt].y = f32x2_to_bf16_out(static_cast<float>(x[dt][2]), static_cast<float>(x[dt][3]));
     }
     // The rescore flag, decided here from the rounded row: rows that read a marked block or
     // whose Q row is out of range always go to the rescore.  Waves past the last query (q_ok
