@@ -56,6 +56,8 @@
 //
 // Chunks of at most 16 new tokens take the multi-token decode path instead
 // (gqa_multitoken.hip), which shares this file's LDS row layout (gqa_prefill_common.h).
+#include <type_traits>
+
 #include "gqa_device.h"
 #include "gqa_internal.h"
 #include "gqa_prefill_common.h"
@@ -558,16 +560,15 @@ hipError_t launch_prefill_stage(const PrefillArgs& a, hipStream_t stream) {
 // straight into LDS (global_load_lds_dwordx4: lane l of an instruction writes bytes
 // [16l, 16l + 16) of a 1 KB stretch = 4 rows), so a row's 16 16-byte chunks are placed by
 // choosing which chunk each lane fetches: chunk c of row r sits at position c ^ pf_swz(r & 15).
-// With that swizzle the K operand reads (16 rows, one chunk) and the V^T transpose reads
-// (16 rows, two chunks) hit 64 distinct banks per pass, and because it depends on r & 15 only,
-// the rows 16 apart that one lane reads differ by a constant offset.
+// With that swizzle the K operand and V^T transpose reads hit no bank twice, and because it
+// depends on r & 15 only, the rows 16 apart that one lane reads differ by a constant offset.
 constexpr int kPlaneB = kPfBlk * kRowB;     // 16 KB per plane
 constexpr int kOffK = 0;                    // + buffer * kPlaneB
 constexpr int kOffV = 2 * kPlaneB;
 constexpr int kOffKlo = 4 * kPlaneB;
 // Then a ring of block scale words: words for blocks [0, 512) are copied at the start and
-// words for blocks [256k + 256, 256k + 512) at step 256k, into the half whose blocks are done,
-// so that a word is in LDS 255 steps before it is read.  Copied like the rows (straight into
+// words for blocks [256k + 256, 256k + 512) at step 256k + 128, into the half whose blocks are
+// done, so that a word is in LDS 126 steps before it is read.  Copied like the rows (straight into
 // LDS, completed by the step's vmcnt(0) wait), it costs no wait of its own: a plain load's
 // wait would also wait for the K/V copies in flight.
 constexpr int kOffSw = 6 * kPlaneB;
@@ -586,8 +587,11 @@ __device__ __forceinline__ void pf_copy_offsets(int wave, int lane, uint32_t (&l
     }
 }
 
-// Request one staged 64-row block (16 KB at `src`) into the LDS plane at `dst`.
+// Request one staged 64-row block (16 KB at `src`, uniform) into the LDS plane at `dst`.  The
+// block's address stays a scalar pair and the lane's offset a 32-bit register (the empty asm
+// keeps the compiler from carrying a 64-bit address per lane and plane through the loop).
 __device__ __forceinline__ void pf_issue(const char* src, const uint32_t (&loff)[2], uint8_t* dst, int wave) {
+    asm("" : "+s"(src));
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii)
         __builtin_amdgcn_global_load_lds(src + loff[ii], (lds_void_t*)(dst + (2 * wave + ii) * 1024), 16, 0, 0);
@@ -595,31 +599,35 @@ __device__ __forceinline__ void pf_issue(const char* src, const uint32_t (&loff)
 
 __device__ __forceinline__ f16x8_t as_f16x8(const uint4& w) { return __builtin_bit_cast(f16x8_t, w); }
 
-// 8 fp16 K values of row `row`, bytes [16 chunk, 16 chunk + 16) of the plane at `plane`.
-__device__ __forceinline__ f16x8_t pf_k16(const uint8_t* plane, int row, int chunk) {
-    return *reinterpret_cast<const f16x8_t*>(plane + row * kRowB + 16 * (chunk ^ pf_swz(row)));
+// Lane (g, n)'s byte offset in a K plane of its operand for 16-key tile 0, dims 8g .. 8g+7
+// (slice 0); slice q is that offset ^ 64 q (the chunk index is swizzled by exclusive or),
+// tile kt 4096 kt further.
+__device__ __forceinline__ uint32_t pf_k_offset(int n, int g) { return n * kRowB + 16 * (g ^ pf_swz(n)); }
+
+// K operands of half a 32-dim slice: dims 32 (i / 2) .., 16-key tiles 2 (i % 2) and the next.
+__device__ __forceinline__ void pf_k_pair(const uint8_t* kplane, int i, uint32_t koff, f16x8_t (&ak)[2]) {
+    const uint8_t* p = kplane + (koff ^ (64u * (i >> 1))) + 32 * (i & 1) * kRowB;
+    ak[0] = *reinterpret_cast<const f16x8_t*>(p);
+    ak[1] = *reinterpret_cast<const f16x8_t*>(p + 16 * kRowB);
 }
 
-// One 32-dim slice (dims 32q .. 32q+31) of the scores S^T[key][query] of one 16-query tile
-// over the block's 4 key tiles: the 2 fp16 parts of Q against the K plane, and for chunk
-// keys the trailing part of K against Q's leading part.
+// The scores S^T[key][query] those operands add to: the 2 fp16 parts of Q against the K
+// plane, and for chunk keys the trailing part of K against Q's leading part.
 template <bool kNew>
-__device__ __forceinline__ void pf_qk_slice(const uint8_t* kplane, const f16x8_t (&qop)[2][4], int q, int n,
-                                            int g, f32x4_t (&sacc)[4]) {
-    f16x8_t ak[4];
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt) ak[kt] = pf_k16(kplane, 16 * kt + n, 4 * q + g);
+__device__ __forceinline__ void pf_qk_pair(const uint8_t* kplane, const f16x8_t (&ak)[2], const f16x8_t (&qop)[2][4],
+                                           int i, uint32_t koff, f32x4_t (&sacc)[4]) {
+    const int q = i >> 1, kt = 2 * (i & 1);
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-            sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak[kt], qop[s][q], sacc[kt], 0, 0, 0);
+        for (int e = 0; e < 2; ++e)
+            sacc[kt + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak[e], qop[s][q], sacc[kt + e], 0, 0, 0);
     if (kNew) {
+        f16x8_t al[2];
+        pf_k_pair(kplane + (kOffKlo - kOffK), i, koff, al);
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) ak[kt] = pf_k16(kplane + (kOffKlo - kOffK), 16 * kt + n, 4 * q + g);
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-            sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak[kt], qop[0][q], sacc[kt], 0, 0, 0);
+        for (int e = 0; e < 2; ++e)
+            sacc[kt + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[e], qop[0][q], sacc[kt + e], 0, 0, 0);
     }
 }
 
@@ -646,28 +654,30 @@ __device__ __forceinline__ void pf_flush(PfTile& t, double cv) {
     }
 }
 
-// Running max after a block: masks keys past each query on diagonal blocks, then returns
-// ceil(block max) where that exceeds the running max m (integer-valued, so every rescale is an
-// exact power of two), else m.  `mult` turns the block's raw scores into log2 units.  The two
-// cross-row steps are gfx950 lane swaps (rows 16 and 32 lanes apart), not LDS permutes.
-__device__ __forceinline__ float pf_next_max(f32x4_t (&sacc)[4], bool diag, int key0, int g, int pos_n, float m,
-                                             float mult) {
-    if (diag) {
+// Masks a diagonal block's keys past the query at pos_n.
+__device__ __forceinline__ void pf_mask(f32x4_t (&sacc)[4], int key0, int g, int pos_n) {
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
+    for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (key0 + 16 * kt + 4 * g + i > pos_n) sacc[kt][i] = -INFINITY;
-    }
+        for (int i = 0; i < 4; ++i)
+            if (key0 + 16 * kt + 4 * g + i > pos_n) sacc[kt][i] = -INFINITY;
+}
+
+// Running max after a block, in two steps: the lane's largest raw score, then ceil(block max)
+// where that exceeds the running max m (integer-valued, so every rescale is an exact power of
+// two), else m.  `mult` turns the block's raw scores into log2 units.  The two cross-row steps
+// are gfx950 lane swaps (rows 16 and 32 lanes apart), not LDS permutes.
+__device__ __forceinline__ float pf_lane_max(const f32x4_t (&sacc)[4]) {
     float bmax = -INFINITY;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) bmax = fmaxf(bmax, sacc[kt][i]);
-    const auto x16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(bmax), __float_as_uint(bmax), false, false);
-    bmax = fmaxf(__uint_as_float(x16[0]), __uint_as_float(x16[1]));
-    const auto x32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(bmax), __float_as_uint(bmax), false, false);
-    bmax = fmaxf(__uint_as_float(x32[0]), __uint_as_float(x32[1])) * mult;
+    return bmax;
+}
+
+__device__ __forceinline__ float pf_next_max(float bmax, float m, float mult) {
+    bmax = swap32_max(swap16_max(bmax)) * mult;
     return bmax > m ? ceilf(bmax) : m;
 }
 
@@ -689,25 +699,22 @@ __device__ __forceinline__ void pf_rescale(PfTile& t, float m_new) {
     }
 }
 
-// p = 2^12 * 2^(s - m) of key tile kt (0 for masked keys; s = raw score * mult), summed into
-// lsum and split into two fp16 parts rounded to nearest (p = p1 + p2 to 2^-22 relative),
+// p = 2^12 * 2^(s - m) of half j of key tile kt (keys 4g + 2j, + 1; 0 for masked keys; s = raw
+// score * mult), summed into lsum and split into two fp16 parts rounded to nearest (p = p1 + p2 to 2^-22 relative),
 // packed as the P^T B operand: ph[part][window][dword].
-__device__ __forceinline__ void pf_probs_tile16(const f32x4_t& s, float mult, float off, float& lsum,
-                                                uint32_t (&ph)[2][2][4], int kt) {
-    float p[4];
+__device__ __forceinline__ void pf_probs_half16(const f32x4_t& s, float mult, float off, float& lsum,
+                                                uint32_t (&ph)[2][2][4], int kt, int j) {
+    float p[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 2; ++i) {
         // v_exp_f32: 2^x, 0 for -inf (masked keys); results below 2^-126 flush to 0.
-        p[i] = __builtin_amdgcn_exp2f(fmaf(s[i], mult, off));
+        p[i] = __builtin_amdgcn_exp2f(fmaf(s[2 * j + i], mult, off));
         lsum += p[i];
     }
     const int w = kt >> 1, d0 = (kt & 1) * 2;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const uint32_t h1 = pk_f16(p[2 * j], p[2 * j + 1]);
-        ph[0][w][d0 + j] = h1;
-        ph[1][w][d0 + j] = pk_f16(sub_f16_lo(p[2 * j], h1), sub_f16_hi(p[2 * j + 1], h1));
-    }
+    const uint32_t h1 = pk_f16(p[0], p[1]);
+    ph[0][w][d0 + j] = h1;
+    ph[1][w][d0 + j] = pk_f16(sub_f16_lo(p[0], h1), sub_f16_hi(p[1], h1));
 }
 
 // V^T operands of one 16-dim tile dt for both 32-key windows: lane (g, m) gets keys
@@ -752,31 +759,66 @@ __device__ __forceinline__ f16x8_t pf_vt_operand(const VtPair& v, int w) {
     return u.v;
 }
 
-// Per-lane LDS address of the transpose reads of dim tile dt (V buffer 0, window 0).
-__device__ __forceinline__ uint32_t pf_vt_addr(uint32_t lds_base, int dt, int lane) {
-    return lds_base + kOffV + vt_tr_offset(dt, lane);
+// A step's instructions are laid out in chunks that the scheduler keeps in this order (it may
+// only move instructions inside a chunk): left to itself it hoists the probabilities' VALU
+// work out of the MFMAs it should run beside, and sinks LDS reads to just before their use.
+__device__ __forceinline__ void pf_chunk_end() { __builtin_amdgcn_sched_barrier(0); }
+
+// The scores of the next block from K buffer `kplane` (kNext: there is one; kNew: it holds chunk
+// keys), beside the second half of the current block's probabilities (key tiles 2 and 3: raw
+// scores `scur`; the first half was formed beside the previous block's V^T P^T).  Four
+// chunks, each two K operand pairs (8 MFMAs), the reads of the pairs two on, and half a key
+// tile of probabilities; with kVt the last one also requests the first V^T operands (cur):
+// only where no branch lies between the request and its wait.
+template <bool kNext, bool kNew, bool kVt>
+__device__ __forceinline__ void pf_scores_beside(const f32x4_t (&scur)[4], float mult, float off, float& lsum,
+                                                 const uint8_t* kplane, const f16x8_t (&qop)[2][4], uint32_t koff,
+                                                 uint32_t vaddr, uint32_t (&ph)[2][2][4], f32x4_t (&snext)[4],
+                                                 VtPair (&cur)[2]) {
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) snext[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f16x8_t ak[3][2];
+    if (kNext) {
+        pf_k_pair(kplane, 0, koff, ak[0]);
+        pf_k_pair(kplane, 1, koff, ak[1]);
+        pf_chunk_end();
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if (kNext && i < 6) pf_k_pair(kplane, i + 2, koff, ak[(i + 2) % 3]);
+        if (kVt && i == 7) {
+            // (after the last K operands have arrived: LDS reads complete in order)
+            asm volatile("" : "+v"(ak[1][0]), "+v"(ak[1][1]));
+            cur[0] = pf_vt_issue(vaddr);
+            cur[1] = pf_vt_issue(vaddr ^ 32u);
+        }
+        if (kNext) pf_qk_pair<kNew>(kplane, ak[i % 3], qop, i, koff, snext);
+        if (!(i & 1)) pf_probs_half16(scur[2 + (i >> 2)], mult, off, lsum, ph, 2 + (i >> 2), (i >> 1) & 1);
+        if (kNext && (i & 1)) pf_chunk_end();
+    }
 }
 
 // The group's fp32 sum += the block's V^T P^T: per 16-dim tile, V^T (transpose reads) against
 // the two P parts of both 32-key windows; two tiles at a time, the next two tiles' operands
-// requested before the current two's products.
-__device__ __forceinline__ void pf_pv(const uint32_t (&vaddr)[8], uint32_t voff, const uint32_t (&ph)[2][2][4],
-                                      PfTile& t) {
+// requested before the current two's products (cur: tiles 0 and 1, requested already).
+// vaddr: the lane's transpose-read address of dim tile 0; tile dt is vaddr ^ 32 dt (its chunk
+// index 2 dt is swizzled by exclusive or, and the planes are aligned).  beside(i), i < 4:
+// work to place among the products of tiles 2i and 2i + 1.
+template <class F>
+__device__ __forceinline__ void pf_pv(uint32_t vaddr, const uint32_t (&ph)[2][2][4], VtPair (&cur)[2], PfTile& t,
+                                      F&& beside) {
     f16x8_t pb[2][2];
 #pragma unroll
     for (int w = 0; w < 2; ++w)
 #pragma unroll
         for (int s = 0; s < 2; ++s) pb[w][s] = as_f16x8(make_uint4(ph[s][w][0], ph[s][w][1], ph[s][w][2], ph[s][w][3]));
-    VtPair cur[2];
-    cur[0] = pf_vt_issue(vaddr[0] + voff);
-    cur[1] = pf_vt_issue(vaddr[1] + voff);
 #pragma unroll
     for (int d0 = 0; d0 < 8; d0 += 2) {
         pf_vt_wait(cur[0], cur[1]);
         VtPair nxt[2];
         if (d0 + 2 < 8) {
-            nxt[0] = pf_vt_issue(vaddr[d0 + 2] + voff);
-            nxt[1] = pf_vt_issue(vaddr[d0 + 3] + voff);
+            nxt[0] = pf_vt_issue(vaddr ^ (32u * (d0 + 2)));
+            nxt[1] = pf_vt_issue(vaddr ^ (32u * (d0 + 3)));
         }
 #pragma unroll
         for (int w = 0; w < 2; ++w)
@@ -786,31 +828,13 @@ __device__ __forceinline__ void pf_pv(const uint32_t (&vaddr)[8], uint32_t voff,
                 for (int e = 0; e < 2; ++e)
                     t.acc[d0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf_vt_operand(cur[e], w), pb[w][s],
                                                                            t.acc[d0 + e], 0, 0, 0);
+        beside(d0 >> 1);
+        pf_chunk_end();
         if (d0 + 2 < 8) {
             cur[0] = nxt[0];
             cur[1] = nxt[1];
         }
     }
-}
-
-// Probabilities of the current block (raw scores `scur` times `mult`, running max already
-// grown) interleaved with the scores of the next block from K buffer `kplane` (kNext: there
-// is one; kNew: it holds chunk keys).
-template <bool kNext, bool kNew>
-__device__ __forceinline__ void pf_probs_and_next(const f32x4_t (&scur)[4], float mult, float vshift,
-                                                  const uint8_t* kplane, const f16x8_t (&qop)[2][4], int n, int g,
-                                                  PfTile& t, uint32_t (&ph)[2][2][4], f32x4_t (&snext)[4]) {
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt) snext[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float lsum = 0.f;
-    // p carries 2^vshift more (the group's V scale over this block's, |vshift| <= 3); l does not
-    const float off = static_cast<float>(kPScaleExp) - t.m_run + vshift;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if (kNext) pf_qk_slice<kNew>(kplane, qop, q, n, g, snext);
-        pf_probs_tile16(scur[q], mult, off, lsum, ph, q);
-    }
-    t.l64 += ldexp(static_cast<double>(lsum), -static_cast<int>(vshift));
 }
 
 // The rescore flag of one output row, in the attention kernel's layout: lane (g, n) holds
@@ -1002,9 +1026,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     uint32_t sw_ahead[kSwAhead];
 #pragma unroll
     for (int i = 0; i < kSwAhead; ++i) sw_ahead[i] = sw[min(i * kWave + lane, nblk_stg - 1)];
-    auto sw_at = [&](int blk) {
-        return __builtin_amdgcn_readfirstlane(
-            *reinterpret_cast<const uint32_t*>(lds + kOffSw + 4 * (blk & (kSwRing - 1))));
+    auto sw_lds = [&](int blk) {
+        return *reinterpret_cast<const uint32_t*>(lds + kOffSw + 4 * (blk & (kSwRing - 1)));
     };
 
     // Q operands: query n = this lane's column, dims 32kb + 8g + j, two fp16 parts of Q
@@ -1087,9 +1110,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     }
 
     const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_t*)(lds)));
-    uint32_t vaddr[8];
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) vaddr[dt] = pf_vt_addr(lds_base, dt, lane);
+    const uint32_t vaddr = lds_base + kOffV + vt_tr_offset(0, lane);
+    const uint32_t koff = pf_k_offset(n, g);
 
     PfTile tl;
 #pragma unroll
@@ -1110,6 +1132,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     // sum only scales by a power of two.  (Blocks of chunk keys that every query of the wave
     // sees join groups like cached ones.)
     int grp_n = 0, grp_sv = 0;
+    int shut_sv = 0;                        // a group to close before the next products, its exponent
+    bool shut = false;
 
     // Raw scores carry 2^(sq + sk): mult = 2^-sq * 2^-sk(block) turns them into log2 units.
     // (Kept at least 2^-126: a smaller factor means scores below ~2^-90, all p = 1 either way,
@@ -1134,52 +1158,114 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     f32x4_t scur[4];
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) scur[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    if (blk_new(0)) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) pf_qk_slice<true>(lds + kOffK, qop, q, n, g, scur);
-    } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) pf_qk_slice<false>(lds + kOffK, qop, q, n, g, scur);
+    for (int i = 0; i < 8; ++i) {
+        f16x8_t ak[2];
+        pf_k_pair(lds + kOffK, i, koff, ak);
+        if (blk_new(0))
+            pf_qk_pair<true>(lds + kOffK, ak, qop, i, koff, scur);
+        else
+            pf_qk_pair<false>(lds + kOffK, ak, qop, i, koff, scur);
     }
-    uint32_t w_cur = sw_at(0);
+    uint32_t w_cur = __builtin_amdgcn_readfirstlane(sw_lds(0));
+    uint32_t w_ahead = sw_lds(1);          // block blk+1's word, read a step ahead
     uint32_t unsafe = w_cur;                // bit 31 of any block read marks all rows
     float mult_cur = blk_mult(w_cur);
-    pf_rescale(tl, pf_next_max(scur, blk_diag(0), 0, g, pos_n, tl.m_run, mult_cur));
+    if (blk_diag(0)) pf_mask(scur, 0, g, pos_n);
+    pf_rescale(tl, pf_next_max(pf_lane_max(scur), tl.m_run, mult_cur));
+    // The group of the next block to be summed (its scale word w; solo: alone) and the factor
+    // 2^vshift its P carries, the group's V scale over the block's (|vshift| <= 3).
+    auto open_group = [&](uint32_t w, bool solo) {
+        const int sv = blk_sv(w);
+        const int far = static_cast<int>(solo) | static_cast<int>(abs(grp_sv - sv) > 3);
+        const int sh = static_cast<int>(grp_n == kPfGroup) | (static_cast<int>(grp_n > 0) & far);
+        shut = sh != 0;
+        shut_sv = grp_sv;
+        const int start = sh | static_cast<int>(grp_n == 0);
+        grp_sv = start ? sv : grp_sv;
+        grp_n = solo ? kPfGroup : (start ? 1 : grp_n + 1);
+        return grp_sv - sv;
+    };
+    // The first half of block 0's probabilities.  lsum: the block's sum of p (with 2^vshift).
+    int vshift = open_group(w_cur, blk_diag(0));
+    float off = static_cast<float>(kPScaleExp + vshift) - tl.m_run;
+    float lsum = 0.f;
+    uint32_t ph[2][2][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pf_probs_half16(scur[i >> 1], mult_cur, off, lsum, ph, i >> 1, i & 1);
     __syncthreads();
 
-    for (int blk = 0; blk < n_blk; ++blk) {
-        // Resident: K of block blk+1 (K buffer (blk+1)&1) and V of block blk (V buffer blk&1).
-        // Free: K buffer blk&1 (block blk, scored in the previous step) and V buffer
-        // (blk+1)&1 (block blk-1).
+    // One step of the block loop.  Resident: K of block blk+1 (K buffer (blk+1)&1) and V of
+    // block blk (V buffer blk&1).  Free: K buffer blk&1 (block blk, scored in the previous step)
+    // and V buffer (blk+1)&1 (block blk-1).  Half of a block's probabilities are formed beside
+    // the next block's scores and half (of the block after) beside V^T P^T, so that both runs of
+    // 32 MFMAs have about as much VALU work beside them as fits: a SIMD's two waves issue
+    // 2 x 32 MFMAs in 1024 cycles, and with all 80 VALU instructions of the probabilities beside
+    // the scores that run took 1700-2400.  kPlain: blocks blk and blk+1 hold cached keys only (no
+    // masks, no trailing K parts), so that the step is one straight run.  With the branches of
+    // the general step in the loop, the compiler formed most probabilities before the scores'
+    // MFMAs: 4 x 512 tokens over 8192 566 us, now 540 us (MFMAs alone 254 us; timing builds:
+    // without the probabilities 64 us less, the copies 38, the LDS reads 30, the rescale of O and
+    // the fp64 sums 17 each).
+    auto step = [&](auto plain, int blk) {
+        constexpr bool kPlain = decltype(plain)::value;
+        const bool next = kPlain || blk + 1 < n_blk;
         if (blk + 2 < n_blk) issue_k(blk + 2, blk & 1, loff);
-        if (blk + 1 < n_blk) issue_v(blk + 1, (blk + 1) & 1, loff);
-        if ((blk & 255) == 0 && blk > 0 && wave < 4 && blk + 256 < n_blk) issue_sw(blk + 256 + 64 * wave);
-        const uint32_t w_next = blk + 1 < n_blk ? sw_at(blk + 1) : w_cur;
+        if (next) issue_v(blk + 1, (blk + 1) & 1, loff);
+        if ((blk & 255) == 128 && wave < 4 && blk + 128 < n_blk) issue_sw(blk + 128 + 64 * wave);
+        const uint32_t w_next = next ? __builtin_amdgcn_readfirstlane(w_ahead) : w_cur;
         unsafe |= w_next;
+        if (shut) pf_flush(tl, static_cast<double>(pow2f(-shut_sv)));
+        const int sv_blk = grp_sv;               // this block's group
+        const int l_shift = -vshift;
+        if (next) vshift = open_group(w_next, !kPlain && blk_diag(blk + 1));
 
-        const int sv = blk_sv(w_cur);
-        const bool solo = blk_diag(blk);
-        if (grp_n == kPfGroup || (grp_n > 0 && (solo || abs(grp_sv - sv) > 3))) {
-            pf_flush(tl, static_cast<double>(pow2f(-grp_sv)));
-            grp_n = 0;
-        }
-        if (grp_n == 0) grp_sv = sv;
-        grp_n = solo ? kPfGroup : grp_n + 1;
-        const float vshift = static_cast<float>(grp_sv - sv);
-
-        uint32_t ph[2][2][4];
         f32x4_t snext[4];
+        VtPair vt[2];
+        const uint32_t va = vaddr + (blk & 1) * kPlaneB;
         const uint8_t* knext = lds + kOffK + ((blk + 1) & 1) * kPlaneB;
         // The two waves of a SIMD run the same steps; the one in this MFMA + VALU mix gets
         // issue priority over the other's V^T P^T.
         __builtin_amdgcn_s_setprio(1);
-        if (blk + 1 >= n_blk)
-            pf_probs_and_next<false, false>(scur, mult_cur, vshift, knext, qop, n, g, tl, ph, snext);
+        if (kPlain)
+            pf_scores_beside<true, false, true>(scur, mult_cur, off, lsum, knext, qop, koff, va, ph, snext, vt);
+        else if (!next)
+            pf_scores_beside<false, false, false>(scur, mult_cur, off, lsum, knext, qop, koff, va, ph, snext, vt);
         else if (blk_new(blk + 1))
-            pf_probs_and_next<true, true>(scur, mult_cur, vshift, knext, qop, n, g, tl, ph, snext);
+            pf_scores_beside<true, true, false>(scur, mult_cur, off, lsum, knext, qop, koff, va, ph, snext, vt);
         else
-            pf_probs_and_next<true, false>(scur, mult_cur, vshift, knext, qop, n, g, tl, ph, snext);
+            pf_scores_beside<true, false, false>(scur, mult_cur, off, lsum, knext, qop, koff, va, ph, snext, vt);
         __builtin_amdgcn_s_setprio(0);
+
+        // The next block's running max is found beside this block's V^T P^T (which still
+        // accumulates at the current max); O and l move to it afterwards.
+        const float l_blk = lsum;
+        const float mult_next = blk_mult(w_next);
+        float m_next = tl.m_run;
+        uint32_t pn[2][2][4];
+        if (!kPlain && next && blk_diag(blk + 1)) pf_mask(snext, (blk + 1) * kPfBlk, g, pos_n);
+        lsum = 0.f;
+        if (!kPlain) {
+            vt[0] = pf_vt_issue(va);
+            vt[1] = pf_vt_issue(va ^ 32u);
+        }
+        pf_pv(va, ph, vt, tl, [&](int i) {
+            if (i == 0) {
+                w_ahead = sw_lds(blk + 2);
+                if (next) {
+                    m_next = pf_next_max(pf_lane_max(snext), tl.m_run, mult_next);
+                    off = static_cast<float>(kPScaleExp + vshift) - m_next;
+                }
+                tl.l64 += ldexp(static_cast<double>(l_blk), l_shift);
+            }
+            if (next && i == 1) pf_probs_half16(snext[0], mult_next, off, lsum, pn, 0, 0);
+            if (next && i == 2) {
+                pf_probs_half16(snext[0], mult_next, off, lsum, pn, 0, 1);
+                pf_probs_half16(snext[1], mult_next, off, lsum, pn, 1, 0);
+            }
+            if (next && i == 3) pf_probs_half16(snext[1], mult_next, off, lsum, pn, 1, 1);
+        });
+
         // fp16's subnormal quantum: a p below 2^-2 (in the units the MFMAs see) has a second part
         // below 2^-14, and the split carries it to within 2^-25 absolutely, not 2^-22 of itself
         // (a p below 2^-25 is dropped).  Harmless while those keys' V is about as large as the
@@ -1188,35 +1274,32 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
         // smallest-V block's or more (a uniform test), a lane with a p below 2^-2 among its 16
         // keys (the fp16 codes of the first parts, below 0x3400; masked keys count,
         // conservatively) adds their bound 16 * 2^-25 * 2^15 (staged |V| < 2^15) = 2^-6, times
-        // 2^-grp_sv, to u, which the epilogue compares with the row's elements.
-        if (grp_sv < sv_hi - 6) {
+        // 2^-sv_blk, to u, which the epilogue compares with the row's elements.
+        if (sv_blk < sv_hi - 6) {
             uint32_t m16 = ph[0][0][0];
 #pragma unroll
             for (int w = 0; w < 2; ++w)
 #pragma unroll
                 for (int d = 0; d < 4; ++d) m16 = pk_min_u16(m16, ph[0][w][d]);
-            if (min(m16 & 0xffffu, m16 >> 16) < 0x3400u) tl.u += pow2f(-6 - grp_sv);
+            if (min(m16 & 0xffffu, m16 >> 16) < 0x3400u) tl.u += pow2f(-6 - sv_blk);
         }
-
-        // The next block's running max is found before this block's V^T P^T (which still
-        // accumulates at the current max); O and l move to it afterwards.
-        const float mult_next = blk_mult(w_next);
-        float m_next = tl.m_run;
-        if (blk + 1 < n_blk)
-            m_next = pf_next_max(snext, blk_diag(blk + 1), (blk + 1) * kPfBlk, g, pos_n, tl.m_run, mult_next);
-
-        pf_pv(vaddr, (blk & 1) * kPlaneB, ph, tl);
-
         pf_rescale(tl, m_next);
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) scur[kt] = snext[kt];
+        for (int kt = 2; kt < 4; ++kt) scur[kt] = snext[kt];
+#pragma unroll
+        for (int part = 0; part < 2; ++part)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) ph[part][0][d] = pn[part][0][d];
         w_cur = w_next;
         mult_cur = mult_next;
         // This wave's copies into LDS are complete; after the barrier every wave's are, and
         // every wave is done with the buffers the next step's copies go to.
         __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0)
         __syncthreads();
-    }
+    };
+    int blk = 0;
+    for (; blk + 1 < cb0; ++blk) step(std::true_type{}, blk);
+    for (; blk < n_blk; ++blk) step(std::false_type{}, blk);
     pf_flush(tl, static_cast<double>(pow2f(-grp_sv)));
 
     double l = tl.l64 + __shfl_xor(tl.l64, 16);
