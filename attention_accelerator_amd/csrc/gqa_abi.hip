@@ -79,6 +79,16 @@ int32_t multi_wgs(const gqa_params_t* p, int32_t n_new) {
     return w > 0 ? w : 1;
 }
 
+// Key runs per query block of the prefill attention kernel: one of its workgroups fills a CU
+// (kWavesPerCu persistent stream workgroups).
+int32_t prefill_splits_of(const gqa_params_t* p, int32_t batch, int32_t n_new) {
+    return prefill_splits(batch, n_new, stream_wgs(p) / kWavesPerCu);
+}
+
+size_t prefill_attn_bytes(const gqa_params_t* p, int32_t batch, int32_t n_new, int32_t capacity) {
+    return align_up(prefill_stage_bytes(batch, n_new, capacity, prefill_splits_of(p, batch, n_new)), 256);
+}
+
 bool geometry_ok(const gqa_params_t* p) {
     if (p->n_q_heads != kHq || p->n_kv_heads != kHkv || p->head_dim != kD) return false;
     if (!(p->scale != 0.0) || !std::isfinite(p->scale)) return false;
@@ -575,7 +585,7 @@ size_t gqa_prefill_workspace_bytes(const gqa_params_t* params, int32_t batch, in
     if (use_multi(params, n_new))
         return align_up(prefill_multi_bytes(batch, n_new, multi_wgs(params, n_new)), 256) +
                rescore_bytes(batch, n_new, 1, n_new, 0);
-    return align_up(prefill_stage_bytes(batch, n_new, capacity), 256) +
+    return prefill_attn_bytes(params, batch, n_new, capacity) +
            rescore_bytes(batch, n_new, prefill_chunk_blocks(n_new), 64, prefill_cache_blocks(capacity));
 }
 
@@ -584,7 +594,7 @@ size_t gqa_prefill_rescored_rows_offset(const gqa_params_t* params, int32_t batc
     if (!gqa_prefill_workspace_bytes(params, batch, n_new, capacity)) return 0;
     // The rescore region (its first word: the flagged-row count) follows the path's own part.
     if (use_multi(params, n_new)) return align_up(prefill_multi_bytes(batch, n_new, multi_wgs(params, n_new)), 256);
-    return align_up(prefill_stage_bytes(batch, n_new, capacity), 256);
+    return prefill_attn_bytes(params, batch, n_new, capacity);
 }
 
 int gqa_kv_append_bf16(const gqa_params_t* params, const uint16_t* k_new, const uint16_t* v_new,
@@ -637,8 +647,9 @@ int gqa_prefill_bf16(const gqa_params_t* params, const uint16_t* q, const uint16
         rescore_layout(a, params, ws + align_up(prefill_multi_bytes(batch, n_new, multi_wgs(params, n_new)), 256), 1,
                        n_new, 0);
     } else {
+        a.n_split = prefill_splits_of(params, batch, n_new);
         prefill_stage_layout(a, workspace);
-        rescore_layout(a, params, ws + align_up(prefill_stage_bytes(batch, n_new, kv->capacity), 256),
+        rescore_layout(a, params, ws + prefill_attn_bytes(params, batch, n_new, kv->capacity),
                        prefill_chunk_blocks(n_new), 64, prefill_cache_blocks(kv->capacity));
     }
     hipStream_t s = static_cast<hipStream_t>(stream);

@@ -111,6 +111,9 @@ struct PrefillArgs {
                               // (int8) << 8, bit 31 set when the block cannot be staged exactly
     int32_t stg_pos;          // positions per (sequence, KV head): capacity rounded up to 64
     int32_t stg_cb;           // chunk blocks per (sequence, KV head): ceil(T / 64) + 1
+    int32_t n_split;          // key runs per query block of the attention kernel (1: no partials)
+    double2* sp_o;            // [query blocks x n_split][8 waves][16][64] partial O of each run
+    void* sp_ml;              // [query blocks x n_split][8 waves][64] (l, running max, u) of each run
     int64_t kv_batch_stride;
     int64_t kv_head_stride;
     int64_t kv_pos_stride;
@@ -265,9 +268,12 @@ int32_t multi_waves(int32_t n_new);
 int32_t multi_simd_waves(int32_t n_new);
 
 // Workspace of the prefill attention path (chunks of more than kMultiMaxNew tokens): the
-// fp32 rotated new K rows, then the fp16 staging planes and block scales.
-size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity);
-void prefill_stage_layout(PrefillArgs& a, void* base);
+// fp32 rotated new K rows, then the fp16 staging planes and block scales, then the partials of
+// the attention kernel's key runs (n_split > 1).
+size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity, int32_t n_split);
+void prefill_stage_layout(PrefillArgs& a, void* base);       // a.n_split set
+// Key runs per query block on a device of `cus` CUs.
+int32_t prefill_splits(int32_t batch, int32_t n_new, int32_t cus);
 hipError_t launch_prefill_stage(const PrefillArgs& a, hipStream_t stream);
 // Workspace of the multi-token path: Q operands, plan, partials, chunk-key scores.
 size_t prefill_multi_bytes(int32_t batch, int32_t n_new, int32_t n_wgs);

@@ -74,20 +74,58 @@ constexpr int kStgThreads = 256;           // staging workgroup: 4 threads per r
 constexpr int kStgMaxWgs = 8192;
 constexpr int kPScaleExp = 12;             // P is formed as 2^12 * 2^(s - m) <= 4096
 
+// Key splits of the attention kernel.  One workgroup per (sequence, KV head, 32 positions)
+// leaves most of the chip idle for a short chunk of one or a few sequences (200 tokens of one
+// sequence: 56 workgroups on 256 CUs), however long the context is.  When at least two
+// workgroups per CU-slot fit (a workgroup's LDS and registers fill a CU), each query block's
+// keys are cut into n_split runs of whole blocks, one workgroup each, whose fp64 partials
+// prefill_merge_kernel combines: as many as fit in one round of the CUs, so that a split never
+// adds a round.  A run keeps at least kPfMinRun blocks (a workgroup costs about 10 us besides
+// its blocks of 1.8 us each, and a partial is 136 KB to write and read).
+constexpr int kPfMaxSplit = 32;
+constexpr int kPfMinRun = 4;
+
 size_t al256(size_t x) { return (x + 255) / 256 * 256; }
 
+// A split workgroup's partial: per wave and lane 32 doubles of O, and (l, m, u).
+constexpr size_t kSplitOB = size_t{kPfWaves} * kWave * 32 * sizeof(double);
+struct SplitMl {
+    double l;
+    float m;
+    float u;
+};
+constexpr size_t kSplitMlB = size_t{kPfWaves} * kWave * sizeof(SplitMl);
+
+size_t split_slots(int32_t batch, int32_t n_new, int32_t n_split) {
+    return n_split > 1 ? static_cast<size_t>(batch) * kHkv * ((n_new + kPfPos - 1) / kPfPos) * n_split : 0;
+}
+
+// The runs of a query block of n_blk key blocks: `per` blocks each, n of them (1: no partial).
+__device__ __forceinline__ int pf_runs(int n_blk, int n_split, int& per) {
+    const int want = max(1, min(n_split, n_blk / kPfMinRun));
+    per = (n_blk + want - 1) / want;
+    return (n_blk + per - 1) / per;
+}
+
 }  // namespace
+
+int32_t prefill_splits(int32_t batch, int32_t n_new, int32_t cus) {
+    const int64_t wgs = static_cast<int64_t>(batch) * kHkv * ((n_new + kPfPos - 1) / kPfPos);
+    const int64_t n = cus / wgs;
+    return n < 2 ? 1 : n > kPfMaxSplit ? kPfMaxSplit : static_cast<int32_t>(n);
+}
 
 // ---------------------------------------------------------------------------------
 // Workspace of the prefill attention path: the rotated new K rows in fp32, the fp16 K and
 // V planes, the trailing-part planes of the chunk blocks and the block scale words.
-size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity) {
+size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity, int32_t n_split) {
     const size_t rows = static_cast<size_t>(batch) * n_new * kHkv;
     const size_t pos = (static_cast<size_t>(capacity) + kPfBlk - 1) / kPfBlk * kPfBlk;
     const size_t cb = static_cast<size_t>(prefill_chunk_blocks(n_new));
     const size_t bh = static_cast<size_t>(batch) * kHkv;
     return al256(rows * kD * sizeof(float)) + 2 * al256(bh * pos * kD * sizeof(uint16_t)) +
-           al256(bh * cb * kPfBlk * kD * sizeof(uint16_t)) + al256(bh * (pos / kPfBlk) * sizeof(uint32_t));
+           al256(bh * cb * kPfBlk * kD * sizeof(uint16_t)) + al256(bh * (pos / kPfBlk) * sizeof(uint32_t)) +
+           split_slots(batch, n_new, n_split) * (kSplitOB + kSplitMlB);
 }
 
 void prefill_stage_layout(PrefillArgs& a, void* base) {
@@ -105,6 +143,9 @@ void prefill_stage_layout(PrefillArgs& a, void* base) {
     a.stg_klo = reinterpret_cast<uint16_t*>(p);
     p += al256(bh * a.stg_cb * kPfBlk * kD * sizeof(uint16_t));
     a.stg_scale = reinterpret_cast<uint32_t*>(p);
+    p += al256(bh * (a.stg_pos / kPfBlk) * sizeof(uint32_t));
+    a.sp_o = reinterpret_cast<double2*>(p);
+    a.sp_ml = p + split_slots(a.batch, a.n_new, a.n_split) * kSplitOB;
 }
 
 // ---------------------------------------------------------------------------------
@@ -776,7 +817,8 @@ __device__ __forceinline__ void pf_scores_beside(const f32x4_t (&scur)[4], float
                                                  uint32_t vaddr, uint32_t (&ph)[2][2][4], f32x4_t (&snext)[4],
                                                  VtPair (&cur)[2]) {
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) snext[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < 4; ++kt)       // (no next block: as if every key were masked)
+        snext[kt] = kNext ? f32x4_t{0.f, 0.f, 0.f, 0.f} : f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     f16x8_t ak[3][2];
     if (kNext) {
         pf_k_pair(kplane, 0, koff, ak[0]);
@@ -847,11 +889,11 @@ __device__ __forceinline__ void pf_pv(uint32_t vaddr, const uint32_t (&ph)[2][2]
 // reads dims 8g .. 8g+7 and 32 + 8g .. (and their pairs 64 on), pair groups g and 4 + g.
 // y and its square in double, as in the multi-token merge (in fp32 y^2 underflows in every
 // dim of a row whose elements lie ~2^63 below their dims' largest |V|).  ul bounds the error
-// fp16's subnormal quantum added to every element (the attention loop's u over l): a row
-// with an element below 8 ul, where that error could reach 64 ULP with a margin of 2, is
-// rescored as well.  Returns the decision for the row in every lane of its column.
+// fp16's subnormal quantum added to every element (the attention loop's u over l; infinite for
+// rows that are always rescored): a row with an element below 8 ul, where that error could
+// reach 64 ULP with a margin of 2, is rescored as well.  Returns the decision for the row in every lane of its column.
 __device__ __forceinline__ bool pf_flag_row(const PrefillArgs& a, int b, int kvh, int st, int pos, int64_t row,
-                                            float m, bool forced, double ul, const uint2 (&pk)[8], int lane) {
+                                            float m, double ul, const uint2 (&pk)[8], int lane) {
     const int g = lane >> 4;
     const int cb = pos / kPfBlk - st / kPfBlk;
     const int r = pos % kPfBlk;
@@ -923,8 +965,7 @@ __device__ __forceinline__ bool pf_flag_row(const PrefillArgs& a, int b, int kvh
     d_max = max(d_max, static_cast<uint32_t>(__shfl_xor(static_cast<int>(d_max), 16)));
     d_max = max(d_max, static_cast<uint32_t>(__shfl_xor(static_cast<int>(d_max), 32)));
     const float mnx = __uint_as_float(min(x_min & 0xffffu, x_min >> 16) << 16);
-    const bool bad = forced || max(x_max & 0xffffu, x_max >> 16) >= 0x7f80u ||
-                     static_cast<double>(mnx) < 8.0 * ul;
+    const bool bad = max(x_max & 0xffffu, x_max >> 16) >= 0x7f80u || !(static_cast<double>(mnx) >= 8.0 * ul);
     // an infinite or NaN V among the row's keys (its y is 0: the row is flagged)
     if (d_max >= 0x7f80u && (lane >> 4) == 0) atomicOr(a.rs_hdr + 2, 1u);
     const double ed = static_cast<double>(e) * fabs(a.qk_scale_log2);
@@ -951,6 +992,37 @@ __device__ __forceinline__ bool pf_flag_row(const PrefillArgs& a, int b, int kvh
     return flagged;
 }
 
+// Ends the rows of one wave's 16 queries (lane (g, n): dims 16dt + 4g + i of query n at
+// position st + t; O, this lane's share of l, the running max and this lane's share of the
+// bound u, infinite for rows that always go to the rescore): normalises, rounds double -> f32 ->
+// BF16, decides the rescore flag from the rounded row and writes it.  q_ok: the lane's query
+// exists (waves past the last query decide and write nothing).
+__device__ __forceinline__ void pf_finish(const PrefillArgs& a, int b, int kvh, int st, int t, bool q_ok, int hq,
+                                          const double (&o64)[8][4], double l64, float m, float u, int lane) {
+    const int g = lane >> 4;
+    double l = l64 + __shfl_xor(l64, 16);
+    l += __shfl_xor(l, 32);
+    u += __shfl_xor(u, 16);
+    u += __shfl_xor(u, 32);
+    const double ul = static_cast<double>(u) / l;     // bound on that error in the row's elements
+    const double inv_l = 1.0 / l;
+    const int64_t row = (static_cast<int64_t>(b) * a.n_new + t) * kHq + hq;
+    uint2 pk[8];
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+        pk[dt].x = f32x2_to_bf16_out(static_cast<float>(o64[dt][0] * inv_l), static_cast<float>(o64[dt][1] * inv_l));
+        pk[dt].y = f32x2_to_bf16_out(static_cast<float>(o64[dt][2] * inv_l), static_cast<float>(o64[dt][3] * inv_l));
+    }
+    if (a.rs_hdr && __ballot(q_ok)) {
+        if (pf_flag_row(a, b, kvh, st, st + t, row, m, ul, pk, lane) && q_ok && g == 0)
+            rs_append(a, static_cast<uint32_t>(row));
+    }
+    if (!q_ok) return;
+    uint16_t* orow = a.out + row * kD;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<uint2*>(orow + 16 * dt + 4 * g) = pk[dt];
+}
+
 __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsB];
 
@@ -958,9 +1030,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     // round-robin; all query blocks of a pair (8 per sequence) go to one XCD so that its K/V
     // blocks are shared in that XCD's L2.  A pair's query blocks are dealt last first: the
     // last ones see the most keys, and the short ones then fill the CUs that finish early.
-    const int k_id = blockIdx.x >> 3;
-    const int qb = a.n_qblk - 1 - k_id % a.n_qblk;
-    const int pair = (k_id / a.n_qblk) * 8 + (blockIdx.x & 7);
+    // Then the runs of a query block (n_split > 1), neighbours on the same XCD.
+    const int unit = (blockIdx.x >> 3) / a.n_split;
+    const int run = (blockIdx.x >> 3) % a.n_split;
+    const int qb = a.n_qblk - 1 - unit % a.n_qblk;
+    const int pair = (unit / a.n_qblk) * 8 + (blockIdx.x & 7);
     const int b = pair / kHkv;
     const int kvh = pair % kHkv;
     const int tid = threadIdx.x;
@@ -977,7 +1051,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     const int st = a.start[b];
 
     if (!prefill_start_ok(a, st)) {
-        if (q_ok && g == 0) {
+        if (q_ok && g == 0 && run == 0) {
             uint4* o = reinterpret_cast<uint4*>(a.out + ((static_cast<int64_t>(b) * T + tq) * kHq + hq) * kD);
             for (int i = 0; i < kD / 8; ++i) o[i] = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
         }
@@ -985,13 +1059,19 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     }
 
     // Every wave runs every block of the workgroup; a block past the keys of this wave's
-    // queries is masked for all of them (block 0 always holds a valid key, so the running
-    // max is finite from the first block on).  Waves past the last query compute the last
-    // query and write nothing.
+    // queries is masked for all of them (without a split block 0 always holds a valid key, so
+    // the running max is finite from the first block on; in a later run it may stay -inf, and
+    // p is formed against 0 then).  Waves past the last query compute the last query and write
+    // nothing.
     const int tq_c = min(tq, T - 1);
     const int pos_n = st + tq_c;            // this lane's query position
     const int n_keys = st + min(T, qb * kPfPos + kPfPos);
-    const int n_blk = (n_keys + kPfBlk - 1) / kPfBlk;
+    const int all_blk = (n_keys + kPfBlk - 1) / kPfBlk;
+    int per_run;
+    const int n_run = pf_runs(all_blk, a.n_split, per_run);
+    if (run >= n_run) return;
+    const int blk0 = run * per_run;
+    const int n_blk = min(all_blk, blk0 + per_run);        // this run: blocks blk0 .. n_blk - 1
     const int nblk_stg = a.stg_pos / kPfBlk;
     const char* kseg = reinterpret_cast<const char*>(a.stg_k + static_cast<int64_t>(pair) * a.stg_pos * kD);
     const char* vseg = reinterpret_cast<const char*>(a.stg_v + static_cast<int64_t>(pair) * a.stg_pos * kD);
@@ -1009,18 +1089,20 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
         pf_issue(vseg + static_cast<int64_t>(blk) * kPlaneB, loff, lds + kOffV + buf * kPlaneB, wave);
     };
 
-    // K of blocks 0 and 1 and V of block 0 are requested before the Q operands are formed.
+    // K of the first two blocks and V of the first are requested before the Q operands are
+    // formed.
     uint32_t loff[2];
     pf_copy_offsets(wave, lane, loff);
-    issue_k(0, 0, loff);
-    issue_v(0, 0, loff);
-    if (n_blk > 1) issue_k(1, 1, loff);
-    // Scale words of blocks 64 wave .. 64 wave + 63 (entries past the last block repeat it).
+    issue_k(blk0, blk0 & 1, loff);
+    issue_v(blk0, blk0 & 1, loff);
+    if (blk0 + 1 < n_blk) issue_k(blk0 + 1, (blk0 + 1) & 1, loff);
+    // Scale words of 64 blocks per wave, from the ring half that holds the first block (entries
+    // past the last block repeat it).
     auto issue_sw = [&](int first) {
         __builtin_amdgcn_global_load_lds(sw + min(first + lane, nblk_stg - 1),
                                          (lds_void_t*)(lds + kOffSw + 4 * (first & (kSwRing - 1))), 4, 0, 0);
     };
-    issue_sw(64 * wave);
+    issue_sw((blk0 & ~255) + 64 * wave);
     // The first scale words again, for their maximum below (requested with the rest).
     constexpr int kSwAhead = 3;
     uint32_t sw_ahead[kSwAhead];
@@ -1142,36 +1224,37 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
         return fmaxf(cq * pow2f(-static_cast<int>(static_cast<int8_t>(w & 0xffu))), 1.17549435e-38f);
     };
     auto blk_sv = [&](uint32_t w) { return static_cast<int>(static_cast<int8_t>((w >> 8) & 0xffu)); };
-    // The largest V scale exponent among this workgroup's blocks (the smallest-V block's).
+    // The largest V scale exponent among the query block's blocks (the smallest-V block's).
     int sv_hi = -128;
 #pragma unroll
     for (int i = 0; i < kSwAhead; ++i)
-        if (i * kWave + lane < n_blk) sv_hi = max(sv_hi, blk_sv(sw_ahead[i]));
-    for (int j = kSwAhead * kWave + lane; j < n_blk; j += kWave) sv_hi = max(sv_hi, blk_sv(sw[j]));
+        if (i * kWave + lane < all_blk) sv_hi = max(sv_hi, blk_sv(sw_ahead[i]));
+    for (int j = kSwAhead * kWave + lane; j < all_blk; j += kWave) sv_hi = max(sv_hi, blk_sv(sw[j]));
 #pragma unroll
     for (int sh = 1; sh < kWave; sh <<= 1) sv_hi = max(sv_hi, __shfl_xor(sv_hi, sh));
     sv_hi = __builtin_amdgcn_readfirstlane(sv_hi);
 
-    // Block 0's scores.  The barrier after them frees K buffer 0 for block 2.
+    // The first block's scores.  The barrier after them frees its K buffer.
     __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0)
     __syncthreads();
     f32x4_t scur[4];
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) scur[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const uint8_t* kfirst = lds + kOffK + (blk0 & 1) * kPlaneB;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         f16x8_t ak[2];
-        pf_k_pair(lds + kOffK, i, koff, ak);
-        if (blk_new(0))
-            pf_qk_pair<true>(lds + kOffK, ak, qop, i, koff, scur);
+        pf_k_pair(kfirst, i, koff, ak);
+        if (blk_new(blk0))
+            pf_qk_pair<true>(kfirst, ak, qop, i, koff, scur);
         else
-            pf_qk_pair<false>(lds + kOffK, ak, qop, i, koff, scur);
+            pf_qk_pair<false>(kfirst, ak, qop, i, koff, scur);
     }
-    uint32_t w_cur = __builtin_amdgcn_readfirstlane(sw_lds(0));
-    uint32_t w_ahead = sw_lds(1);          // block blk+1's word, read a step ahead
+    uint32_t w_cur = __builtin_amdgcn_readfirstlane(sw_lds(blk0));
+    uint32_t w_ahead = sw_lds(blk0 + 1);          // block blk+1's word, read a step ahead
     uint32_t unsafe = w_cur;                // bit 31 of any block read marks all rows
     float mult_cur = blk_mult(w_cur);
-    if (blk_diag(0)) pf_mask(scur, 0, g, pos_n);
+    if (blk_diag(blk0)) pf_mask(scur, blk0 * kPfBlk, g, pos_n);
     pf_rescale(tl, pf_next_max(pf_lane_max(scur), tl.m_run, mult_cur));
     // The group of the next block to be summed (its scale word w; solo: alone) and the factor
     // 2^vshift its P carries, the group's V scale over the block's (|vshift| <= 3).
@@ -1186,9 +1269,14 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
         grp_n = solo ? kPfGroup : (start ? 1 : grp_n + 1);
         return grp_sv - sv;
     };
-    // The first half of block 0's probabilities.  lsum: the block's sum of p (with 2^vshift).
-    int vshift = open_group(w_cur, blk_diag(0));
-    float off = static_cast<float>(kPScaleExp + vshift) - tl.m_run;
+    // The first half of the first block's probabilities.  lsum: the block's sum of p (with
+    // 2^vshift).  p = 2^(s + off); a running max still at -inf (every key so far masked) counts
+    // as 0, so that p = 0.
+    auto p_off = [&](int shift, float m) {
+        return static_cast<float>(kPScaleExp + shift) - (m == -INFINITY ? 0.f : m);
+    };
+    int vshift = open_group(w_cur, blk_diag(blk0));
+    float off = p_off(vshift, tl.m_run);
     float lsum = 0.f;
     uint32_t ph[2][2][4];
 #pragma unroll
@@ -1250,20 +1338,19 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
             vt[1] = pf_vt_issue(va ^ 32u);
         }
         pf_pv(va, ph, vt, tl, [&](int i) {
+            // (no branches here: V^T operands are in flight)
             if (i == 0) {
                 w_ahead = sw_lds(blk + 2);
-                if (next) {
-                    m_next = pf_next_max(pf_lane_max(snext), tl.m_run, mult_next);
-                    off = static_cast<float>(kPScaleExp + vshift) - m_next;
-                }
+                m_next = pf_next_max(pf_lane_max(snext), tl.m_run, mult_next);
+                off = kPlain ? static_cast<float>(kPScaleExp + vshift) - m_next : p_off(vshift, m_next);
                 tl.l64 += ldexp(static_cast<double>(l_blk), l_shift);
             }
-            if (next && i == 1) pf_probs_half16(snext[0], mult_next, off, lsum, pn, 0, 0);
-            if (next && i == 2) {
+            if (i == 1) pf_probs_half16(snext[0], mult_next, off, lsum, pn, 0, 0);
+            if (i == 2) {
                 pf_probs_half16(snext[0], mult_next, off, lsum, pn, 0, 1);
                 pf_probs_half16(snext[1], mult_next, off, lsum, pn, 1, 0);
             }
-            if (next && i == 3) pf_probs_half16(snext[1], mult_next, off, lsum, pn, 1, 1);
+            if (i == 3) pf_probs_half16(snext[1], mult_next, off, lsum, pn, 1, 1);
         });
 
         // fp16's subnormal quantum: a p below 2^-2 (in the units the MFMAs see) has a second part
@@ -1297,50 +1384,106 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
         __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0)
         __syncthreads();
     };
-    int blk = 0;
-    for (; blk + 1 < cb0; ++blk) step(std::true_type{}, blk);
+    int blk = blk0;
+    for (; blk + 1 < min(cb0, n_blk); ++blk) step(std::true_type{}, blk);
     for (; blk < n_blk; ++blk) step(std::false_type{}, blk);
     pf_flush(tl, static_cast<double>(pow2f(-grp_sv)));
 
-    double l = tl.l64 + __shfl_xor(tl.l64, 16);
-    l += __shfl_xor(l, 32);
-    float u = tl.u + __shfl_xor(tl.u, 16);
-    u += __shfl_xor(u, 32);
-    const double ul = static_cast<double>(u) / l;     // bound on that error in the row's elements
-    // The row of query n: lanes n, n+16, n+32, n+48 hold dims 16dt + 4g ..
-    const double inv_l = 1.0 / l;
-    double x[8][4];
+    // Rows that read a marked block or whose Q row is out of range always go to the rescore:
+    // their error bound is infinite.
+    if ((unsafe >> 31) != 0u || q_bad) tl.u = INFINITY;
+    if (n_run > 1) {
+        const int64_t slot = (static_cast<int64_t>(pair) * a.n_qblk + qb) * a.n_split + run;
+        double2* po = a.sp_o + (slot * kPfWaves + wave) * 16 * kWave + lane;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                po[(2 * dt + j) * kWave] = make_double2(tl.o64[dt][2 * j], tl.o64[dt][2 * j + 1]);
+        static_cast<SplitMl*>(a.sp_ml)[(slot * kPfWaves + wave) * kWave + lane] = SplitMl{tl.l64, tl.m_run, tl.u};
+        return;
+    }
+    pf_finish(a, b, kvh, st, tq_c, q_ok, hq, tl.o64, tl.l64, tl.m_run, tl.u, lane);
+}
+
+// Combines the runs of one wave's 16 queries (grid: 8 waves per query block and pair): wave v
+// of the workgroup sums dim tile v over the runs in order, each scaled by the exact power of two
+// between its running max and the largest so far, and the sums meet in LDS for the first
+// wave, which ends the rows as the attention kernel does.
+__global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(PrefillArgs a) {
+    __shared__ double2 o_s[kPfWaves][2][kWave];
+    const int unit = blockIdx.x / kPfWaves;
+    const int wt = blockIdx.x % kPfWaves;
+    const int pair = unit / a.n_qblk;
+    const int qb = unit % a.n_qblk;
+    const int b = pair / kHkv;
+    const int kvh = pair % kHkv;
+    const int v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & (kWave - 1);
+    const int T = a.n_new;
+    const int st = a.start[b];
+    if (!prefill_start_ok(a, st)) return;
+    int per;
+    const int n_run = pf_runs((st + min(T, qb * kPfPos + kPfPos) + kPfBlk - 1) / kPfBlk, a.n_split, per);
+    if (n_run == 1) return;
+    const int t_wave0 = qb * kPfPos + (wt >> 2) * 16;
+    if (t_wave0 >= T) return;
+    const int tq = t_wave0 + (lane & 15);
+    const int64_t slot0 = (static_cast<int64_t>(pair) * a.n_qblk + qb) * a.n_split;
+    const double2* po = a.sp_o + ((slot0 * kPfWaves + wt) * 16 + 2 * v) * kWave + lane;
+    const SplitMl* pml = static_cast<const SplitMl*>(a.sp_ml) + (slot0 * kPfWaves + wt) * kWave + lane;
+    double o[4] = {0.0, 0.0, 0.0, 0.0};
+    double l = 0.0;
+    float m = -INFINITY, u = 0.f;
+    constexpr int kAhead = 8;
+    for (int r0 = 0; r0 < n_run; r0 += kAhead) {
+        double2 x[kAhead][2];
+        SplitMl ml[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const int64_t r = min(r0 + i, n_run - 1);
+            ml[i] = pml[r * kPfWaves * kWave];
+            x[i][0] = po[r * kPfWaves * 16 * kWave];
+            x[i][1] = po[r * kPfWaves * 16 * kWave + kWave];
+        }
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            if (r0 + i >= n_run) break;                       // (uniform)
+            const float m_new = fmaxf(m, ml[i].m);
+            const int sa = m == m_new ? 0 : max_shift(m, m_new);
+            const int sx = ml[i].m == m_new ? 0 : max_shift(ml[i].m, m_new);
+            o[0] = ldexp(o[0], sa) + ldexp(x[i][0].x, sx);
+            o[1] = ldexp(o[1], sa) + ldexp(x[i][0].y, sx);
+            o[2] = ldexp(o[2], sa) + ldexp(x[i][1].x, sx);
+            o[3] = ldexp(o[3], sa) + ldexp(x[i][1].y, sx);
+            l = ldexp(l, sa) + ldexp(ml[i].l, sx);
+            u = ldexpf(u, sa) + ldexpf(ml[i].u, sx);
+            m = m_new;
+        }
+    }
+    o_s[v][0][lane] = make_double2(o[0], o[1]);
+    o_s[v][1][lane] = make_double2(o[2], o[3]);
+    __syncthreads();
+    if (v > 0) return;
+    double o64[8][4];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[dt][i] = tl.o64[dt][i] * inv_l;
-    const bool q_bad_row = __shfl_xor(static_cast<int>(q_bad), 16) | __shfl_xor(static_cast<int>(q_bad), 32) |
-                           __shfl_xor(static_cast<int>(q_bad), 48) | static_cast<int>(q_bad);
-    const int64_t row = (static_cast<int64_t>(b) * T + tq_c) * kHq + hq;
-    uint2 pk[8];
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-        pk[dt].x = f32x2_to_bf16_out(static_cast<float>(x[dt][0]), static_cast<float>(x[dt][1]));
-        pk[dt].y = f32x2_to_bf16_out(static_cast<float>(x[dt][2]), static_cast<float>(x[dt][3]));
-    }
-    // The rescore flag, decided here from the rounded row: rows that read a marked block or
-    // whose Q row is out of range always go to the rescore.  Waves past the last query (q_ok
-    // false in every lane) decide nothing.
-    if (a.rs_hdr && __ballot(q_ok)) {
-        const bool forced = (unsafe >> 31) != 0u || q_bad_row;
-        if (pf_flag_row(a, b, kvh, st, st + tq_c, row, tl.m_run, forced, ul, pk, lane) && q_ok && g == 0)
-            rs_append(a, static_cast<uint32_t>(row));
-    }
-    if (!q_ok) return;
-    uint16_t* orow = a.out + row * kD;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<uint2*>(orow + 16 * dt + 4 * g) = pk[dt];
+        for (int j = 0; j < 2; ++j) {
+            o64[dt][2 * j] = o_s[dt][j][lane].x;
+            o64[dt][2 * j + 1] = o_s[dt][j][lane].y;
+        }
+    pf_finish(a, b, kvh, st, min(tq, T - 1), tq < T, kvh * kGroup + (wt & 3), o64, l, m, u, lane);
 }
 
 hipError_t launch_prefill_attention(const PrefillArgs& a, hipStream_t stream) {
-    const int64_t n_wg = static_cast<int64_t>(a.batch) * kHkv * a.n_qblk;
-    if (n_wg == 0) return hipSuccess;
-    hipLaunchKernelGGL(prefill_attn_kernel, dim3(static_cast<unsigned>(n_wg)), dim3(kPfThreads), 0, stream, a);
+    const int64_t n_unit = static_cast<int64_t>(a.batch) * kHkv * a.n_qblk;
+    if (n_unit == 0) return hipSuccess;
+    hipLaunchKernelGGL(prefill_attn_kernel, dim3(static_cast<unsigned>(n_unit * a.n_split)), dim3(kPfThreads), 0,
+                       stream, a);
+    if (a.n_split > 1)
+        hipLaunchKernelGGL(prefill_merge_kernel, dim3(static_cast<unsigned>(n_unit * kPfWaves)), dim3(kPfThreads), 0,
+                           stream, a);
     return hipGetLastError();
 }
 
