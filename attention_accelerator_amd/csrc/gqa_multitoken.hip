@@ -135,6 +135,16 @@ void prefill_multi_layout(PrefillArgs& a, void* base, int32_t n_wgs) {
     a.n_wgs = n_wgs;
 }
 
+// Smallest range of a batch with a segment of kMtLongKeys keys or more.  Where a few long
+// segments are cut into the smallest ranges there are (one sequence of 4001 positions, T =
+// 5: 63 ranges of 64 keys per segment), half as many of twice the keys leave the stream
+// kernel's time as it is (20 us, most of it a range's fixed cost) and halve the merge's work
+// (T = 5 step 38.5 -> 35.5 us, T = 16 50.1 -> 45.5); ranges of 192 and 256 keys measured 36.6
+// and 38.7.  With shorter segments the pieces are few either way and 64 keys are faster
+// (8 x 500 positions, T = 2: 27.7 us against 29.4).
+constexpr int kMtLongKeys = 2048;
+constexpr int kMtLongRange = 128;
+
 // The stream-K plan (one wave): seq_off[b] = stream position of sequence b's first segment,
 // seq_off[B] = total, header {total, positions per workgroup, lead, XCD extra}
 // (gqa_streamk.h).
@@ -154,7 +164,8 @@ __device__ __forceinline__ void mt_build_plan(const PrefillArgs& a, int lane) {
     }
     int lead;
     int64_t total, per_wg;
-    plan_lead_totals(sum, max_keys, n_seq, a.n_wgs, lead, total, per_wg, mt_seg_lead(kW));
+    plan_lead_totals(sum, max_keys, n_seq, a.n_wgs, lead, total, per_wg, mt_seg_lead(kW),
+                     max_keys >= kMtLongKeys ? kMtLongRange : kMinRangeKeys);
     if (lane == 0) {
         a.plan_hdr[0] = total;
         a.plan_hdr[1] = per_wg;
@@ -1162,6 +1173,78 @@ __device__ __forceinline__ void mt_flag_row(const PrefillArgs& a, int64_t row, f
     }
 }
 
+// One thread's share (8 dims of a column) of a segment's sum: running max, l and O.
+struct MtSum {
+    float m;
+    double l;
+    double o[8];
+};
+
+// Sums pieces first, first + stride, .. of a segment (partial slots from slot0) for column
+// col, dims d0 .. d0 + 7, kGroupP at a time, every load of a group issued before any is used
+// (one memory round trip per group); the running max moves by whole powers of two, so
+// rescaling what is already summed is exact.
+template <int kGroupP, int kCols>
+__device__ __forceinline__ void mt_sum_pieces(const PrefillArgs& a, int64_t slot0, int n_pieces, int first, int stride,
+                                              int col, int d0, MtSum& t) {
+    t.m = -INFINITY;
+    t.l = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t.o[i] = 0.0;
+    for (int p0 = first; p0 < n_pieces; p0 += kGroupP * stride) {
+        float2 ml[kGroupP];
+        float v[kGroupP][8];                        // widened where summed
+#pragma unroll
+        for (int q = 0; q < kGroupP; ++q) {
+            ml[q] = make_float2(-INFINITY, 0.f);
+            if (p0 + q * stride < n_pieces) {
+                const int64_t c = (slot0 + p0 + q * stride) * kCols + col;
+                ml[q] = a.part_ml[c];
+                const float4* po = reinterpret_cast<const float4*>(a.part_o + c * kD + d0);
+                const float4 x0 = po[0], x1 = po[1];
+                v[q][0] = x0.x;
+                v[q][1] = x0.y;
+                v[q][2] = x0.z;
+                v[q][3] = x0.w;
+                v[q][4] = x1.x;
+                v[q][5] = x1.y;
+                v[q][6] = x1.z;
+                v[q][7] = x1.w;
+            }
+        }
+        float mb = t.m;
+#pragma unroll
+        for (int q = 0; q < kGroupP; ++q) mb = fmaxf(mb, ml[q].x);
+        if (t.m != -INFINITY && mb != t.m) {
+            const int e = max_shift(t.m, mb);
+            t.l = ldexp(t.l, e);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) t.o[i] = ldexp(t.o[i], e);
+        }
+        t.m = mb;
+#pragma unroll
+        for (int q = 0; q < kGroupP; ++q) {
+            if (ml[q].x == -INFINITY) continue;
+            const int e = max_shift(ml[q].x, t.m);
+            t.l += ldexp(static_cast<double>(ml[q].y), e);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) t.o[i] += ldexp(static_cast<double>(v[q][i]), e);
+        }
+    }
+}
+
+// Normalises and writes the thread's 8 elements of a row (ow: their BF16 codes).
+__device__ __forceinline__ void mt_write_row(const PrefillArgs& a, int64_t row, int d0, const MtSum& t,
+                                             uint32_t (&ow)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        ow[i] = f32_to_bf16_out(static_cast<float>(t.o[2 * i] / t.l)) |
+                (static_cast<uint32_t>(f32_to_bf16_out(static_cast<float>(t.o[2 * i + 1] / t.l))) << 16);
+    uint2* dst = reinterpret_cast<uint2*>(a.out + row * kD + d0);   // out is 8-byte aligned
+    dst[0] = make_uint2(ow[0], ow[1]);
+    dst[1] = make_uint2(ow[2], ow[3]);
+}
+
 // One workgroup per (KV head, sequence), 16 threads per column: thread i handles column
 // i/16 (token c/4, head c%4), dims 8(i%16) .. +8.  It reduces the segment's cached-key
 // maxima from every piece's records, merges the partials of a split segment's pieces
@@ -1228,64 +1311,127 @@ __global__ __launch_bounds__(256 * kW) __attribute__((amdgpu_waves_per_eu(8))) v
     mt_lds_barrier();
     if (!live) return;
     if (n_pieces > 1) {
-        // Pieces two at a time, every load of a group issued before any is used (one memory
-        // round trip per group; with 61 registers eight waves fit on a SIMD, so a 16-wave
-        // workgroup per segment at T = 16 no longer leaves half of them waiting for a CU);
-        // the running max moves by whole powers of two, so rescaling what is already summed
-        // is exact.
-        constexpr int kGroupP = 2;
-        m = -INFINITY;
-        double l = 0.0, o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int p0 = 0; p0 < n_pieces; p0 += kGroupP) {
-            float2 ml[kGroupP];
-            float v[kGroupP][8];                        // widened where summed
-#pragma unroll
-            for (int q = 0; q < kGroupP; ++q) {
-                ml[q] = make_float2(-INFINITY, 0.f);
-                if (p0 + q < n_pieces) {
-                    const int64_t c = (slot0 + p0 + q) * kCols + col;
-                    ml[q] = a.part_ml[c];
-                    const float4* po = reinterpret_cast<const float4*>(a.part_o + c * kD + d0);
-                    const float4 x0 = po[0], x1 = po[1];
-                    v[q][0] = x0.x;
-                    v[q][1] = x0.y;
-                    v[q][2] = x0.z;
-                    v[q][3] = x0.w;
-                    v[q][4] = x1.x;
-                    v[q][5] = x1.y;
-                    v[q][6] = x1.z;
-                    v[q][7] = x1.w;
-                }
-            }
-            float mb = m;
-#pragma unroll
-            for (int q = 0; q < kGroupP; ++q) mb = fmaxf(mb, ml[q].x);
-            if (m != -INFINITY && mb != m) {
-                const int e = max_shift(m, mb);
-                l = ldexp(l, e);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) o[i] = ldexp(o[i], e);
-            }
-            m = mb;
-#pragma unroll
-            for (int q = 0; q < kGroupP; ++q) {
-                if (ml[q].x == -INFINITY) continue;
-                const int e = max_shift(ml[q].x, m);
-                l += ldexp(static_cast<double>(ml[q].y), e);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) o[i] += ldexp(static_cast<double>(v[q][i]), e);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            ow[i] = f32_to_bf16_out(static_cast<float>(o[2 * i] / l)) |
-                    (static_cast<uint32_t>(f32_to_bf16_out(static_cast<float>(o[2 * i + 1] / l))) << 16);
-        uint2* dst = reinterpret_cast<uint2*>(a.out + row * kD + d0);   // out is 8-byte aligned
-        dst[0] = make_uint2(ow[0], ow[1]);
-        dst[1] = make_uint2(ow[2], ow[3]);
+        // Pieces two at a time (with 61 registers eight waves fit on a SIMD, so a 16-wave
+        // workgroup per segment at T = 16 no longer leaves half of them waiting for a CU).
+        MtSum t;
+        mt_sum_pieces<2, kCols>(a, slot0, n_pieces, 0, 1, col, d0, t);
+        m = t.m;
+        mt_write_row(a, row, d0, t, ow);
     }
     if (a.rs_hdr) mt_flag_row(a, row, m, ow, fin, seg_st, j);
 }
+
+// The same for a batch of few segments, whose pieces are many (one sequence over 256 CUs:
+// up to 128 per segment): one workgroup of 16 waves per (KV head, sequence, column tile),
+// the pieces dealt over four groups of 256 threads, four requested at a time, and the
+// groups' sums combined in order through LDS.  One sequence of 4001 positions, T = 5 (63
+// pieces per segment): 26.8 us with the kernel above, whose 32 dependent rounds of loads
+// take all of it.
+template <int kW>
+__global__ __launch_bounds__(1024) void mt_merge_wide_kernel(PrefillArgs a) {
+    constexpr int kCols = kMtTile * kW;
+    constexpr int kGroups = 4;                      // piece groups of the sums
+    constexpr int kStats = 8 + kD;
+    constexpr int kStGroups = 1024 / kStats;        // piece groups of the cached-key maxima
+    __shared__ double sum_s[kGroups - 1][10][256];
+    __shared__ uint32_t st_s[kStGroups][kStats];
+    const int kvh = blockIdx.x;
+    const int b = blockIdx.y;
+    const int64_t per_wg = a.plan_hdr[1];
+    const int lead = static_cast<int>(a.plan_hdr[2]);
+    const int64_t extra = a.plan_hdr[3];
+    const int64_t off = a.seq_off[b];
+    const int span = static_cast<int>((a.seq_off[b + 1] - off) / kHkv);
+    if (span == 0) return;                          // no keys: a start out of range, NaN rows
+    const int nk = span - lead;
+    const int64_t seg_off = off + static_cast<int64_t>(kvh) * span + lead;
+    const int64_t w_first = range_of(per_wg, extra, seg_off);
+    const int n_pieces = static_cast<int>(range_of(per_wg, extra, seg_off + nk - 1) - w_first) + 1;
+    const int64_t slot0 = w_first + static_cast<int64_t>(b) * kHkv + kvh;
+    const int64_t bh = static_cast<int64_t>(b) * kHkv + kvh;
+    const int grp = threadIdx.x >> 8;
+    const int t = threadIdx.x & 255;
+    const int col = kMtTile * blockIdx.z + (t >> 4);
+    const int j = t & 15;
+    const int d0 = 8 * j;
+    const int tok = col >> 2;
+    const bool live = tok < a.n_new;
+    const int64_t row = (static_cast<int64_t>(b) * a.n_new + min(tok, a.n_new - 1)) * kHq + kvh * kGroup + (col & 3);
+    MtFlagIn fin{};
+    uint32_t ow[4] = {0u, 0u, 0u, 0u};
+    float m = 0.f;
+    if (grp == 0 && a.rs_hdr && live) {
+        mt_flag_load(a, bh, tok, row, j, fin);
+        if (n_pieces == 1) {
+            const uint2* src = reinterpret_cast<const uint2*>(a.out + row * kD + d0);   // out is 8-byte aligned
+            const uint2 x0 = src[0], x1 = src[1];
+            ow[0] = x0.x;
+            ow[1] = x0.y;
+            ow[2] = x1.x;
+            ow[3] = x1.y;
+            m = a.rs_m[row];
+        }
+    }
+    if (a.rs_hdr && threadIdx.x < kStGroups * kStats) {
+        const int sg = threadIdx.x / kStats, e = threadIdx.x % kStats;
+        uint32_t x = 0u;
+        for (int p0 = sg; p0 < n_pieces; p0 += 4 * kStGroups) {
+            uint32_t r[4][kW];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int w = 0; w < kW; ++w) {
+                    const int p = p0 + q * kStGroups;
+                    r[q][w] = p < n_pieces ? a.piece_st[((slot0 + p) * kW + w) * kStats + e] : 0u;
+                }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int w = 0; w < kW; ++w) x = max(x, r[q][w]);
+        }
+        st_s[sg][e] = x;
+    }
+    MtSum acc;
+    if (live && n_pieces > 1) {
+        mt_sum_pieces<4, kCols>(a, slot0, n_pieces, grp, kGroups, col, d0, acc);
+        if (grp > 0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum_s[grp - 1][i][t] = acc.o[i];
+            sum_s[grp - 1][8][t] = acc.l;
+            sum_s[grp - 1][9][t] = static_cast<double>(acc.m);
+        }
+    }
+    __syncthreads();
+    if (a.rs_hdr && threadIdx.x < kStats) {
+        uint32_t x = st_s[0][threadIdx.x];
+#pragma unroll
+        for (int i = 1; i < kStGroups; ++i) x = max(x, st_s[i][threadIdx.x]);
+        st_s[0][threadIdx.x] = x;
+    }
+    __syncthreads();
+    if (grp > 0 || !live) return;
+    if (n_pieces > 1) {
+#pragma unroll
+        for (int gi = 0; gi < kGroups - 1; ++gi) {
+            const float mg = static_cast<float>(sum_s[gi][9][t]);
+            if (mg == -INFINITY) continue;
+            const float mb = fmaxf(acc.m, mg);
+            const int ea = acc.m == mb ? 0 : max_shift(acc.m, mb);
+            const int eg = max_shift(mg, mb);
+            acc.l = ldexp(acc.l, ea) + ldexp(sum_s[gi][8][t], eg);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc.o[i] = ldexp(acc.o[i], ea) + ldexp(sum_s[gi][i][t], eg);
+            acc.m = mb;
+        }
+        m = acc.m;
+        mt_write_row(a, row, d0, acc, ow);
+    }
+    if (a.rs_hdr) mt_flag_row(a, row, m, ow, fin, st_s[0], j);
+}
+
+// Segments so few that one has this many pieces or more take the wide merge: below it the
+// segments' own workgroups fill the chip and their rounds of loads are few.
+constexpr int kMtWidePieces = 16;
 
 template <int kW>
 hipError_t launch_multi_w(const PrefillArgs& a, hipStream_t stream, hipEvent_t* ev) {
@@ -1309,7 +1455,11 @@ hipError_t launch_multi_w(const PrefillArgs& a, hipStream_t stream, hipEvent_t* 
     e = hipGetLastError();
     if (ev) (void)hipEventRecord(ev[2], stream);
     if (e != hipSuccess) return done(3, e);
-    hipLaunchKernelGGL(mt_merge_kernel<kW>, dim3(kHkv, static_cast<unsigned>(a.batch)), dim3(256 * kW), 0, stream, a);
+    if (a.n_wgs >= static_cast<int64_t>(kMtWidePieces) * kHkv * a.batch)
+        hipLaunchKernelGGL(mt_merge_wide_kernel<kW>, dim3(kHkv, static_cast<unsigned>(a.batch), kW), dim3(1024), 0,
+                           stream, a);
+    else
+        hipLaunchKernelGGL(mt_merge_kernel<kW>, dim3(kHkv, static_cast<unsigned>(a.batch)), dim3(256 * kW), 0, stream, a);
     e = hipGetLastError();
     if (ev) (void)hipEventRecord(ev[3], stream);
     return e;

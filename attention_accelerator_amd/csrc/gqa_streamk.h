@@ -92,10 +92,10 @@ __device__ __forceinline__ int64_t range_extra(int64_t per, int skew_pm) {
     return per * skew_pm / 1000 / kRangeAlign * kRangeAlign;
 }
 
-// Range size for `total` stream positions over n_wgs workgroups.
-__device__ __forceinline__ int64_t range_size(int64_t total, int n_wgs) {
+// Range size for `total` stream positions over n_wgs workgroups, at least min_keys.
+__device__ __forceinline__ int64_t range_size(int64_t total, int n_wgs, int min_keys) {
     int64_t per = (total + n_wgs - 1) / n_wgs;
-    per = per < kMinRangeKeys ? kMinRangeKeys : per;
+    per = per < min_keys ? min_keys : per;
     return (per + kRangeAlign - 1) / kRangeAlign * kRangeAlign;
 }
 
@@ -105,8 +105,9 @@ __device__ __forceinline__ int64_t range_size(int64_t total, int n_wgs) {
 // kSegLead is cut to a quarter of the lead-free range size (never below kSegLead), so that
 // a range always reaches past a lead into keys.
 __device__ __forceinline__ void plan_lead_totals(int64_t sum, int max_keys, int n_seq, int n_wgs, int& lead,
-                                                 int64_t& total, int64_t& per_wg, int seg_lead = kSegLead) {
-    const int64_t per0 = range_size(sum * kHkv, n_wgs);
+                                                 int64_t& total, int64_t& per_wg, int seg_lead = kSegLead,
+                                                 int min_keys = kMinRangeKeys) {
+    const int64_t per0 = range_size(sum * kHkv, n_wgs, min_keys);
     int want = seg_lead;
     if (want > kSegLead) {
         const int64_t quarter = per0 / 4 / kRangeAlign * kRangeAlign;
@@ -114,7 +115,7 @@ __device__ __forceinline__ void plan_lead_totals(int64_t sum, int max_keys, int 
     }
     lead = static_cast<int64_t>(max_keys) < kLeadRanges * per0 ? want : 0;
     total = (sum + static_cast<int64_t>(n_seq) * lead) * kHkv;
-    per_wg = range_size(total, n_wgs);
+    per_wg = range_size(total, n_wgs, min_keys);
 }
 
 }  // namespace gqa

@@ -335,3 +335,28 @@ def test_every_row_rescored(dev, n_new, rope_q, rope_k):
     assert np.all(got[..., 5] == 0)
     w = _check(want, got.reshape(-1, 128), f"T={n_new} rope_q={rope_q} rope_k={rope_k}, all rows rescored")
     print("worst ULP", w)
+
+
+@pytest.mark.parametrize("n_new,starts", [
+    (1, [2047]),              # 2048 keys: the first length cut into ranges of 128
+    (4, [1100]),              # 64-key ranges, 18 pieces a segment (wide merge, one column tile)
+    (5, [2300, 1]),           # a long and a one-piece segment in one wide merge
+    (8, [40, -1, 2500]),      # an invalid start (NaN rows) between them
+    (16, [2100]),             # four column tiles
+])
+def test_multi_few_segments(dev, n_new, starts):
+    """Few segments of many pieces: the wide merge and the longer smallest range."""
+    ok = [s >= 0 for s in starts]
+    cap = max(starts) + n_new + 5
+    q, kn, vn, k, v = _chunk([max(s, 0) for s in starts], n_new, cap, 70 + n_new)
+    st = torch.tensor(starts, dtype=torch.int32, device=dev)
+    got, _, _ = _run(q, kn, vn, k, v, st, dev)
+    again, _, _ = _run(q, kn, vn, k, v, st, dev)
+    assert np.array_equal(got, again)
+    for b, s in enumerate(starts):
+        if not ok[b]:
+            assert (got[b] == 0x7FC0).all()
+            continue
+        sl = slice(b, b + 1)
+        want = _oracle(q[sl], kn[sl], vn[sl], k[sl], v[sl], [s])
+        _check(want, got[b].reshape(-1, 128), f"T={n_new} start={s}")
