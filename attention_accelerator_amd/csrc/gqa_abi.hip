@@ -34,6 +34,13 @@ constexpr int32_t kWavesPerCu = 4;
 // the stream path cost more than the HBM traffic.  GQA_PLAN_STREAM_K turns it off.
 constexpr int64_t kSingleLaunchMaxKeys = int64_t{1} << 18;
 
+// The one-launch path's piece counters sit kCounterPad words (128 bytes) apart for up to
+// kPaddedCounters segments: side by side, every piece of a batch counted in the same cache
+// line, one atomic after the other (B=1 L=4096, 256 pieces: 14.0 us, apart 11.9 us).  With
+// more segments the pieces of each are few and their ends spread.
+constexpr int64_t kPaddedCounters = 512;
+constexpr int32_t kCounterPad = 16;
+
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 int32_t device_stream_wgs() {
@@ -135,14 +142,17 @@ DecodePlan plan_decode(const gqa_params_t* params, int32_t batch, int32_t capaci
     const int64_t keys_cap = static_cast<int64_t>(batch) * kHkv * capacity;
     const bool single_fits = max_single_segments < 0 || static_cast<int64_t>(batch) * kHkv <= max_single_segments;
     if (!paged && (params->flags & GQA_PLAN_STREAM_K) == 0u && keys_cap <= kSingleLaunchMaxKeys && single_fits) {
-        // Single launch: about one 4-wave workgroup per CU (n_wgs / 4), pieces of at least
-        // 256 keys (64 per wave: below that the last piece's merge of more partials costs
-        // more than the shorter streams save; B=1 L=4096 runs in 18.7 us with 256-key pieces,
-        // 20.7 us with 128) in multiples of 64, sized from the capacity (the lengths live on
-        // the device); pieces past a sequence's length exit at once.
+        // Single launch: about one 4-wave workgroup per CU (n_wgs / 4), pieces in multiples of
+        // 64 keys sized from the capacity (the lengths live on the device; there a segment of up
+        // to 128 keys is one piece); pieces past a sequence's length exit at once.  A piece is
+        // at least 64 keys (one chunk per wave) while that gives at most 16 pieces, else 128:
+        // shorter chains per wave, until counting and merging more pieces costs as much.  B=1,
+        // smallest piece 64 / 128 / 256 keys: L=1024 8.2 / 9.0 / 10.8 us, L=2048 10.2 / 9.2 /
+        // 10.9, L=4096 11.1 / 11.2 / 11.3 (RoPE on K 14.1 / 14.0 / 15.6).
         const int64_t n_pieces = plan.n_wgs / 4 > 0 ? plan.n_wgs / 4 : 1;
         int64_t pk = (keys_cap + n_pieces - 1) / n_pieces;
-        pk = pk < 256 ? 256 : (pk + 63) / 64 * 64;
+        const int64_t pk_min = capacity <= 1024 ? 64 : 128;
+        pk = pk < pk_min ? pk_min : (pk + 63) / 64 * 64;
         plan.piece_keys = static_cast<int32_t>(pk);
         plan.pieces_cap = static_cast<int32_t>((capacity + pk - 1) / pk);
         plan.n_slots = static_cast<int64_t>(batch) * kHkv * plan.pieces_cap;
@@ -154,7 +164,9 @@ DecodePlan plan_decode(const gqa_params_t* params, int32_t batch, int32_t capaci
     }
     plan.part_o_bytes = align_up(static_cast<size_t>(plan.n_slots) * kGroup * kD * sizeof(double), 256);
     plan.part_ml_bytes = align_up(static_cast<size_t>(plan.n_slots) * kGroup * sizeof(double2), 256);
-    plan.count_bytes = align_up(static_cast<size_t>(batch) * kHkv * sizeof(unsigned long long), 256);
+    plan.count_stride = batch * static_cast<int64_t>(kHkv) <= kPaddedCounters ? kCounterPad : 1;
+    plan.count_bytes =
+        align_up(static_cast<size_t>(batch) * kHkv * plan.count_stride * sizeof(unsigned long long), 256);
     plan.workspace_bytes =
         plan.part_o_bytes + plan.part_ml_bytes + plan.q_op_bytes + plan.plan_bytes + plan.count_bytes;
     return plan;
@@ -304,6 +316,7 @@ int decode_launch(const DecodePlan& plan, const gqa_params_t* params, const uint
     a.seg_count = counters ? counters : reinterpret_cast<unsigned long long*>(pl + plan.plan_bytes);
     a.pieces_cap = plan.pieces_cap;
     a.piece_keys = plan.piece_keys;
+    a.count_stride = plan.count_stride;
     a.block_table = block_table;
     a.max_blocks = max_blocks;
     a.n_blocks = n_blocks;

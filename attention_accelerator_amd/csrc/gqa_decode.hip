@@ -192,11 +192,84 @@ __device__ __forceinline__ double exp2_f64(double x) {
     return ldexp(y, static_cast<int>(fmax(n, -2000.0)));
 }
 
+// ---- RoPE on cached K rows (a cache kept before rotation).  A lane of a 16-key chunk rotates 16
+// pairs of key kc + d, d = lane % 16.  Its (cos, sin) come from the chunk's first position kc,
+// one sincos per lane for the 64 frequencies shared through LDS, turned by the angle of d,
+// a table of 16 rotations per frequency that a workgroup forms once: rot(kc + d) = rot(kc)
+// rot(d).  Both are formed for the exact angles kc f and d f (the rounding error of the product,
+// which fma gives, turned back), and the result turned by the rounding error of (kc + d) f:
+// the golden rotates at the rounded angle.  Largest error against 113-bit values over positions
+// up to 400,000: 3.2e-16, rms 6.0e-17 (a sincos of the library per pair: 2.5e-16 and
+// 6.2e-17), in 12 fp64 instructions per pair instead of about 110.  Decode of 8 x 4096
+// unrotated keys: 80.8 us with that sincos per pair, 39.0 us so.
+struct KRopeLds {
+    double2 rot[16][kWave];           // [pair 8kb + j][lane]: (cos, sin) of (lane % 16) f
+    double2 base[4][kPairs];          // each wave's current chunk: (cos, sin) of kc f
+    double freq[kPairs];
+};
+
+__device__ __forceinline__ KRopeLds& k_rope_lds() {
+    __shared__ KRopeLds t;
+    return t;
+}
+
+// cos and sin of the exact product p * f.
+__device__ __forceinline__ double2 rot_exact(double p, double f) {
+    const double ang = p * f;
+    const double dl = fma(p, f, -ang);
+    double s, c;
+    sincos_f64(ang, s, c);
+    return make_double2(fma(-dl, s, c), fma(dl, c, s));
+}
+
+// The table (every thread of the workgroup, once; ends with a barrier).
+__device__ __forceinline__ void k_rope_init(const RopeTable& rope) {
+    KRopeLds& t = k_rope_lds();
+#pragma unroll 2
+    for (int i = threadIdx.x; i < 16 * kWave; i += blockDim.x) {
+        const int l = i & (kWave - 1), pair = i >> 6;
+        t.rot[pair][l] = rot_exact(l & 15, rope.inv_freq[32 * (pair >> 3) + 8 * (l >> 4) + (pair & 7)]);
+    }
+    if (threadIdx.x < kPairs) t.freq[threadIdx.x] = rope.inv_freq[threadIdx.x];
+    __syncthreads();
+}
+
+// The chunk's K values (lane: key kc + lane % 16) rotated in double.
+__device__ __forceinline__ void k_rope_rotate(int kc, const Chunk& c, double (&kr)[4][8]) {
+    KRopeLds& t = k_rope_lds();
+    const int lane = threadIdx.x & (kWave - 1);
+    const int g = lane >> 4;
+    double2* base = t.base[(threadIdx.x >> 6) & 3];
+    base[lane] = rot_exact(kc, t.freq[lane]);        // (one wave: its LDS accesses run in order)
+    const double pos = kc + (lane & 15);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+        float xf[8], yf[8];
+        unpack8(c.kw[kb], xf);
+        unpack8(c.kw[kb + 2], yf);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int fi = 32 * kb + 8 * g + j;
+            const double2 b = base[fi];
+            const double2 d = t.rot[8 * kb + j][lane];
+            const double f = t.freq[fi];
+            const double ang = pos * f;
+            const double dl = fma(pos, f, -ang);
+            const double cs0 = b.x * d.x - b.y * d.y;
+            const double sn0 = b.y * d.x + b.x * d.y;
+            const double cs = fma(dl, sn0, cs0);
+            const double sn = fma(-dl, cs0, sn0);
+            const double x = xf[j], y = yf[j];
+            kr[kb][j] = x * cs - y * sn;
+            kr[kb + 2][j] = x * sn + y * cs;
+        }
+    }
+}
+
 // Scores, online softmax and weighted V of one chunk [kc, kc+16) (keys >= k_b masked).
-// kRope: each K row is rotated first, at position rope_pos0 + its key index.
+// kRope: each K row is rotated first, at its key index (k_rope_init has run).
 template <int kRope>
-__device__ __forceinline__ void compute_chunk(const RopeTable& rope, int rope_pos0, int kc, int k_b, const Chunk& c,
-                                              const QOps& qa, PieceState& st) {
+__device__ __forceinline__ void compute_chunk(int kc, int k_b, const Chunk& c, const QOps& qa, PieceState& st) {
     // p exchange slice of this wave (workgroups of up to four waves).
     __shared__ double p_lds[4][kWave];
     double* pl = p_lds[(threadIdx.x >> 6) & 3];
@@ -205,23 +278,8 @@ __device__ __forceinline__ void compute_chunk(const RopeTable& rope, int rope_po
     double s4[4] = {0.0, 0.0, 0.0, 0.0};
     if (kRope) {
         // Rotate the K row at its position in double: pairs (kb, kb+2) of this lane.
-        const int kkey = kc + (lane & 15);
-        const int g = lane >> 4;
         double kr[4][8];
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            float xf[8], yf[8];
-            unpack8(c.kw[kb], xf);
-            unpack8(c.kw[kb + 2], yf);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int fi = 32 * kb + 8 * g + j;
-                double xr, yr;
-                rope_pair(xf[j], yf[j], rope_pos0 + kkey, rope.inv_freq[fi], xr, yr);
-                kr[kb][j] = xr;
-                kr[kb + 2][j] = yr;
-            }
-        }
+        k_rope_rotate(kc, c, kr);
 #pragma unroll
         for (int e = 0; e < 8; ++e)
 #pragma unroll
@@ -613,9 +671,9 @@ __device__ __forceinline__ void process_piece(const DecodeArgs& a, int b, int kv
     const int n_chunks = (k_b - k_a + kChunk - 1) / kChunk;
     for (int i = 0;; i += 2) {
         load_cur_or_next(true, cur, nxt, step, c1);
-        compute_chunk<kRopeK>(a.rope, 0, k_a + i * kChunk, k_b, c0, qa, st);
+        compute_chunk<kRopeK>(k_a + i * kChunk, k_b, c0, qa, st);
         load_cur_or_next(i + 2 < n_chunks, cur, nxt, step, c0);
-        if (i + 1 < n_chunks) compute_chunk<kRopeK>(a.rope, 0, k_a + (i + 1) * kChunk, k_b, c1, qa, st);
+        if (i + 1 < n_chunks) compute_chunk<kRopeK>(k_a + (i + 1) * kChunk, k_b, c1, qa, st);
         if (i + 2 >= n_chunks) break;
     }
 
@@ -700,6 +758,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void
             sw = t;
         }
     }
+    if (kRopeK) k_rope_init(a.rope);
     sw.lead = lead;
     int kvh, key, nvb;
     locate_first_piece(off, next, lead, x, kvh, key, nvb);
@@ -854,7 +913,7 @@ __device__ __forceinline__ void process_page_piece(const DecodeArgs& a, const Pa
                 all_ok = all_ok && ok;
                 id_next = id_after;
             }
-            compute_chunk<kRopeK>(a.rope, 0, k_a + i * kChunk, kend, c0, qa, st);
+            compute_chunk<kRopeK>(k_a + i * kChunk, kend, c0, qa, st);
             {
                 const bool last = i + 2 >= n_chunks;
                 const bool to_next = last && has_next;
@@ -870,7 +929,7 @@ __device__ __forceinline__ void process_page_piece(const DecodeArgs& a, const Pa
                     all_ok = all_ok && ok;
                 id_next = id_after;
             }
-            if (i + 1 < n_chunks) compute_chunk<kRopeK>(a.rope, 0, k_a + (i + 1) * kChunk, kend, c1, qa, st);
+            if (i + 1 < n_chunks) compute_chunk<kRopeK>(k_a + (i + 1) * kChunk, kend, c1, qa, st);
             if (i + 2 >= n_chunks) break;
         }
     } else if (has_next) {
@@ -917,6 +976,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void
             sw = t;
         }
     }
+    if (kRopeK) k_rope_init(a.rope);
     PagePiece cur;
     {
         sw.lead = lead;
@@ -1068,6 +1128,35 @@ __global__ __launch_bounds__(kGroup * kWave) void decode_merge_kernel(DecodeArgs
 // workspace needs zeroing (gqa_decode_workspace_init) before its first use only.
 
 constexpr int kSingleWaves = 4;
+constexpr int kSingleOnePiece = 128;
+
+// Sums the partials of n_pieces <= kN pieces (slots from slot0) of head h, dims 2*lane and
+// 2*lane + 1.
+template <int kN>
+__device__ __forceinline__ void merge_at_once(const DecodeArgs& a, int64_t slot0, int n_pieces, int h, double& l,
+                                              double& o0, double& o1) {
+    const int lane = threadIdx.x & (kWave - 1);
+    // lane u < kN holds piece u's (m, l) (copies of the last piece past n_pieces)
+    double2 ov[kN];
+    const double2 mlu = load_agent_d2(reinterpret_cast<const double*>(
+        a.part_ml + (slot0 + min(lane & (kN - 1), n_pieces - 1)) * kGroup + h));
+#pragma unroll
+    for (int u = 0; u < kN; ++u) {
+        const int p = min(u, n_pieces - 1);
+        ov[u] = load_agent_d2(a.part_o + ((slot0 + p) * kGroup + h) * kD + 2 * lane);
+    }
+    const double m_all = wave_max_f64(mlu.x);     // copies of the last piece add nothing
+    const int e_l = lane < n_pieces ? max_shift_f64(mlu.x, m_all) : -1100;
+    // l over the lanes that hold a piece; O piece by piece, each weight from its lane.
+    l = row16_sum_f64(lane < n_pieces ? ldexp(mlu.y, e_l) : 0.0);
+    l = swap_add_f64<true>(swap_add_f64<false>(l));
+#pragma unroll
+    for (int u = 0; u < kN; ++u) {
+        const int e = __builtin_amdgcn_readlane(e_l, u);
+        o0 += ldexp(ov[u].x, e);
+        o1 += ldexp(ov[u].y, e);
+    }
+}
 
 template <bool kRopeQ, bool kRopeK>
 __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(DecodeArgs a) {
@@ -1082,6 +1171,11 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
     const int kvh = seg % kHkv;
     const int wave = threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
+    // The wave's Q row, requested with the lengths (it exists whatever they are): behind the K/V
+    // loads its values would wait for those (loads return in order).
+    const uint16_t* qrow = a.q + (static_cast<int64_t>(b) * kHq + kvh * kGroup + wave) * kD;
+    const uint16_t qx = qrow[lane], qy = qrow[lane + kPairs];
+    const double freq = kRopeQ ? a.rope.inv_freq[lane] : 0.0;
     const int nv = seq_valid_keys(a, b);
     if (nv == 0) {
         if (kvh == 0 && piece == 0) {
@@ -1091,11 +1185,16 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
         }
         return;
     }
-    const int n_pieces = (nv + a.piece_keys - 1) / a.piece_keys;
+    // A segment of up to kSingleOnePiece keys is one piece: no partial, no count.
+    const int piece_keys = nv <= kSingleOnePiece ? max(a.piece_keys, kSingleOnePiece) : a.piece_keys;
+    const int n_pieces = (nv + piece_keys - 1) / piece_keys;
     if (piece >= n_pieces) return;                       // uniform over the workgroup
-    const int quarter = a.piece_keys / kSingleWaves;
-    const int k_a = min(nv, piece * a.piece_keys + wave * quarter);
-    const int k_b = min(nv, k_a + quarter);
+    // A quarter of the piece's keys per wave, in whole chunks (the last piece may be short).
+    const int p_a = piece * piece_keys;
+    const int p_b = min(nv, p_a + piece_keys);
+    const int quarter = (p_b - p_a + kSingleWaves * kChunk - 1) / (kSingleWaves * kChunk) * kChunk;
+    const int k_a = min(p_b, p_a + wave * quarter);
+    const int k_b = min(p_b, k_a + quarter);
     const bool busy = k_a < k_b;                         // uniform over the wave
 
     // First chunk of this wave's quarter, requested before the Q operands are formed.
@@ -1108,12 +1207,10 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
     // Q operands: wave h rotates and scales Q head 4*kvh + h into q_s; every wave then
     // reads its QOps back.
     {
-        const int qpos = a.query_pos[b];
         double sn = 0.0, cs = 1.0;
-        if (kRopeQ) rope_sincos(qpos, a.rope.inv_freq[lane], sn, cs);
-        const uint16_t* qrow = a.q + (static_cast<int64_t>(b) * kHq + kvh * kGroup + wave) * kD;
-        const double x = bf16_to_f32(qrow[lane]);
-        const double y = bf16_to_f32(qrow[lane + kPairs]);
+        if (kRopeQ) rope_sincos(a.query_pos[b], freq, sn, cs);
+        const double x = bf16_to_f32(qx);
+        const double y = bf16_to_f32(qy);
         double xr = x, yr = y;
         if (kRopeQ) {
             xr = x * cs - y * sn;
@@ -1122,7 +1219,10 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
         q_s[wave][lane] = xr * a.qk_scale_log2;
         q_s[wave][lane + kPairs] = yr * a.qk_scale_log2;
     }
-    __syncthreads();
+    if (kRopeK)
+        k_rope_init(a.rope);                             // (ends with a barrier)
+    else
+        __syncthreads();
     QOps qa;
     read_q_ops(&q_s[0][0], qa);
 
@@ -1132,10 +1232,10 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
         const int n_chunks = (k_b - k_a + kChunk - 1) / kChunk;
         for (int i = 0;; i += 2) {
             load_next(cur, step, c1);
-            compute_chunk<kRopeK>(a.rope, 0, k_a + i * kChunk, k_b, c0, qa, st);
+            compute_chunk<kRopeK>(k_a + i * kChunk, k_b, c0, qa, st);
             if (i + 1 >= n_chunks) break;
             load_next(cur, step, c0);
-            compute_chunk<kRopeK>(a.rope, 0, k_a + (i + 1) * kChunk, k_b, c1, qa, st);
+            compute_chunk<kRopeK>(k_a + (i + 1) * kChunk, k_b, c1, qa, st);
             if (i + 2 >= n_chunks) break;
         }
     }
@@ -1195,37 +1295,23 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
     __syncthreads();
     // Count finished pieces (device-scope atomic); the last piece merges and resets the
     // counter for the next call on this workspace.
-    if (threadIdx.x == 0) last_s = atomicAdd(&a.seg_count[seg], 1ull) == static_cast<unsigned long long>(n_pieces - 1);
+    if (threadIdx.x == 0) last_s = atomicAdd(&a.seg_count[static_cast<int64_t>(seg) * a.count_stride], 1ull) == static_cast<unsigned long long>(n_pieces - 1);
     __syncthreads();
     if (!last_s) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    if (threadIdx.x == 0) __hip_atomic_store(&a.seg_count[seg], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) __hip_atomic_store(&a.seg_count[static_cast<int64_t>(seg) * a.count_stride], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
     // Merge the segment's pieces, wave h for head h (lane owns dims 2*lane, 2*lane + 1), in
-    // piece order.  Up to 16 pieces: every (m, l) and O row requested at once.  More: the
-    // (m, l) of 64 pieces per pass, one per lane, first, then the O rows 16 at a time.
+    // piece order.  Up to 32 pieces (every plan of one launch but those with stream_wgs raised):
+    // each (m, l) and O row requested at once.  More: the (m, l) of 64 pieces per pass, one
+    // per lane, first, then the O rows 16 at a time.
     l = 0.0;
     o0 = 0.0;
     o1 = 0.0;
     if (n_pieces <= 16) {
-        // lane u < 16 holds piece u's (m, l) (copies of the last piece past n_pieces)
-        double2 ov[16];
-        const double2 mlu = load_agent_d2(reinterpret_cast<const double*>(
-            a.part_ml + (slot0 + min(lane & 15, n_pieces - 1)) * kGroup + h));
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int p = min(u, n_pieces - 1);
-            ov[u] = load_agent_d2(a.part_o + ((slot0 + p) * kGroup + h) * kD + 2 * lane);
-        }
-        const double m_all = wave_max_f64(mlu.x);     // copies of the last piece add nothing
-        const int e_l = (lane & 15) < n_pieces ? max_shift_f64(mlu.x, m_all) : -1100;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int e = __shfl(e_l, u);
-            l += ldexp(__shfl(mlu.y, u), e);
-            o0 += ldexp(ov[u].x, e);
-            o1 += ldexp(ov[u].y, e);
-        }
+        merge_at_once<16>(a, slot0, n_pieces, h, l, o0, o1);
+    } else if (n_pieces <= 32) {
+        merge_at_once<32>(a, slot0, n_pieces, h, l, o0, o1);
     } else {
         double m_all = -INFINITY;
         for (int p0 = 0; p0 < n_pieces; p0 += kWave) {

@@ -23,7 +23,8 @@ struct DecodeArgs {
     int32_t* seq_nreal;       // [B] keys of sequence b that count (n_valid; the plan pads to blocks)
     double* part_o;           // [n_slots][4][128] unnormalised partial outputs
     double2* part_ml;         // [n_slots][4] (integer-valued running max in log2 units, sum)
-    unsigned long long* seg_count;  // [B*8] pieces finished per segment, single-launch path (zero between calls)
+    unsigned long long* seg_count;  // [B*8] pieces finished per segment, single-launch path (zero between
+                                    // calls), count_stride words apart
     const int32_t* block_table;  // paged cache: [B][max_blocks] block ids (nullptr: contiguous cache)
     int64_t kv_batch_stride;  // contiguous: elements per sequence; paged: per block of the pool
     int64_t kv_head_stride;
@@ -36,6 +37,7 @@ struct DecodeArgs {
     int32_t skew_pm;          // stream and paged kernels: XCD weighting of the ranges (per mille)
     int32_t pieces_cap;       // > 0: single-launch path, pieces per segment (grid x)
     int32_t piece_keys;       // single-launch path: keys per piece
+    int32_t count_stride;
     double qk_scale_log2;     // scale * log2(e), folded into Q
     uint32_t flags;           // bit0 RoPE on Q, bit1 RoPE on K
     RopeTable rope;
@@ -47,6 +49,7 @@ struct DecodePlan {
     int32_t n_wgs;
     int32_t pieces_cap;       // > 0 selects the single-launch path
     int32_t piece_keys;
+    int32_t count_stride;     // words between two segments' counters
     int64_t n_slots;          // stream path: n_wgs + 8 * batch; single path: 8 * batch * pieces_cap
     size_t part_o_bytes;      // fp64 partial outputs at offset 0
     size_t part_ml_bytes;     // then the (m, l) pairs
