@@ -38,6 +38,8 @@ EXPORTS = (
     "gqa_decode_paged_workspace_bytes",
     "gqa_decode_paged_bf16",
     "gqa_kv_append_paged_bf16",
+    "gqa_decode_host_workspace_bytes",
+    "gqa_decode_host_bf16",
     "gqa_prefill_workspace_bytes",
     "gqa_prefill_bf16",
     "gqa_prefill_rescored_rows_offset",
@@ -128,6 +130,10 @@ def lib() -> ctypes.CDLL:
                                   ctypes.POINTER(GqaKvLayout), vp, vp, ctypes.c_int32, vp, vp,
                                   ctypes.c_size_t, vp]
     L.gqa_decode_bf16.restype = ctypes.c_int
+    L.gqa_decode_host_workspace_bytes.argtypes = L.gqa_decode_workspace_bytes.argtypes
+    L.gqa_decode_host_workspace_bytes.restype = ctypes.c_size_t
+    L.gqa_decode_host_bf16.argtypes = L.gqa_decode_bf16.argtypes
+    L.gqa_decode_host_bf16.restype = ctypes.c_int
     L.gqa_decode_bf16_noalloc.argtypes = [ctypes.POINTER(GqaParams), vp, vp, vp,
                                           ctypes.POINTER(GqaKvLayout), vp, vp, ctypes.c_int32, vp, vp]
     L.gqa_decode_bf16_noalloc.restype = ctypes.c_int

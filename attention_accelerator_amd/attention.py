@@ -29,6 +29,7 @@ ROPE_THETA = 500000.0
 DEFAULT_SCALE = 1.0 / math.sqrt(HEAD_DIM)
 
 Lengths = Union[int, Sequence[int], torch.Tensor]
+_I32P = ctypes.POINTER(ctypes.c_int32)
 
 
 def make_params(*, rope_q: bool = True, rope_k: bool = False, theta: float = ROPE_THETA,
@@ -54,6 +55,21 @@ def _plan_key(p: GqaParams, batch: int, capacity: int):
 
 def _stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def _lengths_on_host(x: Lengths, batch: int, name: str):
+    """Host values as `batch` int32 entries: an object whose address a C call can take (a
+    ctypes array or a tensor) and that address."""
+    if type(x) is int and batch == 1 and -0x80000000 <= x <= 0x7FFFFFFF:
+        arr = ctypes.c_int32(x)
+        return arr, ctypes.addressof(arr)
+    host = torch.as_tensor(x, dtype=torch.int32).reshape(-1)
+    if host.numel() == 1 and batch > 1:
+        host = host.expand(batch)
+    if host.numel() != batch:
+        raise ValueError(f"{name} has {host.numel()} entries for a batch of {batch}")
+    host = host.contiguous()
+    return host, host.data_ptr()
 
 
 def _lengths_to_device(x: Lengths, batch: int, device: torch.device, name: str):
@@ -123,7 +139,7 @@ def gqa_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     rope_q / rope_k: rotate Q at query_position / each K row at its position
              (the reference core does both; a cache stored post-RoPE sets rope_k=False)
     workspace: from new_workspace(B, S, device) to reuse across calls (else one is
-             allocated and prepared per call)
+             allocated per call, and prepared where the lengths are device tensors)
     Returns out [.., 32, 128] bfloat16.  Key p contributes iff p < seq_len and
     p <= query_position.  Raises GqaConfigError for what the reference rejects."""
     single = q.dim() == 2
@@ -147,33 +163,47 @@ def gqa_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     p = params or make_params(rope_q=rope_q, rope_k=rope_k, theta=theta, scale=scale,
                               n_q_heads=q.shape[1], n_kv_heads=k_cache.shape[1],
                               head_dim=q.shape[2])
-    sl_dev, sl_host = _lengths_to_device(seq_len, batch, device, "seq_len")
-    qp_dev, qp_host = _lengths_to_device(query_position, batch, device, "query_position")
-    if sl_host is not None and qp_host is not None:
-        check(lib().gqa_validate_lengths(
-            ctypes.cast(sl_host.data_ptr(), ctypes.POINTER(ctypes.c_int32)),
-            ctypes.cast(qp_host.data_ptr(), ctypes.POINTER(ctypes.c_int32)), batch, capacity),
-            "gqa_validate_lengths")
-    ws_bytes = int(lib().gqa_decode_workspace_bytes(ctypes.byref(p), batch, capacity))
-    if ws_bytes == 0:
-        check(_lib.GQA_ERR_INVALID_CONFIG, "gqa_decode_workspace_bytes")
-    if workspace is None:
-        workspace = new_workspace(batch, capacity, device, p)
-    elif workspace.numel() * workspace.element_size() < ws_bytes:
-        raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} bytes; "
-                         f"{ws_bytes} needed")
-    _check_workspace_plan(workspace, p, batch, capacity)
+    # Without a workspace of the caller's, host lengths travel with the launches of one call (as
+    # copies to the GPU each would wait for it, and a fresh workspace would be cleared first).
+    host_lens = workspace is None and not any(isinstance(x, torch.Tensor) and x.is_cuda
+                                              for x in (seq_len, query_position))
+    if host_lens:
+        sl_keep, sl_ptr = _lengths_on_host(seq_len, batch, "seq_len")
+        qp_keep, qp_ptr = _lengths_on_host(query_position, batch, "query_position")
+        ws_bytes = int(lib().gqa_decode_host_workspace_bytes(ctypes.byref(p), batch, capacity))
+        # lengths are checked before the configuration, as for device copies of them
+        check(lib().gqa_validate_lengths(ctypes.cast(sl_ptr, _I32P), ctypes.cast(qp_ptr, _I32P), batch, capacity),
+              "gqa_validate_lengths")
+        if ws_bytes == 0:
+            check(_lib.GQA_ERR_INVALID_CONFIG, "gqa_decode_workspace_bytes")
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+    else:
+        sl_dev, sl_host = _lengths_to_device(seq_len, batch, device, "seq_len")
+        qp_dev, qp_host = _lengths_to_device(query_position, batch, device, "query_position")
+        if sl_host is not None and qp_host is not None:
+            check(lib().gqa_validate_lengths(ctypes.cast(sl_host.data_ptr(), _I32P),
+                                             ctypes.cast(qp_host.data_ptr(), _I32P), batch, capacity),
+                  "gqa_validate_lengths")
+        ws_bytes = int(lib().gqa_decode_workspace_bytes(ctypes.byref(p), batch, capacity))
+        if ws_bytes == 0:
+            check(_lib.GQA_ERR_INVALID_CONFIG, "gqa_decode_workspace_bytes")
+        if workspace is None:
+            workspace = new_workspace(batch, capacity, device, p)
+        elif workspace.numel() * workspace.element_size() < ws_bytes:
+            raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} bytes; "
+                             f"{ws_bytes} needed")
+        _check_workspace_plan(workspace, p, batch, capacity)
+        sl_ptr, qp_ptr = sl_dev.data_ptr(), qp_dev.data_ptr()
     if out is None:
         out = torch.empty((batch, q.shape[1], q.shape[2]), dtype=torch.bfloat16, device=device)
     elif out.shape != (batch, q.shape[1], q.shape[2]) or out.dtype != torch.bfloat16 \
             or not out.is_contiguous():
         raise ValueError("out must be a contiguous bfloat16 [B,32,128] tensor")
     layout = GqaKvLayout(k_cache.stride(0), k_cache.stride(1), k_cache.stride(2), capacity)
-    status = lib().gqa_decode_bf16(
-        ctypes.byref(p), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-        ctypes.byref(layout), sl_dev.data_ptr(), qp_dev.data_ptr(), batch, out.data_ptr(),
-        workspace.data_ptr(), workspace.numel() * workspace.element_size(),
-        _stream_handle(device))
+    fn = lib().gqa_decode_host_bf16 if host_lens else lib().gqa_decode_bf16
+    status = fn(ctypes.byref(p), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                ctypes.byref(layout), sl_ptr, qp_ptr, batch, out.data_ptr(), workspace.data_ptr(),
+                workspace.numel() * workspace.element_size(), _stream_handle(device))
     check(status, "gqa_decode_bf16")
     return out[0] if single else out
 

@@ -16,7 +16,18 @@ namespace gqa {
 
 void fill_rope_table(double theta, RopeTable* t) {
     // angle = position * theta ** (-2.0 * i / 128), pyfiles/gen_gqa_wrapper_vectors.py:30.
-    for (int i = 0; i < kPairs; ++i) t->inv_freq[i] = std::pow(theta, (-2.0 * i) / kD);
+    // The 64 powers take a few microseconds, as long as the launch of a small call: each host
+    // thread keeps the table of the last theta it was given.
+    struct Last {
+        double theta;
+        RopeTable table;
+    };
+    thread_local Last last{0.0, {}};                 // (theta is positive wherever it is used)
+    if (last.theta != theta) {
+        for (int i = 0; i < kPairs; ++i) last.table.inv_freq[i] = std::pow(theta, (-2.0 * i) / kD);
+        last.theta = theta;
+    }
+    *t = last.table;
 }
 
 namespace {
@@ -294,7 +305,8 @@ int decode_launch(const DecodePlan& plan, const gqa_params_t* params, const uint
                   const uint16_t* v, int64_t s0, int64_t s1, int64_t s2, int32_t capacity,
                   const int32_t* block_table, int32_t max_blocks, int32_t n_blocks, const int32_t* seq_len,
                   const int32_t* query_pos, int32_t batch, uint16_t* out, void* workspace,
-                  size_t workspace_bytes, void* stream, unsigned long long* counters = nullptr) {
+                  size_t workspace_bytes, void* stream, unsigned long long* counters = nullptr,
+                  const int32_t* inline_len = nullptr) {
     const size_t need = counters ? plan.workspace_bytes - plan.count_bytes : plan.workspace_bytes;
     if (!workspace || workspace_bytes < need || !aligned(workspace, 256)) return GQA_ERR_WORKSPACE;
 
@@ -330,6 +342,10 @@ int decode_launch(const DecodePlan& plan, const gqa_params_t* params, const uint
     a.qk_scale_log2 = qk_scale_log2(params);
     a.flags = params->flags;
     fill_rope_table(params->rope_theta, &a.rope);
+    if (inline_len) {
+        a.inline_n = batch;
+        std::memcpy(a.inline_len, inline_len, sizeof(int32_t) * 2 * static_cast<size_t>(batch));
+    }
     const hipError_t e = launch_decode(a, batch, static_cast<hipStream_t>(stream), profile_slot());
     return e == hipSuccess ? GQA_OK : GQA_ERR_HIP;
 }
@@ -418,6 +434,52 @@ int gqa_decode_bf16(const gqa_params_t* params, const uint16_t* q, const uint16_
     return decode_launch(plan_decode(params, batch, kv->capacity), params, q, k, v, kv->batch_stride, kv->head_stride,
                          kv->pos_stride, kv->capacity,
                          nullptr, 0, 0, seq_len, query_pos, batch, out, workspace, workspace_bytes, stream);
+}
+
+size_t gqa_decode_host_workspace_bytes(const gqa_params_t* params, int32_t batch, int32_t capacity) {
+    const size_t n = gqa_decode_workspace_bytes(params, batch, capacity);
+    return n ? n + align_up(static_cast<size_t>(batch) * 2 * sizeof(int32_t), 256) : 0;
+}
+
+int gqa_decode_host_bf16(const gqa_params_t* params, const uint16_t* q, const uint16_t* k, const uint16_t* v,
+                         const gqa_kv_layout_t* kv, const int32_t* seq_len, const int32_t* query_pos,
+                         int32_t batch, uint16_t* out, void* workspace, size_t workspace_bytes, void* stream) {
+    int st = decode_args_status(params, q, k, v, kv, seq_len, query_pos, batch, out);
+    if (st != GQA_OK) return st;
+    st = gqa_validate_lengths(seq_len, query_pos, batch, kv->capacity);
+    if (st != GQA_OK) return st;
+    if (!workspace || workspace_bytes < gqa_decode_host_workspace_bytes(params, batch, kv->capacity) ||
+        !aligned(workspace, 256))
+        return GQA_ERR_WORKSPACE;
+    const DecodePlan plan = plan_decode(params, batch, kv->capacity);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    char* ws = static_cast<char*>(workspace);
+    int32_t* len_dev = reinterpret_cast<int32_t*>(ws + plan.workspace_bytes);
+    const int32_t* inl = nullptr;
+    int32_t pairs[2 * kInlineSeqs];
+    bool counted = plan.pieces_cap > 0;      // the one-launch path counts pieces, unless ...
+    if (plan.pieces_cap > 0 && batch <= kInlineSeqs) {
+        // ... every segment is one piece.  The lengths travel with the launch.
+        counted = false;
+        for (int32_t b = 0; b < batch; ++b) {
+            pairs[2 * b] = seq_len[b];
+            pairs[2 * b + 1] = query_pos[b];
+            counted |= query_pos[b] >= kSingleOnePiece;      // keys: min(seq_len, query_pos + 1)
+        }
+        inl = pairs;
+    }
+    hipError_t e = hipSuccess;
+    if (counted)
+        e = launch_zero_words(reinterpret_cast<uint32_t*>(ws + plan.workspace_bytes - plan.count_bytes),
+                              static_cast<int64_t>(plan.count_bytes / 4), s);
+    if (e == hipSuccess && !inl) {
+        e = launch_set_words(len_dev, seq_len, batch, s);
+        if (e == hipSuccess) e = launch_set_words(len_dev + batch, query_pos, batch, s);
+    }
+    if (e != hipSuccess) return GQA_ERR_HIP;
+    return decode_launch(plan, params, q, k, v, kv->batch_stride, kv->head_stride, kv->pos_stride, kv->capacity,
+                         nullptr, 0, 0, len_dev, len_dev + batch, batch, out, workspace, plan.workspace_bytes, stream,
+                         nullptr, inl);
 }
 
 int gqa_decode_bf16_noalloc(const gqa_params_t* params, const uint16_t* q, const uint16_t* k,

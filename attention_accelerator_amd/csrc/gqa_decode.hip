@@ -59,6 +59,8 @@
 //    4q + l/16, dims 8(l%16) .. -- four whole rows per load instruction.  B lane l holds
 //    p of head l%4, key 4q + l/16, gathered through 512 bytes of LDS from the score lanes.
 //    C: lane l accumulates O[head l%4][8(4((l/4)%4) + l/16) + e] over all keys.
+#include <cstring>
+
 #include "gqa_device.h"
 #include "gqa_internal.h"
 #include "gqa_streamk.h"
@@ -67,11 +69,13 @@ namespace gqa {
 
 constexpr int kChunk = 16;           // keys per MFMA group
 
-__device__ __forceinline__ int seq_valid_keys(const DecodeArgs& a, int b) {
-    const int L = a.seq_len[b];
-    const int qp = a.query_pos[b];
-    if (L < 1 || L > a.capacity || qp < 0 || qp >= L) return 0;
+__device__ __forceinline__ int valid_keys(int L, int qp, int capacity) {
+    if (L < 1 || L > capacity || qp < 0 || qp >= L) return 0;
     return min(L, qp + 1);
+}
+
+__device__ __forceinline__ int seq_valid_keys(const DecodeArgs& a, int b) {
+    return valid_keys(a.seq_len[b], a.query_pos[b], a.capacity);
 }
 
 // Keys of sequence b's segments in the stream-K key space: n_valid, rounded up to the
@@ -1128,7 +1132,6 @@ __global__ __launch_bounds__(kGroup * kWave) void decode_merge_kernel(DecodeArgs
 // workspace needs zeroing (gqa_decode_workspace_init) before its first use only.
 
 constexpr int kSingleWaves = 4;
-constexpr int kSingleOnePiece = 128;
 
 // Sums the partials of n_pieces <= kN pieces (slots from slot0) of head h, dims 2*lane and
 // 2*lane + 1.
@@ -1176,7 +1179,9 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
     const uint16_t* qrow = a.q + (static_cast<int64_t>(b) * kHq + kvh * kGroup + wave) * kD;
     const uint16_t qx = qrow[lane], qy = qrow[lane + kPairs];
     const double freq = kRopeQ ? a.rope.inv_freq[lane] : 0.0;
-    const int nv = seq_valid_keys(a, b);
+    const int len = a.inline_n > 0 ? a.inline_len[2 * b] : a.seq_len[b];
+    const int qpos = a.inline_n > 0 ? a.inline_len[2 * b + 1] : a.query_pos[b];
+    const int nv = valid_keys(len, qpos, a.capacity);
     if (nv == 0) {
         if (kvh == 0 && piece == 0) {
             uint4* out = reinterpret_cast<uint4*>(a.out + static_cast<int64_t>(b) * kHq * kD);
@@ -1208,7 +1213,7 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
     // reads its QOps back.
     {
         double sn = 0.0, cs = 1.0;
-        if (kRopeQ) rope_sincos(a.query_pos[b], freq, sn, cs);
+        if (kRopeQ) rope_sincos(qpos, freq, sn, cs);
         const double x = bf16_to_f32(qx);
         const double y = bf16_to_f32(qy);
         double xr = x, yr = y;
@@ -2137,6 +2142,31 @@ hipError_t launch_zero_words(uint32_t* p, int64_t n, hipStream_t stream) {
     hipLaunchKernelGGL(zero_words_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
                        stream, p, n);
     return hipGetLastError();
+}
+
+// Words per launch: kernel arguments hold 4 KB.
+constexpr int kSetWords = 960;
+struct SetWordsArgs {
+    int32_t* dst;
+    int32_t n;
+    int32_t v[kSetWords];
+};
+
+__global__ __launch_bounds__(256) void set_words_kernel(SetWordsArgs a) {
+    for (int i = threadIdx.x; i < a.n; i += 256) a.dst[i] = a.v[i];
+}
+
+hipError_t launch_set_words(int32_t* dst, const int32_t* words, int64_t n, hipStream_t stream) {
+    for (int64_t i = 0; i < n; i += kSetWords) {
+        SetWordsArgs a;
+        a.dst = dst + i;
+        a.n = static_cast<int32_t>(n - i < kSetWords ? n - i : kSetWords);
+        std::memcpy(a.v, words + i, sizeof(int32_t) * static_cast<size_t>(a.n));
+        hipLaunchKernelGGL(set_words_kernel, dim3(1), dim3(256), 0, stream, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stream, hipEvent_t* ev) {

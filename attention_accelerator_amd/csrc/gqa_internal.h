@@ -40,8 +40,13 @@ struct DecodeArgs {
     int32_t count_stride;
     double qk_scale_log2;     // scale * log2(e), folded into Q
     uint32_t flags;           // bit0 RoPE on Q, bit1 RoPE on K
+    int32_t inline_n;         // single-launch path: sequences whose lengths lie here (0: in seq_len)
+    int32_t inline_len[2 * 8];  // their (seq_len, query_pos)
     RopeTable rope;
 };
+constexpr int32_t kInlineSeqs = 8;
+// A one-launch segment of at most this many keys is one piece (no partial, no counter).
+constexpr int kSingleOnePiece = 128;
 
 // Launch plan for a batch: stream-kernel workgroups and partial slots, or (small batches)
 // the single-launch piece size.
@@ -71,6 +76,9 @@ constexpr int32_t kStreamWgsMax = 65536;
 hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stream,
                          hipEvent_t* ev = nullptr);
 hipError_t launch_zero_words(uint32_t* p, int64_t n, hipStream_t stream);
+// Stores n host words at dst, in stream order, as kernel arguments (no copy from host memory,
+// which would wait for the GPU).
+hipError_t launch_set_words(int32_t* dst, const int32_t* words, int64_t n, hipStream_t stream);
 
 struct RopeArgs {
     const uint16_t* in;

@@ -143,6 +143,18 @@ int gqa_decode_bf16(const gqa_params_t* params, const uint16_t* q, const uint16_
                     const int32_t* query_pos, int32_t batch, uint16_t* out, void* workspace,
                     size_t workspace_bytes, void* stream);
 
+/* gqa_decode_bf16 with the lengths in host memory (seq_len and query_pos: host arrays, read
+ * before the call returns): they are checked first (GQA_ERR_INVALID_CONFIG as
+ * gqa_validate_lengths, nothing launched) and reach the GPU with the call's own launches, so
+ * no copy waits for it.  The workspace (gqa_decode_host_workspace_bytes bytes, 256-byte
+ * aligned) may hold anything; otherwise as gqa_decode_bf16.  Under graph capture the lengths are
+ * part of the captured call. */
+size_t gqa_decode_host_workspace_bytes(const gqa_params_t* params, int32_t batch, int32_t capacity);
+int gqa_decode_host_bf16(const gqa_params_t* params, const uint16_t* q, const uint16_t* k,
+                         const uint16_t* v, const gqa_kv_layout_t* kv, const int32_t* seq_len,
+                         const int32_t* query_pos, int32_t batch, uint16_t* out, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
 /* gqa_decode_bf16 without a workspace argument, allocating nothing.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same arguments (less the
