@@ -241,9 +241,9 @@ void rescore_layout(PrefillArgs& a, const gqa_params_t* params, void* base, int3
     a.rs_kblk = reinterpret_cast<uint32_t*>(p + l.kblk);
     a.rs_dblk = reinterpret_cast<uint32_t*>(p + l.dblk);
     a.rs_nblk = nblk;
-    // One-wave workgroups, one per SIMD (the kernel's registers allow one wave per SIMD):
-    // the flagged rows' tiles are cut into about as many (tile, piece) pairs as run at once.
-    const int32_t wgs = stream_wgs(params);
+    // Four-wave workgroups, one per CU (the kernel's registers allow one wave per SIMD): the
+    // flagged rows are cut into about as many (row or tile, piece) pairs as run at once.
+    const int32_t wgs = stream_wgs(params) / kWavesPerCu;
     a.rs_wgs = wgs < 1 ? 1 : wgs > static_cast<int32_t>(kRsSlots) ? static_cast<int32_t>(kRsSlots) : wgs;
 }
 

@@ -1367,15 +1367,24 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
 // own last key start + t (later keys score -inf, p = 0 exactly).  The columns do not mix: a
 // row's arithmetic is the same whichever rows share its tile.
 //
-// A persistent grid of one-wave workgroups takes (tile, piece) pairs; piece p of a tile's
-// np pieces takes its 16-key chunks p, p + np, p + 2 np, ... (so every piece of a tile has
-// about the same work whatever its rows' lengths), two chunks ahead in flight.  np follows
-// from the tile count, the partial slots and the capacity only -- the flagged rows' count
-// per (sequence, KV head) and the call's sizes, never the order rows were flagged in -- so
-// the results are bit-for-bit repeatable.  A piece's partial (fp64 O, running max and sum
-// per column) is published with agent-scope stores and the tile's last piece merges them
-// (the pieces' (m, l) one piece per lane, their O eight pieces at a time), as in
-// decode_single_kernel.
+// A persistent grid of four-wave workgroups, one per CU, takes (tile, piece) pairs; wave w of
+// piece p of a tile's np pieces takes its 16-key chunks 4p + w, 4(p + np) + w, .. (so every
+// wave of a tile has about the same work whatever its rows' lengths), two chunks ahead in
+// flight.  The waves' sums meet in LDS; a piece's partial (fp64 O, running max and sum per
+// column) is published with agent-scope stores and the tile's last piece merges them, a wave per
+// column.  np follows from the tile count, the grid and the capacity only -- the flagged rows'
+// count per (sequence, KV head) and the call's sizes, never the order rows were flagged in or
+// who takes an item -- so the results are bit-for-bit repeatable.
+//
+// The time of a call with few rows is a chain of memory round trips: counts, rows, Q and first
+// chunks (2.4 + 3.5 us), the chunks, the sums, the count, the merge.  One-wave pieces, four
+// times as many, spent 4 to 6 us on the merge alone and 2 us per chunk of new keys, whose (cos,
+// sin) rows were read when needed (now with the chunk's rows): two prompts of 1000 tokens (148
+// rows) step 132.9 -> 119.8 us, 1000 over 4000 (101 rows) 247 -> 220, four prompts of 1000 with
+// 1300 rows 272 -> 268; rows path: 200 over 5003 (4 rows) 100.9 -> 98.6, 4 x 512 over 8192 (55
+// rows) 653 -> 650, T = 4 / 16 of 64 sequences (6 / 30 rows) 246.6 -> 243.2 / 385 -> 382.
+// Two such workgroups per CU do not fit: at 256 registers per wave the
+// chunks in flight spill (slower by 1 to 8 %).
 
 // Rows path (the flagged rows spread thin over their (sequence, KV head) pairs): one row per
 // wave, fp64 VALU (an fp64 MFMA would compute four columns for one and costs more than the
@@ -1383,9 +1392,9 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
 // dims {8c + i, 64 + 8c + i : i < 8}, c = l % 8 -- 8 rotate_half pairs, so a chunk key's
 // rotation is lane-local.  A key's score is the sum over its eight lanes; each lane
 // accumulates p * V over its own keys for its 16 dims, and the 8 key slots are summed once
-// per piece.  A persistent grid of one-wave workgroups takes (row, piece) pairs, piece p of
-// a row taking its chunks p, p + n_pieces, ..., so that the pieces share the costlier chunk
-// keys evenly.  With at most 64 flagged rows (one per lane) every workgroup reads all of them
+// per wave, the four waves' sums per piece.  The workgroups take (row, piece) pairs, wave w of
+// piece p of a row taking its chunks 4p + w, 4(p + n_pieces) + w, ..., so that the waves share
+// the costlier chunk keys evenly.  With at most 64 flagged rows (one per lane) every workgroup reads all of them
 // and gives each row pieces in proportion to its chunks (at least kRsMinChunks per piece, at
 // most kRsMaxPieces pieces): the longest row, which sets the kernel's time, gets the most.
 // With more rows each gets gridDim / rows pieces.  A row's result depends on its keys and
@@ -1393,8 +1402,9 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
 // from the order they were flagged in.
 
 constexpr int kRsKeys = 8;              // keys per rescore chunk (one per 8 lanes)
-constexpr int kRsMinChunks = 4;         // chunks per piece at least (proportional split)
-constexpr int kRsMergeBatch = 32;       // partials loaded at once by a row's merge
+constexpr int kRsWaves = 4;             // waves per rescore workgroup
+constexpr int kRsMinChunks = 16;        // chunks per piece at least (proportional split)
+constexpr int kRsMergeBatch = 8;        // partials a wave of a row's merge loads at once
 
 // This lane's 16 dims of one K row and one V row (BF16): x dims 8c .. 8c+7, y dims 64 + 8c ..
 struct RsRows {
@@ -1550,7 +1560,7 @@ constexpr int kRsGroup = 4;
 constexpr int kRsInflight = 2;
 
 __device__ __forceinline__ void rs_issue_group(const RsItem& it, int ci, int c_end, int step, RsRows (&r)[kRsGroup]) {
-    const int j = threadIdx.x >> 3;
+    const int j = (threadIdx.x & (kWave - 1)) >> 3;
 #pragma unroll
     for (int g = 0; g < kRsGroup; ++g) {
         const int cc = min(ci + g * step, max(c_end - 1, 0));
@@ -1568,7 +1578,7 @@ __device__ __forceinline__ void rs_prefetch(const RsItem& it, int c0, int c_end,
 __device__ __forceinline__ void rs_cached(const RsItem& it, int c0, int c_end, int step, const double (&q)[16],
                                           RsState& st, RsRows (&r)[kRsInflight][kRsGroup]) {
     if (c0 >= c_end) return;
-    const int j = threadIdx.x >> 3;
+    const int j = (threadIdx.x & (kWave - 1)) >> 3;
     const double2 (*no_cs)[8] = nullptr;
     for (int ci = c0;; ci += kRsInflight * kRsGroup * step) {
 #pragma unroll
@@ -1591,7 +1601,7 @@ __device__ __forceinline__ void rs_cached(const RsItem& it, int c0, int c_end, i
 __device__ __forceinline__ void rs_new(const RsItem& it, int c0, int c_end, int step, const double (&q)[16],
                                        RsState& st) {
     if (c0 >= c_end) return;
-    const int j = threadIdx.x >> 3;
+    const int j = (threadIdx.x & (kWave - 1)) >> 3;
     RsRows r[2];
     double2 cs[2][8];
     auto issue = [&](int ci, RsRows& rr, double2 (&cc)[8]) {
@@ -1625,10 +1635,54 @@ __device__ __forceinline__ int rs_first(int p, int step, int lo) {
     return p >= lo ? p : p + (lo - p + step - 1) / step * step;
 }
 
+// Adds the rows of pieces first, first + step, .. < np of one output row (piece p's O at po +
+// p * stride, this lane's two dims), piece p weighted by 2^(my_ex of lane p), kRsMergeBatch
+// pieces at a time: every load of a batch is issued before any is used (unused entries repeat
+// the last piece), so a batch waits for memory once.
+__device__ __forceinline__ void rs_sum_pieces(const double* po, int64_t stride, int first, int step, int np, int my_ex,
+                                              double& o0, double& o1) {
+    for (int u0 = first; u0 < np; u0 += step * kRsMergeBatch) {
+        double2 ov[kRsMergeBatch];
+#pragma unroll
+        for (int u = 0; u < kRsMergeBatch; ++u) ov[u] = load_agent_d2(po + min(u0 + step * u, np - 1) * stride);
+#pragma unroll
+        for (int u = 0; u < kRsMergeBatch; ++u) {
+            const int p = u0 + step * u;
+            if (p < np) {
+                const int ex = __builtin_amdgcn_readlane(my_ex, p);
+                o0 += ldexp(ov[u].x, ex);
+                o1 += ldexp(ov[u].y, ex);
+            }
+        }
+    }
+}
+
+// Lane p's weight exponent against the largest running max of np <= 64 pieces (ml: piece
+// min(lane, np - 1)'s), and the sum of their weighted l.  A piece with no key has m = -inf,
+// weight 0.
+__device__ __forceinline__ int rs_piece_ex(const double2& ml) {
+    const double m_all = wave_max_f64(ml.x);
+    return ml.x == -INFINITY ? -1100 : max_shift_f64(ml.x, m_all);
+}
+__device__ __forceinline__ double rs_piece_l(const double2& ml, int my_ex, int np) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const double l = row16_sum_f64(lane < np ? ldexp(ml.y, my_ex) : 0.0);
+    return swap_add_f64<true>(swap_add_f64<false>(l));
+}
+
+__device__ __forceinline__ uint32_t rs_out2(double o0, double o1, double l) {
+    return f32_to_bf16_out(static_cast<float>(o0 / l)) |
+           (static_cast<uint32_t>(f32_to_bf16_out(static_cast<float>(o1 / l))) << 16);
+}
+
 __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_rows) {
-    __shared__ double o_s[kRsKeys][8][16];      // per key slot, per lane group
+    __shared__ double o_s[kRsWaves][kRsKeys][8][17];      // per wave, key slot and lane group (16, padded)
+    __shared__ double2 ow_s[kRsWaves][kWave];             // each wave's O (dims 2i, 2i + 1)
+    __shared__ double2 ml_s[kRsWaves];                    // and its (m, l)
+    __shared__ int last_s;
     const int T = a.n_new;
-    const int lane = threadIdx.x;
+    const int wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1);
     const int c = lane & 7;
     // The plan.  Proportional (n_rows <= 64): lane r holds row r, its pieces np_l and its
     // first item first_l; items first_l .. first_l + np_l - 1 are its pieces, and its partial
@@ -1637,7 +1691,7 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
     // Uniform otherwise: n_pieces per row, row idx at items idx * n_pieces ...
     const bool prop = n_rows <= static_cast<uint32_t>(kWave);
     uint32_t row_l = 0;
-    int np_l = 0, first_l = 0;
+    int np_l = 0, first_l = 0, st_l = 0;
     int64_t n_work;
     uint32_t n_pieces = 1;
     if (prop) {
@@ -1645,7 +1699,8 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
         if (lane < static_cast<int>(n_rows)) {
             row_l = a.rs_flat[lane];
             const int64_t bt = row_l / kHq;
-            nc = (a.start[bt / T] + static_cast<int>(bt % T) + kRsKeys) / kRsKeys;   // ceil((start + t + 1) / 8)
+            st_l = a.start[bt / T];
+            nc = (st_l + static_cast<int>(bt % T) + kRsKeys) / kRsKeys;   // ceil((start + t + 1) / 8)
         }
         const int64_t total = wave_sum_i64(nc);
         const int64_t budget = max(static_cast<int64_t>(gridDim.x) - static_cast<int64_t>(n_rows), int64_t{1});
@@ -1661,7 +1716,7 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
     }
     for (int64_t wk = blockIdx.x; wk < n_work; wk += gridDim.x) {
         uint32_t idx, row;
-        int piece, np;
+        int piece, np, st = 0;
         int64_t slot0;
         if (prop) {
             const uint64_t m = __ballot(lane < static_cast<int>(n_rows) && first_l <= wk);
@@ -1670,6 +1725,7 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
             row = __shfl(row_l, r);
             slot0 = __shfl(first_l, r);
             np = __shfl(np_l, r);
+            st = __shfl(st_l, r);
             piece = static_cast<int>(wk - slot0);
         } else {
             idx = static_cast<uint32_t>(wk / n_pieces);
@@ -1684,7 +1740,7 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
         const int t = static_cast<int>(bt % T);
         const int kvh = h / kGroup;
         RsItem it;
-        it.st = a.start[b];
+        it.st = prop ? st : a.start[b];
         it.n_keys = it.st + t + 1;
         it.stride_c = a.kv_pos_stride * 2;
         const int64_t head_elem = static_cast<int64_t>(b) * a.kv_batch_stride + static_cast<int64_t>(kvh) * a.kv_head_stride;
@@ -1695,6 +1751,7 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
         const int n_chunks = (it.n_keys + kRsKeys - 1) / kRsKeys;
         // first chunk holding a chunk key (with RoPE on K those are rotated from the new rows)
         const int c_split = (a.flags & 2u) ? it.st / kRsKeys : n_chunks;
+        const int first = kRsWaves * piece + wave, step = kRsWaves * np;     // this wave's chunks
 
         // Q of head h at token t, rotated at start + t (the cos/sin row of token t) and
         // scaled by scale * log2(e): this lane's 8 pairs.  Its loads are issued first, then
@@ -1707,7 +1764,7 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
             const uint4 qy = load_stream16(qrow + 2 * kPairs + 16 * c);
             double2 cs[8];
             rs_load_cs(a.rs_cs + bt * kPairs, cs);
-            rs_prefetch(it, piece, c_split, np, pre);
+            rs_prefetch(it, first, c_split, step, pre);
             rs_widen(qx, q);
             rs_widen(qy, q + 8);
             if (a.flags & 1u) {
@@ -1727,81 +1784,88 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
         for (int i = 0; i < 16; ++i) stt.o[i] = 0.0;
         stt.l = 0.0;
         stt.m = -INFINITY;
-        rs_cached(it, piece, c_split, np, q, stt, pre);
-        rs_new(it, rs_first(piece, np, c_split), n_chunks, np, q, stt);
+        rs_cached(it, first, c_split, step, q, stt, pre);
+        rs_new(it, rs_first(first, step, c_split), n_chunks, step, q, stt);
 
-        // The piece's O over its 8 key slots (through LDS, summed in slot order) and l.
+        // The wave's O over its 8 key slots (through its part of LDS, summed in slot order)
+        // and l; then the waves' sums, in wave order, by wave 0.
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o_s[lane >> 3][c][i] = stt.o[i];
+        for (int i = 0; i < 16; ++i) o_s[wave][lane >> 3][c][i] = stt.o[i];
         double l_tot = stt.l;
 #pragma unroll
         for (int sh = 1; sh < kWave; sh <<= 1) l_tot += __shfl_xor(l_tot, sh);
         l_tot *= 0.125;                              // each key counted in its eight lanes
-        __syncthreads();
-        // lane i merges dims 2i, 2i + 1 (lane group cd, index ii within its 16)
+        __builtin_amdgcn_wave_barrier();             // (one wave's LDS accesses run in order)
+        // lane i sums dims 2i, 2i + 1 (lane group cd, index ii within its 16)
         const int d0 = 2 * lane;
         const int cd = (d0 % kPairs) / 8;
         const int ii = d0 % 8 + (d0 >= kPairs ? 8 : 0);
         double o0 = 0.0, o1 = 0.0;
 #pragma unroll
         for (int jj = 0; jj < kRsKeys; ++jj) {
-            o0 += o_s[jj][cd][ii];
-            o1 += o_s[jj][cd][ii + 1];
+            o0 += o_s[wave][jj][cd][ii];
+            o1 += o_s[wave][jj][cd][ii + 1];
         }
+        ow_s[wave][lane] = make_double2(o0, o1);
+        if (lane == 0) ml_s[wave] = make_double2(stt.m, l_tot);
+        __syncthreads();
         uint32_t* orow = reinterpret_cast<uint32_t*>(a.out + static_cast<int64_t>(row) * kD);
-        if (np == 1) {
-            orow[lane] = f32_to_bf16_out(static_cast<float>(o0 / l_tot)) |
-                         (static_cast<uint32_t>(f32_to_bf16_out(static_cast<float>(o1 / l_tot))) << 16);
-        } else {
-            const int64_t slot = slot0 + piece;
-            unsigned long long* po = reinterpret_cast<unsigned long long*>(a.rs_part_o + slot * kD) + 2 * lane;
-            store_agent(po, o0);
-            store_agent(po + 1, o1);
-            if (lane == 0) {
-                unsigned long long* pml = reinterpret_cast<unsigned long long*>(a.rs_part_ml + slot);
-                store_agent(pml, stt.m);
-                store_agent(pml + 1, l_tot);
+        if (wave == 0) {
+            double m_tot = ml_s[0].x;
+#pragma unroll
+            for (int w = 1; w < kRsWaves; ++w) m_tot = fmax(m_tot, ml_s[w].x);
+            o0 = 0.0;
+            o1 = 0.0;
+            l_tot = 0.0;
+#pragma unroll
+            for (int w = 0; w < kRsWaves; ++w) {
+                const double2 ml = ml_s[w], ow = ow_s[w][lane];
+                const int ex = ml.x == -INFINITY ? -1100 : max_shift_f64(ml.x, m_tot);   // (no key: weight 0)
+                l_tot += ldexp(ml.y, ex);
+                o0 += ldexp(ow.x, ex);
+                o1 += ldexp(ow.y, ex);
             }
-            wait_vmem();                              // the stores have completed ...
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);  // ... and stay before the count
-            int last = 0;
-            if (lane == 0) last = atomicAdd(&a.rs_done[row], 1u) == static_cast<uint32_t>(np) - 1u;
-            last = __shfl(last, 0);
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);  // the merge's loads stay after it
-            if (last) {
-                // Lane u reads piece u's (m, l); lane i merges dims 2i, 2i + 1, the pieces in
-                // order, kRsMergeBatch at a time: every load of a batch is issued before any
-                // is used (unused entries repeat the last piece), so a batch waits for memory
-                // once.  A piece with no key has m = -inf, weight 0.
-                const double2 ml = load_agent_d2(reinterpret_cast<const double*>(a.rs_part_ml + slot0 + min(lane, np - 1)));
-                double m_all = ml.x;
-#pragma unroll
-                for (int sh = 1; sh < kWave; sh <<= 1) m_all = fmax(m_all, __shfl_xor(m_all, sh));
-                const int my_ex = ml.x == -INFINITY ? -1100 : max_shift_f64(ml.x, m_all);
-                double lw = lane < np ? ldexp(ml.y, my_ex) : 0.0;
-#pragma unroll
-                for (int sh = 1; sh < kWave; sh <<= 1) lw += __shfl_xor(lw, sh);
-                o0 = 0.0;
-                o1 = 0.0;
-                for (int u0 = 0; u0 < np; u0 += kRsMergeBatch) {
-                    double2 ov[kRsMergeBatch];
-#pragma unroll
-                    for (int u = 0; u < kRsMergeBatch; ++u)
-                        ov[u] = load_agent_d2(a.rs_part_o + (slot0 + min(u0 + u, np - 1)) * kD + 2 * lane);
-#pragma unroll
-                    for (int u = 0; u < kRsMergeBatch; ++u) {
-                        const int ex = __shfl(my_ex, u0 + u);
-                        if (u0 + u < np) {
-                            o0 += ldexp(ov[u].x, ex);
-                            o1 += ldexp(ov[u].y, ex);
-                        }
-                    }
+            if (np == 1) {
+                orow[lane] = rs_out2(o0, o1, l_tot);
+            } else {
+                const int64_t slot = slot0 + piece;
+                unsigned long long* po = reinterpret_cast<unsigned long long*>(a.rs_part_o + slot * kD) + 2 * lane;
+                store_agent(po, o0);
+                store_agent(po + 1, o1);
+                if (lane == 0) {
+                    unsigned long long* pml = reinterpret_cast<unsigned long long*>(a.rs_part_ml + slot);
+                    store_agent(pml, m_tot);
+                    store_agent(pml + 1, l_tot);
                 }
-                orow[lane] = f32_to_bf16_out(static_cast<float>(o0 / lw)) |
-                             (static_cast<uint32_t>(f32_to_bf16_out(static_cast<float>(o1 / lw))) << 16);
+                wait_vmem();                              // the stores have completed ...
+                __atomic_signal_fence(__ATOMIC_SEQ_CST);  // ... and stay before the count
+                if (lane == 0) last_s = atomicAdd(&a.rs_done[row], 1u) == static_cast<uint32_t>(np) - 1u;
             }
         }
-        __syncthreads();                // o_s is rewritten by the next work item
+        __syncthreads();                // (also: ow_s and ml_s have been read)
+        if (np == 1 || !last_s) continue;
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);      // the merge's loads stay after the count
+        // Lane u of each wave reads piece u's (m, l); wave w sums pieces w, w + 4, .., lane i
+        // dims 2i, 2i + 1.
+        const double2 ml = load_agent_d2(reinterpret_cast<const double*>(a.rs_part_ml + slot0 + min(lane, np - 1)));
+        const int my_ex = rs_piece_ex(ml);
+        o0 = 0.0;
+        o1 = 0.0;
+        rs_sum_pieces(a.rs_part_o + slot0 * kD + 2 * lane, kD, wave, kRsWaves, np, my_ex, o0, o1);
+        ow_s[wave][lane] = make_double2(o0, o1);
+        __syncthreads();
+        if (wave == 0) {
+            const double lw = rs_piece_l(ml, my_ex, np);
+            o0 = 0.0;
+            o1 = 0.0;
+#pragma unroll
+            for (int w = 0; w < kRsWaves; ++w) {
+                o0 += ow_s[w][lane].x;
+                o1 += ow_s[w][lane].y;
+            }
+            orow[lane] = rs_out2(o0, o1, lw);
+        }
+        __syncthreads();                // ow_s is rewritten by the next work item
     }
 }
 
@@ -1809,50 +1873,84 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
 // Tiles path (the flagged rows of a pair numerous enough to fill the four columns):
 constexpr int kRsMinPieceKeys = 128;
 
-// Where (tile, piece) pair wk lies: the tile's (sequence * 8 + KV head), its index j among
-// that pair's tiles and the pair's flagged-row count.  Tiles are numbered pair by pair.
-__device__ __forceinline__ void rs_locate(const PrefillArgs& a, int64_t ti, uint32_t per_bh, int& bh, int& j,
-                                          uint32_t& cnt) {
+// Flagged rows and tiles of 64 (sequence, KV head) pairs, one per lane: pair base + lane has cnt
+// rows in tiles [incl - ceil(cnt / 4), incl) (tiles are numbered pair by pair).
+struct RsPairs {
+    uint32_t cnt;
+    int64_t incl;
+    int start;            // first chunk key of the pair's sequence
+};
+
+__device__ __forceinline__ RsPairs rs_load_pairs(const PrefillArgs& a, int base, int64_t before) {
     const int lane = threadIdx.x & (kWave - 1);
+    const int x = base + lane;
+    RsPairs p;
+    p.cnt = 0u;
+    p.start = 0;
+    if (x < a.batch * kHkv) {
+        p.cnt = min(a.rs_gcnt[x], 4u * static_cast<uint32_t>(a.n_new));
+        p.start = a.start[x / kHkv];
+    }
+    p.incl = wave_incl_scan_i64((p.cnt + 3u) / 4u, lane) + before;
+    return p;
+}
+
+// Where tile ti lies: its (sequence * 8 + KV head), its index j among that pair's tiles, the
+// pair's flagged-row count and first chunk key.  first: the first 64 pairs.
+__device__ __forceinline__ void rs_locate(const PrefillArgs& a, int64_t ti, const RsPairs& first, int& bh, int& j,
+                                          int& cnt, int& st) {
     const int n_bh = a.batch * kHkv;
-    int64_t before = 0;
+    RsPairs p = first;
     bh = 0;
     j = 0;
-    cnt = 0u;
-    for (int base = 0; base < n_bh; base += kWave) {
-        const int x = base + lane;
-        const uint32_t c = x < n_bh ? min(a.rs_gcnt[x], per_bh) : 0u;
-        const int64_t t = (c + 3u) / 4u;
-        const int64_t incl = wave_incl_scan_i64(t, lane) + before;
-        const uint64_t m = __ballot(t > 0 && incl - t <= ti && ti < incl);
+    cnt = 0;
+    st = 0;
+    for (int base = 0;;) {
+        const int64_t t = (p.cnt + 3u) / 4u;
+        const uint64_t m = __ballot(t > 0 && p.incl - t <= ti && ti < p.incl);
         if (m) {
             const int l = __ffsll(static_cast<unsigned long long>(m)) - 1;
             bh = base + l;
-            j = static_cast<int>(ti - __shfl(incl - t, l));
-            cnt = __shfl(c, l);
+            j = static_cast<int>(ti - __shfl(p.incl - t, l));
+            cnt = __builtin_amdgcn_readlane(static_cast<int>(p.cnt), l);
+            st = __builtin_amdgcn_readlane(p.start, l);
             return;
         }
-        before = __shfl(incl, kWave - 1);
+        base += kWave;
+        if (base >= n_bh) return;
+        p = rs_load_pairs(a, base, __shfl(p.incl, kWave - 1));
     }
 }
 
 // This lane's Q operands for its column: Q row `row` (b, t, h), rotated at start + t with the
 // (cos, sin) table and scaled by scale*log2(e) in double -- q[kb][e] = Q[32kb + 8(l/16) + e].
-__device__ __forceinline__ void rs_q_operands(const PrefillArgs& a, uint32_t row, QOps& qa) {
+// Two steps, so that the first chunks are requested between them.
+__device__ __forceinline__ void rs_q_load(const PrefillArgs& a, uint32_t row, uint4 (&qw)[4], double2 (&cs)[2][8]) {
     const int g = (threadIdx.x & (kWave - 1)) >> 4;
-    const int64_t bt = row / kHq;
-    const uint16_t* qrow = a.q + static_cast<int64_t>(row) * kD;
-    const double2* cs = a.rs_cs + bt * kPairs;
+    const uint16_t* qrow = a.q + static_cast<int64_t>(row) * kD + 8 * g;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) qw[kb] = *reinterpret_cast<const uint4*>(qrow + 32 * kb);
+    if (a.flags & 1u) {
+        const double2* p = a.rs_cs + static_cast<int64_t>(row / kHq) * kPairs + 8 * g;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) cs[kb][e] = p[32 * kb + e];
+    }
+}
+
+__device__ __forceinline__ void rs_q_operands(const PrefillArgs& a, const uint4 (&qw)[4], const double2 (&cs)[2][8],
+                                              QOps& qa) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
         float xf[8], yf[8];
-        unpack8(*reinterpret_cast<const uint4*>(qrow + 32 * kb + 8 * g), xf);
-        unpack8(*reinterpret_cast<const uint4*>(qrow + kPairs + 32 * kb + 8 * g), yf);
+        unpack8(qw[kb], xf);
+        unpack8(qw[kb + 2], yf);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             double x = xf[e], y = yf[e];
             if (a.flags & 1u) {
-                const double2 c = cs[32 * kb + 8 * g + e];
+                const double2 c = cs[kb][e];
                 const double xr = x * c.x - y * c.y;
                 y = x * c.y + y * c.x;
                 x = xr;
@@ -1865,11 +1963,13 @@ __device__ __forceinline__ void rs_q_operands(const PrefillArgs& a, uint32_t row
 
 // One 16-key chunk [kc, kc + 16) of a tile: scores of the 4 columns, each column's keys up
 // to col_lim (and below k_hi) counting, online softmax and weighted V, all in fp64 (the
-// arithmetic of compute_chunk).  With RoPE on K, a key >= st is its new row (loaded by the
-// caller) rotated in double with the (cos, sin) row of its token.
-__device__ __forceinline__ void rs_tile_chunk(const PrefillArgs& a, int b, int st, int kc, int k_hi, int col_lim,
-                                              const Chunk& c, const QOps& qa, PieceState& ps) {
-    __shared__ double p_lds[kWave];
+// arithmetic of compute_chunk).  With RoPE on K, a key >= st is its new row rotated in double
+// with cs, the (cos, sin) values of its token (both loaded by the caller).
+__device__ __forceinline__ void rs_tile_chunk(const PrefillArgs& a, int st, int kc, int k_hi, int col_lim,
+                                              const Chunk& c, const double2 (&cs)[2][8], const QOps& qa,
+                                              PieceState& ps) {
+    __shared__ double p_lds4[kRsWaves][kWave];
+    double* p_lds = p_lds4[threadIdx.x / kWave];
     const int lane = threadIdx.x & (kWave - 1);
     double kd[4][8];
 #pragma unroll
@@ -1879,21 +1979,15 @@ __device__ __forceinline__ void rs_tile_chunk(const PrefillArgs& a, int b, int s
 #pragma unroll
         for (int e = 0; e < 8; ++e) kd[kb][e] = static_cast<double>(kf[e]);
     }
-    if ((a.flags & 2u) && kc + 15 >= st) {
-        const int key = min(kc + (lane & 15), k_hi - 1);
-        if (key >= st) {
-            const int g = lane >> 4;
-            const double2* cs = a.rs_cs + (static_cast<int64_t>(b) * a.n_new + (key - st)) * kPairs;
+    if ((a.flags & 2u) && kc + 15 >= st && min(kc + (lane & 15), k_hi - 1) >= st) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const double2 r = cs[32 * kb + 8 * g + e];
-                    const double x = kd[kb][e], y = kd[kb + 2][e];
-                    kd[kb][e] = x * r.x - y * r.y;
-                    kd[kb + 2][e] = x * r.y + y * r.x;
-                }
-        }
+            for (int e = 0; e < 8; ++e) {
+                const double x = kd[kb][e], y = kd[kb + 2][e];
+                kd[kb][e] = x * cs[kb][e].x - y * cs[kb][e].y;
+                kd[kb + 2][e] = x * cs[kb][e].y + y * cs[kb][e].x;
+            }
     }
     double s4[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -1937,165 +2031,179 @@ __device__ __forceinline__ void rs_tile_chunk(const PrefillArgs& a, int b, int s
         for (int e = 0; e < 8; ++e) ps.acc[e] = mfma_f64(vd[q][e], pq[q], ps.acc[e]);
 }
 
-// One BF16 output row segment: this lane's 8 dims of its column's row, O / l rounded
-// double -> f32 -> BF16.
-__device__ __forceinline__ void rs_write8(const PrefillArgs& a, uint32_t row, int d0, const double (&o)[8], double l) {
-    uint16_t o8[8];
+// Pieces per tile for n_tiles tiles on this grid: as many as fill one to four rounds of
+// workgroups, whichever takes least by the keys of a piece (of the capacity) plus what a piece
+// costs beside its keys, about 128 keys' time (Q operands, the sums over waves and pieces).
+__device__ __forceinline__ int rs_tile_pieces(int64_t n_tiles, int capacity) {
+    const int64_t grid = gridDim.x;
+    const int np_max =
+        max(1, min(min(kRsMaxPieces, capacity / kRsMinPieceKeys), static_cast<int>(kRsSlots / max(n_tiles, int64_t{1}))));
+    int np = 1;
+    float best = INFINITY;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o8[e] = f32_to_bf16_out(static_cast<float>(o[e] / l));
-    *reinterpret_cast<bf16x8_t*>(a.out + static_cast<int64_t>(row) * kD + d0) = pack8(o8);
+    for (int r = 1; r <= 4; ++r) {
+        const int n = min(np_max, static_cast<int>(r * grid / max(n_tiles, int64_t{1})));
+        const float cost = r * (static_cast<float>(capacity) / n + 128.f);
+        if (n >= 1 && cost < best) {
+            best = cost;
+            np = n;
+        }
+    }
+    return np;
 }
 
-__device__ __forceinline__ void rs_tiles_path(const PrefillArgs& a, int64_t n_tiles) {
+__device__ __forceinline__ void rs_tiles_path(const PrefillArgs& a, int64_t n_tiles, const RsPairs& pairs) {
+    __shared__ double oc_s[kRsWaves][kGroup][kD];     // each wave's O of the four columns
+    __shared__ double2 mlc_s[kRsWaves][kGroup];       // and their (m, l)
+    __shared__ int lastc_s;
+    __shared__ int64_t next_s[2];
     const int T = a.n_new;
-    const int lane = threadIdx.x;
+    const int wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1);
     const uint32_t per_bh = 4u * static_cast<uint32_t>(T);
-    int np = n_tiles >= kRsSlots ? 1 : static_cast<int>(kRsSlots / n_tiles);
-    np = min(np, kRsMaxPieces);
-    np = max(1, min(np, a.capacity / kRsMinPieceKeys));
+    const int np = rs_tile_pieces(n_tiles, a.capacity);
     const int64_t n_work = n_tiles * np;
     const int col = lane & 3;
     const int64_t rb = a.kv_pos_stride * 2;      // cache row bytes
-    for (int64_t wk = blockIdx.x; wk < n_work; wk += gridDim.x) {
+    // The grid's first items are its workgroups', the rest are claimed as workgroups come free
+    // (tiles differ in keys; what an item computes does not depend on who takes it).  The
+    // claim is requested with the item's loads and passed on at its first barrier.
+    int64_t wk_next = 0;
+    for (int64_t wk = blockIdx.x, turn = 0; wk < n_work; wk = wk_next, turn ^= 1) {
+        wk_next = n_work;
+        if (n_work > gridDim.x && threadIdx.x == 0) wk_next = gridDim.x + static_cast<int64_t>(atomicAdd(a.rs_hdr + kRsClaim, 1u));
         const int64_t ti = wk / np;
         const int piece = static_cast<int>(wk % np);
-        int bh, j;
-        uint32_t cnt;
-        rs_locate(a, ti, per_bh, bh, j, cnt);
+        int bh, j, cnt, st;
+        rs_locate(a, ti, pairs, bh, j, cnt, st);
         const int b = bh / kHkv;
         const int kvh = bh % kHkv;
-        const int st = a.start[b];
-        const int nr = min(4, static_cast<int>(cnt) - 4 * j);
+        const int nr = min(4, cnt - 4 * j);
         const uint32_t* rows = a.rs_rows + static_cast<int64_t>(bh) * per_bh + 4 * j;
         // This lane's column: row `row` (a repeat of the tile's first row past nr, which
         // counts no key and is not written).
         const uint32_t row = rows[col < nr ? col : 0];
+        const uint32_t wrow = __builtin_amdgcn_readlane(row, wave);     // column `wave`'s row
         const int col_lim = col < nr ? st + static_cast<int>((row / kHq) % T) : -1;
         int lim_max = col_lim;
         lim_max = max(lim_max, __shfl_xor(lim_max, 1));
         lim_max = max(lim_max, __shfl_xor(lim_max, 2));
         const int k_hi = lim_max + 1;                     // keys [0, k_hi) of the tile
-        const int k_lo = piece * kChunk;                  // first chunk of this piece
-        const int k_step = np * kChunk;
+        const int k_lo = (kRsWaves * piece + wave) * kChunk;     // first chunk of this wave
+        const int k_step = kRsWaves * np * kChunk;
 
+        const char* kseg = reinterpret_cast<const char*>(a.k + static_cast<int64_t>(b) * a.kv_batch_stride +
+                                                         static_cast<int64_t>(kvh) * a.kv_head_stride);
+        const char* vseg = reinterpret_cast<const char*>(a.v + static_cast<int64_t>(b) * a.kv_batch_stride +
+                                                         static_cast<int64_t>(kvh) * a.kv_head_stride);
+        const bool rope_k = (a.flags & 2u) != 0;
+        // Rows of chunk [kc, kc + 16): clamped to the piece's last key (masked there).  Plain
+        // (cached) loads: the tiles of one pair run at the same time and read the same rows
+        // (config 5 with Q x 16: 171 -> 161 us).
+        auto load = [&](int kc, Chunk& c) {
+            const int kk = min(kc + (lane & 15), k_hi - 1);
+            const char* kp = rope_k && kk >= st
+                                 ? reinterpret_cast<const char*>(
+                                       a.k_new + ((static_cast<int64_t>(b) * T + (kk - st)) * kHkv + kvh) * kD)
+                                 : kseg + kk * rb;
+            kp += 16 * (lane >> 4);
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb) c.kw[kb] = *reinterpret_cast<const uint4*>(kp + 64 * kb);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int kv = min(kc + 4 * q + (lane >> 4), k_hi - 1);
+                c.vw[q] = *reinterpret_cast<const uint4*>(vseg + kv * rb + 16 * (lane & 15));
+            }
+        };
+        // (cos, sin) of the chunk's new keys, a chunk ahead.
+        auto load_cs = [&](int kc, double2 (&cs)[2][8]) {
+            if (!rope_k || kc + 15 < st) return;      // (uniform)
+            const int u = max(min(kc + (lane & 15), k_hi - 1) - st, 0);
+            const double2* p = a.rs_cs + (static_cast<int64_t>(b) * T + u) * kPairs + 8 * (lane >> 4);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) cs[kb][e] = p[32 * kb + e];
+        };
+        // The Q row and the first chunks are requested before the Q operands are formed.
+        Chunk c0, c1, c2;
+        double2 cs0[2][8] = {}, cs1[2][8] = {}, csq[2][8] = {};
+        uint4 qw[4];
+        rs_q_load(a, row, qw, csq);
+        load(min(k_lo, k_hi - 1), c0);
+        load_cs(k_lo, cs0);
+        load(min(k_lo + k_step, k_hi - 1), c1);
         QOps qa;
-        rs_q_operands(a, row, qa);
+        rs_q_operands(a, qw, csq, qa);
         PieceState ps;
         init_piece(ps);
-        if (k_lo < k_hi) {
-            const char* kseg = reinterpret_cast<const char*>(a.k + static_cast<int64_t>(b) * a.kv_batch_stride +
-                                                             static_cast<int64_t>(kvh) * a.kv_head_stride);
-            const char* vseg = reinterpret_cast<const char*>(a.v + static_cast<int64_t>(b) * a.kv_batch_stride +
-                                                             static_cast<int64_t>(kvh) * a.kv_head_stride);
-            const bool rope_k = (a.flags & 2u) != 0;
-            // Rows of chunk [kc, kc + 16): clamped to the piece's last key (masked there).  Plain
-            // (cached) loads: the tiles of one pair run at the same time and read the same rows
-            // (config 5 with Q x 16: 171 -> 161 us).
-            auto load = [&](int kc, Chunk& c) {
-                const int kk = min(kc + (lane & 15), k_hi - 1);
-                const char* kp = rope_k && kk >= st
-                                     ? reinterpret_cast<const char*>(
-                                           a.k_new + ((static_cast<int64_t>(b) * T + (kk - st)) * kHkv + kvh) * kD)
-                                     : kseg + kk * rb;
-                kp += 16 * (lane >> 4);
+        for (int kc = k_lo; kc < k_hi; kc += k_step) {
+            if (kc + k_step < k_hi) load_cs(kc + k_step, cs1);
+            load(min(kc + 2 * k_step, k_hi - 1), c2);
+            rs_tile_chunk(a, st, kc, k_hi, col_lim, c0, cs0, qa, ps);
+            c0 = c1;
+            c1 = c2;
 #pragma unroll
-                for (int kb = 0; kb < 4; ++kb) c.kw[kb] = *reinterpret_cast<const uint4*>(kp + 64 * kb);
+            for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int kv = min(kc + 4 * q + (lane >> 4), k_hi - 1);
-                    c.vw[q] = *reinterpret_cast<const uint4*>(vseg + kv * rb + 16 * (lane & 15));
-                }
-            };
-            Chunk c0, c1, c2;
-            load(k_lo, c0);
-            load(min(k_lo + k_step, k_hi - 1), c1);
-            for (int kc = k_lo; kc < k_hi; kc += k_step) {
-                load(min(kc + 2 * k_step, k_hi - 1), c2);
-                rs_tile_chunk(a, b, st, kc, k_hi, col_lim, c0, qa, ps);
-                c0 = c1;
-                c1 = c2;
-            }
+                for (int e = 0; e < 8; ++e) cs0[kb][e] = cs1[kb][e];
         }
         double l_tot;
         finish_piece(ps, l_tot);
+        // The waves' sums meet in LDS; wave w then holds column w, lane i dims 2i, 2i + 1.
+#pragma unroll
+        for (int e = 0; e < 8; ++e) oc_s[wave][col][out_dim_of_lane(lane) + e] = ps.acc[e];
+        if (lane < kGroup) mlc_s[wave][lane] = make_double2(ps.m_run, l_tot);
+        if (threadIdx.x == 0) next_s[turn] = wk_next;      // (two slots: a slow wave may still read the last)
+        __syncthreads();
+        wk_next = next_s[turn];
+        double o0 = 0.0, o1 = 0.0, l = 0.0;
+        double m = mlc_s[0][wave].x;
+#pragma unroll
+        for (int w = 1; w < kRsWaves; ++w) m = fmax(m, mlc_s[w][wave].x);
+#pragma unroll
+        for (int w = 0; w < kRsWaves; ++w) {
+            const double2 ml = mlc_s[w][wave];
+            const int ex = ml.x == -INFINITY ? -1100 : max_shift_f64(ml.x, m);       // (no key: weight 0)
+            l += ldexp(ml.y, ex);
+            o0 += ldexp(oc_s[w][wave][2 * lane], ex);
+            o1 += ldexp(oc_s[w][wave][2 * lane + 1], ex);
+        }
+        uint32_t* orow = reinterpret_cast<uint32_t*>(a.out + static_cast<int64_t>(wrow) * kD);
         if (np == 1) {
-            if (col < nr) rs_write8(a, row, out_dim_of_lane(lane), ps.acc, l_tot);
+            if (wave < nr) orow[lane] = rs_out2(o0, o1, l);
+            __syncthreads();              // oc_s is rewritten by the next work item
             continue;
         }
         // Partial at slot wk: O[column][dim] and (m, l) per column.
         {
-            unsigned long long* po = reinterpret_cast<unsigned long long*>(a.rs_part_o + wk * kGroup * kD) +
-                                     col * kD + out_dim_of_lane(lane);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) store_agent(po + e, ps.acc[e]);
-            if (lane < kGroup) {
-                unsigned long long* pml = reinterpret_cast<unsigned long long*>(a.rs_part_ml + wk * kGroup + lane);
-                store_agent(pml, ps.m_run);
-                store_agent(pml + 1, l_tot);
+            unsigned long long* po =
+                reinterpret_cast<unsigned long long*>(a.rs_part_o + (wk * kGroup + wave) * kD) + 2 * lane;
+            store_agent(po, o0);
+            store_agent(po + 1, o1);
+            if (lane == 0) {
+                unsigned long long* pml = reinterpret_cast<unsigned long long*>(a.rs_part_ml + wk * kGroup + wave);
+                store_agent(pml, m);
+                store_agent(pml + 1, l);
             }
         }
         wait_vmem();                              // the stores have completed ...
         __atomic_signal_fence(__ATOMIC_SEQ_CST);  // ... and stay before the count
-        int last = 0;
-        if (lane == 0) last = atomicAdd(&a.rs_done[ti], 1u) == static_cast<uint32_t>(np) - 1u;
-        last = __shfl(last, 0);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);  // the merge's loads stay after it
-        if (!last) continue;
-        // Merge: lane u reads piece u's (m, l) of all four columns; lane l then takes column
-        // c = l / 16, dims 8 (l % 16) .. +7, the pieces in order, eight at a time (their loads
-        // issued before any is used).  A piece with no key has m = -inf, weight 0.
-        const int mc = lane >> 4;
-        const int d0 = 8 * (lane & 15);
+        __syncthreads();
+        if (threadIdx.x == 0) lastc_s = atomicAdd(&a.rs_done[ti], 1u) == static_cast<uint32_t>(np) - 1u;
+        __syncthreads();                          // (lastc_s is next written after two more barriers)
+        if (!lastc_s) continue;
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);  // the merge's loads stay after the count
+        // Merge: wave w takes column w, the pieces in order (lane u: piece u's (m, l)).
         const int64_t slot0 = ti * np;
-        int ex[kGroup];
-        double lw = 0.0;
-        {
-            double2 ml[kGroup];
-#pragma unroll
-            for (int c = 0; c < kGroup; ++c)
-                ml[c] = load_agent_d2(
-                    reinterpret_cast<const double*>(a.rs_part_ml + (slot0 + min(lane, np - 1)) * kGroup + c));
-#pragma unroll
-            for (int c = 0; c < kGroup; ++c) {
-                double m_all = lane < np ? ml[c].x : -INFINITY;
-#pragma unroll
-                for (int sh = 1; sh < kWave; sh <<= 1) m_all = fmax(m_all, __shfl_xor(m_all, sh));
-                ex[c] = ml[c].x == -INFINITY ? -1100 : max_shift_f64(ml[c].x, m_all);
-                double lc = lane < np ? ldexp(ml[c].y, ex[c]) : 0.0;
-#pragma unroll
-                for (int sh = 1; sh < kWave; sh <<= 1) lc += __shfl_xor(lc, sh);
-                if (c == mc) lw = lc;
-            }
-        }
-        double o[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        constexpr int kMb = 8;
-        for (int u0 = 0; u0 < np; u0 += kMb) {
-            double2 v[kMb][4];
-#pragma unroll
-            for (int u = 0; u < kMb; ++u) {
-                const double* src = a.rs_part_o + ((slot0 + min(u0 + u, np - 1)) * kGroup + mc) * kD + d0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[u][e] = load_agent_d2(src + 2 * e);
-            }
-#pragma unroll
-            for (int u = 0; u < kMb; ++u) {
-                int e_u = __shfl(ex[0], u0 + u);
-#pragma unroll
-                for (int c = 1; c < kGroup; ++c) {
-                    const int x = __shfl(ex[c], u0 + u);
-                    e_u = c == mc ? x : e_u;
-                }
-                if (u0 + u < np) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        o[2 * e] += ldexp(v[u][e].x, e_u);
-                        o[2 * e + 1] += ldexp(v[u][e].y, e_u);
-                    }
-                }
-            }
-        }
-        const uint32_t mrow = rows[mc < nr ? mc : 0];
-        if (mc < nr) rs_write8(a, mrow, d0, o, lw);
+        const double2 ml = load_agent_d2(
+            reinterpret_cast<const double*>(a.rs_part_ml + (slot0 + min(lane, np - 1)) * kGroup + wave));
+        const int my_ex = rs_piece_ex(ml);
+        o0 = 0.0;
+        o1 = 0.0;
+        rs_sum_pieces(a.rs_part_o + (slot0 * kGroup + wave) * kD + 2 * lane, kGroup * kD, 0, 1, np, my_ex, o0, o1);
+        const double lw = rs_piece_l(ml, my_ex, np);
+        if (wave < nr) orow[lane] = rs_out2(o0, o1, lw);
     }
 }
 
@@ -2105,7 +2213,7 @@ __device__ __forceinline__ void rs_tiles_path(const PrefillArgs& a, int64_t n_ti
 // one row about twice as much.
 constexpr int kRsTileFill = 3;
 
-__global__ __launch_bounds__(kWave) void rescore_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(kRsWaves * kWave) void rescore_kernel(PrefillArgs a) {
     const uint32_t cap = static_cast<uint32_t>(a.batch) * static_cast<uint32_t>(a.n_new) * kHq;
     const uint32_t n_rows = min(a.rs_hdr[0], cap);
     if (n_rows == 0) return;
@@ -2114,21 +2222,16 @@ __global__ __launch_bounds__(kWave) void rescore_kernel(PrefillArgs a) {
         rs_rows_path(a, n_rows);
         return;
     }
-    const int lane = threadIdx.x;
-    const int n_bh = a.batch * kHkv;
-    const uint32_t per_bh = 4u * static_cast<uint32_t>(a.n_new);
-    int64_t n_tiles = 0;
-    for (int base = 0; base < n_bh; base += kWave) {
-        const int x = base + lane;
-        const uint32_t c = x < n_bh ? min(a.rs_gcnt[x], per_bh) : 0u;
-        n_tiles += wave_sum_i64((c + 3u) / 4u);
-    }
-    rs_tiles_path(a, n_tiles);
+    const RsPairs pairs = rs_load_pairs(a, 0, 0);
+    int64_t n_tiles = __shfl(pairs.incl, kWave - 1);
+    for (int base = kWave; base < a.batch * kHkv; base += kWave)
+        n_tiles = __shfl(rs_load_pairs(a, base, n_tiles).incl, kWave - 1);
+    rs_tiles_path(a, n_tiles, pairs);
 }
 
 hipError_t launch_rescore(const PrefillArgs& a, hipStream_t stream) {
     if (!a.rs_hdr) return hipSuccess;
-    hipLaunchKernelGGL(rescore_kernel, dim3(static_cast<unsigned>(a.rs_wgs)), dim3(kWave), 0, stream, a);
+    hipLaunchKernelGGL(rescore_kernel, dim3(static_cast<unsigned>(a.rs_wgs)), dim3(kRsWaves * kWave), 0, stream, a);
     return hipGetLastError();
 }
 

@@ -233,6 +233,7 @@ __host__ __device__ inline bool rs_flag_decide(double mn2, double ss, double m, 
 // HIP events per call of the opt-in kernel timing: up to four stages between them.
 constexpr int kProfileEvents = 5;
 constexpr int kRsSlots = 1024;                            // partial slots (tiles x pieces)
+constexpr int kRsClaim = 32;                              // rs_hdr word: items of the tiles path claimed
 constexpr int kRsMaxPieces = 64;                          // pieces per tile at most
 // Rescore region of a workspace; ncb, nr: the chunk-prefix blocks and rows (prefill:
 // ceil(T / 64) + 1 and 64; multi-token: 1 and T); nblk: 64-position blocks of the cache
@@ -265,7 +266,7 @@ __device__ __forceinline__ void rs_append(const PrefillArgs& a, uint32_t row) {
 // flagged row sees a V that is not finite (the rescore then takes its rows path: the tiles
 // path shares V between rows of different causal limits, and 0 * inf would give NaN).
 __device__ __forceinline__ void rs_clear(const PrefillArgs& a, int t) {
-    if (a.rs_hdr && t < 3) a.rs_hdr[t] = 0u;
+    if (a.rs_hdr && (t < 3 || t == kRsClaim)) a.rs_hdr[t] = 0u;
 }
 
 // The same kernel clears row (b*T + t)*32 + h's piece counter and, with RoPE on K, stores
