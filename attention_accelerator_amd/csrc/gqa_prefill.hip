@@ -518,9 +518,12 @@ __global__ __launch_bounds__(kStgThreads) void prefill_stage_kernel(PrefillArgs 
 // (thread t: dword column t % 64 of every 16th block; norm group t % 8 of every 64th),
 // meeting in LDS; then, chunk block by chunk block, the previous chunk blocks' maxima (row
 // 63 of their running maxima).
+// Bound by its round trips: a chunk block's row read only after the one before was stored was 17
+// of them for 1000 tokens; eight at a time, two prompts of 1000 tokens step 120.1 -> 117.2 us.
 __global__ __launch_bounds__(1024) void prefill_stat_reduce_kernel(PrefillArgs a) {
     __shared__ uint32_t vpart[16][kD / 2];
     __shared__ uint32_t kpart[64][8];
+    constexpr int kAhead = 8;             // chunk blocks whose last rows are requested together
     const int bh = blockIdx.x;
     const int tid = threadIdx.x;
     const int st = a.start[bh / kHkv];
@@ -559,11 +562,19 @@ __global__ __launch_bounds__(1024) void prefill_stat_reduce_kernel(PrefillArgs a
         for (int i = 0; i < 16; ++i) v = pk_max_u16(v, vpart[i][tid]);
         // Chunk block cb: the cached maxima and chunk blocks 0 .. cb-1 (their last row).
         const int64_t pre0 = static_cast<int64_t>(bh) * a.rs_ncb * a.rs_nr;
-        for (int cb = 0; cb < a.rs_ncb; ++cb) {
-            uint32_t* dc = a.rs_dc + (static_cast<int64_t>(bh) * a.rs_ncb + cb) * kD + 2 * tid;
-            dc[0] = v & 0xffffu;
-            dc[1] = v >> 16;
-            v = pk_max_u16(v, *reinterpret_cast<const uint32_t*>(a.rs_dpre + (pre0 + static_cast<int64_t>(cb) * a.rs_nr + a.rs_nr - 1) * kD + 2 * tid));
+        for (int cb = 0; cb < a.rs_ncb; cb += kAhead) {
+            uint32_t w[kAhead];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j)
+                w[j] = *reinterpret_cast<const uint32_t*>(
+                    a.rs_dpre + (pre0 + static_cast<int64_t>(min(cb + j, a.rs_ncb - 1)) * a.rs_nr + a.rs_nr - 1) * kD + 2 * tid);
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                if (cb + j < a.rs_ncb)
+                    *reinterpret_cast<uint2*>(a.rs_dc + (static_cast<int64_t>(bh) * a.rs_ncb + cb + j) * kD + 2 * tid) =
+                        make_uint2(v & 0xffffu, v >> 16);
+                v = pk_max_u16(v, w[j]);
+            }
         }
     } else if (tid < kD / 2 + 8) {
         const int g = tid - kD / 2;
@@ -571,9 +582,16 @@ __global__ __launch_bounds__(1024) void prefill_stat_reduce_kernel(PrefillArgs a
 #pragma unroll 8
         for (int i = 0; i < 64; ++i) y = max(y, kpart[i][g]);
         const int64_t pre0 = static_cast<int64_t>(bh) * a.rs_ncb * a.rs_nr;
-        for (int cb = 0; cb < a.rs_ncb; ++cb) {
-            a.rs_kc[(static_cast<int64_t>(bh) * a.rs_ncb + cb) * 8 + g] = y;
-            y = max(y, a.rs_kpre[(pre0 + static_cast<int64_t>(cb) * a.rs_nr + a.rs_nr - 1) * 8 + g]);
+        for (int cb = 0; cb < a.rs_ncb; cb += kAhead) {
+            uint32_t w[kAhead];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j)
+                w[j] = a.rs_kpre[(pre0 + static_cast<int64_t>(min(cb + j, a.rs_ncb - 1)) * a.rs_nr + a.rs_nr - 1) * 8 + g];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                if (cb + j < a.rs_ncb) a.rs_kc[(static_cast<int64_t>(bh) * a.rs_ncb + cb + j) * 8 + g] = y;
+                y = max(y, w[j]);
+            }
         }
     }
 }
