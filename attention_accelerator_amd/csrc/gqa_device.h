@@ -232,16 +232,23 @@ __device__ __forceinline__ float wave_max(float x) { return cross_row_max(row16_
 
 
 // sin and cos of an angle in double: reduced to |r| <= pi/4 with a two-part Cody-Waite pi/2
-// and fused multiply-adds, then the Taylor series of both (truncation below 5e-19) and the
-// quadrant.  Against 113-bit values for every frequency of theta = 500000 at positions up to
-// 400,000 (and angles of 2e9): largest error 1.2e-16, rms 3.1e-17; the library's sincos of the
-// angle reduced modulo 2 pi had 2.5e-16 and 6.2e-17, in about three times the instructions (the
-// kernels here wait for one sincos after the other at their start).  An angle past ~2^53 has
-// no meaningful reduction: r is clamped, so that the results stay bounded.
+// and fused multiply-adds, then the Taylor series of both (first omitted terms at pi/4: 9e-20
+// for the sine, 2.1e-18 for the cosine) and the quadrant.  The reduction runs twice: from
+// angles of about 2^46 on the rounding of angle * 2/pi can put k one off, and the second step
+// takes that back (on smaller angles its j is 0, or +-1 where r sits at pi/4).  Against 113-bit
+// values for every frequency of theta = 500000 at positions up to 400,000: largest error
+// 1.2e-16, rms 3.1e-17; over all angles below 2^53 1.9e-16 (the library's sincos of the angle
+// reduced modulo 2 pi: 2.5e-16 and 6.2e-17, in about three times the instructions; the kernels
+// here wait for one sincos after the other at their start).  From 2^54 on the two parts of pi/2
+// are too few bits and the error grows with the angle (1.9e-15 below 2^58); the clamp keeps
+// what is left past about 2^105 bounded.
 __device__ __forceinline__ void sincos_f64(double angle, double& s, double& c) {
     const double k = rint(angle * 0.63661977236758134308);    // 2 / pi
     double r = fma(-k, 1.5707963267948965580, angle);          // pi / 2 rounded to double
     r = fma(-k, 6.1232339957367658e-17, r);                    // pi / 2 - that
+    const double j = rint(r * 0.63661977236758134308);
+    r = fma(-j, 1.5707963267948965580, r);
+    r = fma(-j, 6.1232339957367658e-17, r);
     r = r > 0.8 ? 0.8 : r;
     r = r < -0.8 ? -0.8 : r;
     const double z = r * r;
@@ -264,8 +271,8 @@ __device__ __forceinline__ void sincos_f64(double angle, double& s, double& c) {
     const double hz = 0.5 * z;
     const double w = 1.0 - hz;
     const double cr = w + fma(z * z, pc, (1.0 - w) - hz);
-    // quadrant k mod 4 (k may exceed the int range)
-    const double q = k * 0.25;
+    // quadrant (k + j) mod 4 (both may exceed the int range, and their sum's last bit a double)
+    const double q = (k * 0.25 - floor(k * 0.25)) + j * 0.25;
     const int n = static_cast<int>(4.0 * (q - floor(q)));
     const double a = (n & 1) ? cr : sr, b = (n & 1) ? sr : cr;
     s = (n & 2) ? -a : a;

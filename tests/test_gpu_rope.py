@@ -58,3 +58,17 @@ def test_rope_pos0_offset(dev):
     b = to_codes(gqa.rope_half_split(to_dev(inp, dev),
                                      torch.arange(1000, 1010, dtype=torch.int32, device=dev)))
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("theta,top", [(1e-10, 131071), (1e-6, 2**31 - 1), (0.5, 2**31 - 1), (1.0, 2**31 - 1)])
+def test_rope_angles_to_2_51(dev, theta, top):
+    """theta below 1 turns the frequencies into multiples: angles up to about 2^51, whose
+    reduction modulo pi/2 has to find the quadrant although angle * 2/pi is rounded.  A double
+    sin or cos within 1e-15 leaves a BF16 code at most one step from the oracle's."""
+    inp = _rope_inputs()[:64]
+    pos = np.array([top - 97 * i for i in range(32)] + [top >> i for i in range(1, 17)] + list(range(16)),
+                   dtype=np.int32)
+    got = to_codes(gqa.rope_half_split(to_dev(inp, dev), torch.from_numpy(pos).to(dev), theta=theta))
+    want = np.stack([[orc.f32_to_bf16(x) for x in orc.rope_row(orc.prepare_rows(r[None], False)[0], int(p), theta)]
+                     for r, p in zip(inp, pos)]).astype(np.uint16)
+    assert_within_ulp(want, got, 1, f"rope theta={theta}")
