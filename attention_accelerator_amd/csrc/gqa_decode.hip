@@ -59,6 +59,7 @@
 //    4q + l/16, dims 8(l%16) .. -- four whole rows per load instruction.  B lane l holds
 //    p of head l%4, key 4q + l/16, gathered through 512 bytes of LDS from the score lanes.
 //    C: lane l accumulates O[head l%4][8(4((l/4)%4) + l/16) + e] over all keys.
+#include <cmath>
 #include <cstring>
 
 #include "gqa_device.h"
@@ -199,13 +200,16 @@ __device__ __forceinline__ double exp2_f64(double x) {
 // ---- RoPE on cached K rows (a cache kept before rotation).  A lane of a 16-key chunk rotates 16
 // pairs of key kc + d, d = lane % 16.  Its (cos, sin) come from the chunk's first position kc,
 // one sincos per lane for the 64 frequencies shared through LDS, turned by the angle of d,
-// a table of 16 rotations per frequency that a workgroup forms once: rot(kc + d) = rot(kc)
-// rot(d).  Both are formed for the exact angles kc f and d f (the rounding error of the product,
-// which fma gives, turned back), and the result turned by the rounding error of (kc + d) f:
-// the golden rotates at the rounded angle.  Largest error against 113-bit values over positions
-// up to 400,000: 3.2e-16, rms 6.0e-17 (a sincos of the library per pair: 2.5e-16 and
-// 6.2e-17), in 12 fp64 instructions per pair instead of about 110.  Decode of 8 x 4096
-// unrotated keys: 80.8 us with that sincos per pair, 39.0 us so.
+// a table of 16 rotations per frequency that a workgroup forms once (rot_exact, rot_turn):
+// 14 fp64 instructions per pair, a sincos of the library per pair about 110.  Decode of 8 x
+// 4096 unrotated keys: 80.8 us with that sincos per pair, 39.0 us with the shared ones.
+//
+// kKRopeShared: so, for angles up to kKRopeMaxAngle (with theta >= 1 every cache that fits the
+// GPU).  kKRopePerPair: beyond it (theta below 1, whose frequencies pass 1) rot_turn's first order
+// is too little, and each pair has a sincos_f64 of its own.
+constexpr int kKRopeShared = 1;
+constexpr int kKRopePerPair = 2;
+
 struct KRopeLds {
     double2 rot[16][kWave];           // [pair 8kb + j][lane]: (cos, sin) of (lane % 16) f
     double2 base[4][kPairs];          // each wave's current chunk: (cos, sin) of kc f
@@ -217,34 +221,35 @@ __device__ __forceinline__ KRopeLds& k_rope_lds() {
     return t;
 }
 
-// cos and sin of the exact product p * f.
-__device__ __forceinline__ double2 rot_exact(double p, double f) {
-    const double ang = p * f;
-    const double dl = fma(p, f, -ang);
-    double s, c;
-    sincos_f64(ang, s, c);
-    return make_double2(fma(-dl, s, c), fma(dl, c, s));
-}
-
 // The table (every thread of the workgroup, once; ends with a barrier).
+template <int kRope>
 __device__ __forceinline__ void k_rope_init(const RopeTable& rope) {
     KRopeLds& t = k_rope_lds();
+    if (kRope == kKRopeShared) {
 #pragma unroll 2
-    for (int i = threadIdx.x; i < 16 * kWave; i += blockDim.x) {
-        const int l = i & (kWave - 1), pair = i >> 6;
-        t.rot[pair][l] = rot_exact(l & 15, rope.inv_freq[32 * (pair >> 3) + 8 * (l >> 4) + (pair & 7)]);
+        for (int i = threadIdx.x; i < 16 * kWave; i += blockDim.x) {
+            const int l = i & (kWave - 1), pair = i >> 6;
+            double2 d;
+            rot_exact(l & 15, rope.inv_freq[32 * (pair >> 3) + 8 * (l >> 4) + (pair & 7)], d.x, d.y);
+            t.rot[pair][l] = d;
+        }
     }
     if (threadIdx.x < kPairs) t.freq[threadIdx.x] = rope.inv_freq[threadIdx.x];
     __syncthreads();
 }
 
 // The chunk's K values (lane: key kc + lane % 16) rotated in double.
+template <int kRope>
 __device__ __forceinline__ void k_rope_rotate(int kc, const Chunk& c, double (&kr)[4][8]) {
     KRopeLds& t = k_rope_lds();
     const int lane = threadIdx.x & (kWave - 1);
     const int g = lane >> 4;
     double2* base = t.base[(threadIdx.x >> 6) & 3];
-    base[lane] = rot_exact(kc, t.freq[lane]);        // (one wave: its LDS accesses run in order)
+    if (kRope == kKRopeShared) {
+        double2 b;
+        rot_exact(kc, t.freq[lane], b.x, b.y);
+        base[lane] = b;                              // (one wave: its LDS accesses run in order)
+    }
     const double pos = kc + (lane & 15);
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
@@ -254,15 +259,15 @@ __device__ __forceinline__ void k_rope_rotate(int kc, const Chunk& c, double (&k
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int fi = 32 * kb + 8 * g + j;
-            const double2 b = base[fi];
-            const double2 d = t.rot[8 * kb + j][lane];
             const double f = t.freq[fi];
-            const double ang = pos * f;
-            const double dl = fma(pos, f, -ang);
-            const double cs0 = b.x * d.x - b.y * d.y;
-            const double sn0 = b.y * d.x + b.x * d.y;
-            const double cs = fma(dl, sn0, cs0);
-            const double sn = fma(-dl, cs0, sn0);
+            double cs, sn;
+            if (kRope == kKRopeShared) {
+                const double2 b = base[fi];
+                const double2 d = t.rot[8 * kb + j][lane];
+                rot_turn(b.x, b.y, d.x, d.y, pos, f, cs, sn);
+            } else {
+                sincos_f64(pos * f, sn, cs);
+            }
             const double x = xf[j], y = yf[j];
             kr[kb][j] = x * cs - y * sn;
             kr[kb + 2][j] = x * sn + y * cs;
@@ -271,7 +276,7 @@ __device__ __forceinline__ void k_rope_rotate(int kc, const Chunk& c, double (&k
 }
 
 // Scores, online softmax and weighted V of one chunk [kc, kc+16) (keys >= k_b masked).
-// kRope: each K row is rotated first, at its key index (k_rope_init has run).
+// kRope (0: none): each K row is rotated first, at its key index (k_rope_init<kRope> has run).
 template <int kRope>
 __device__ __forceinline__ void compute_chunk(int kc, int k_b, const Chunk& c, const QOps& qa, PieceState& st) {
     // p exchange slice of this wave (workgroups of up to four waves).
@@ -283,7 +288,7 @@ __device__ __forceinline__ void compute_chunk(int kc, int k_b, const Chunk& c, c
     if (kRope) {
         // Rotate the K row at its position in double: pairs (kb, kb+2) of this lane.
         double kr[4][8];
-        k_rope_rotate(kc, c, kr);
+        k_rope_rotate<kRope>(kc, c, kr);
 #pragma unroll
         for (int e = 0; e < 8; ++e)
 #pragma unroll
@@ -658,7 +663,7 @@ __device__ __forceinline__ void load_q_operands(const DecodeArgs& a, int b, int 
 // at a piece boundary.  Writes the output rows itself when the piece is the whole
 // segment; otherwise leaves a partial for the merge kernel.  (Requesting the next piece's
 // second chunk too, before this piece's end work, measured 1 % slower on long segments.)
-template <bool kRopeK>
+template <int kRopeK>
 __device__ __forceinline__ void process_piece(const DecodeArgs& a, int b, int kvh, int nv, int k_a,
                                               int k_b, int64_t wg, PieceRows& cur,
                                               const PieceRows& nxt, Chunk& c0, Chunk& c1,
@@ -731,7 +736,7 @@ __device__ __forceinline__ bool next_segment(const DecodeArgs& a, SeqWindow& sw,
     }
 }
 
-template <bool kRopeK>
+template <int kRopeK>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void decode_stream_kernel(DecodeArgs a) {
     // The first window of sequence offsets does not depend on the plan header: both are
     // requested at once.
@@ -762,7 +767,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void
             sw = t;
         }
     }
-    if (kRopeK) k_rope_init(a.rope);
+    if (kRopeK) k_rope_init<kRopeK>(a.rope);
     sw.lead = lead;
     int kvh, key, nvb;
     locate_first_piece(off, next, lead, x, kvh, key, nvb);
@@ -889,7 +894,7 @@ __device__ __forceinline__ bool load_first_page_chunk(const DecodeArgs& a, const
 // One piece whose first chunk is in c0.  The last iteration's second load fetches the first
 // chunk of `nx` (when has_next; its first block id nx_id0) into c0 -- so that the next
 // piece never waits for its first data -- and sets nx.ok.
-template <bool kRopeK>
+template <int kRopeK>
 __device__ __forceinline__ void process_page_piece(const DecodeArgs& a, const PagePiece& p, int64_t wg, Chunk& c0,
                                                    Chunk& c1, const QOps& qa, bool has_next, PagePiece& nx,
                                                    int nx_id0) {
@@ -953,7 +958,7 @@ __device__ __forceinline__ void process_page_piece(const DecodeArgs& a, const Pa
     write_partial(a, wg + static_cast<int64_t>(b) * kHkv + kvh, st, l_tot);
 }
 
-template <bool kRopeK>
+template <int kRopeK>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void decode_paged_stream_kernel(DecodeArgs a) {
     const int64_t w = blockIdx.x;
     const int64_t total = a.plan_hdr[0];
@@ -980,7 +985,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void
             sw = t;
         }
     }
-    if (kRopeK) k_rope_init(a.rope);
+    if (kRopeK) k_rope_init<kRopeK>(a.rope);
     PagePiece cur;
     {
         sw.lead = lead;
@@ -1161,7 +1166,7 @@ __device__ __forceinline__ void merge_at_once(const DecodeArgs& a, int64_t slot0
     }
 }
 
-template <bool kRopeQ, bool kRopeK>
+template <bool kRopeQ, int kRopeK>
 __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(DecodeArgs a) {
     __shared__ double q_s[kGroup][kD];
     __shared__ double o_s[kSingleWaves][kGroup][kD];     // each wave's O (blocks summed)
@@ -1225,7 +1230,7 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
         q_s[wave][lane + kPairs] = yr * a.qk_scale_log2;
     }
     if (kRopeK)
-        k_rope_init(a.rope);                             // (ends with a barrier)
+        k_rope_init<kRopeK>(a.rope);                             // (ends with a barrier)
     else
         __syncthreads();
     QOps qa;
@@ -2272,8 +2277,9 @@ hipError_t launch_set_words(int32_t* dst, const int32_t* words, int64_t n, hipSt
     return hipSuccess;
 }
 
-hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stream, hipEvent_t* ev) {
-    const bool rq = (a.flags & 1u) != 0, rk = (a.flags & 2u) != 0;
+template <int kRopeK>
+hipError_t launch_decode_k(const DecodeArgs& a, int batch, hipStream_t stream, hipEvent_t* ev) {
+    const bool rq = (a.flags & 1u) != 0;
     // Records the call's events from `from` on: a failed launch leaves none unrecorded, so
     // that the profiler can still read the call's stage times.
     auto done = [&](int from, hipError_t err) {
@@ -2285,14 +2291,10 @@ hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stream, hip
         // Single launch (small batches, contiguous cache).
         if (ev) (void)hipEventRecord(ev[0], stream);
         const dim3 grid(a.pieces_cap, batch * kHkv);
-        if (rq && rk)
-            hipLaunchKernelGGL((decode_single_kernel<true, true>), grid, dim3(kSingleWaves * kWave), 0, stream, a);
-        else if (rq)
-            hipLaunchKernelGGL((decode_single_kernel<true, false>), grid, dim3(kSingleWaves * kWave), 0, stream, a);
-        else if (rk)
-            hipLaunchKernelGGL((decode_single_kernel<false, true>), grid, dim3(kSingleWaves * kWave), 0, stream, a);
+        if (rq)
+            hipLaunchKernelGGL((decode_single_kernel<true, kRopeK>), grid, dim3(kSingleWaves * kWave), 0, stream, a);
         else
-            hipLaunchKernelGGL((decode_single_kernel<false, false>), grid, dim3(kSingleWaves * kWave), 0, stream, a);
+            hipLaunchKernelGGL((decode_single_kernel<false, kRopeK>), grid, dim3(kSingleWaves * kWave), 0, stream, a);
         return done(1, hipGetLastError());
     }
     if (rq)
@@ -2302,21 +2304,23 @@ hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stream, hip
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return done(0, e);
     if (ev) (void)hipEventRecord(ev[0], stream);
-    if (a.block_table) {
-        if (rk)
-            hipLaunchKernelGGL((decode_paged_stream_kernel<true>), dim3(a.n_wgs), dim3(kWave), 0, stream, a);
-        else
-            hipLaunchKernelGGL((decode_paged_stream_kernel<false>), dim3(a.n_wgs), dim3(kWave), 0, stream, a);
-    } else if (rk) {
-        hipLaunchKernelGGL((decode_stream_kernel<true>), dim3(a.n_wgs), dim3(kWave), 0, stream, a);
-    } else {
-        hipLaunchKernelGGL((decode_stream_kernel<false>), dim3(a.n_wgs), dim3(kWave), 0, stream, a);
-    }
+    if (a.block_table)
+        hipLaunchKernelGGL((decode_paged_stream_kernel<kRopeK>), dim3(a.n_wgs), dim3(kWave), 0, stream, a);
+    else
+        hipLaunchKernelGGL((decode_stream_kernel<kRopeK>), dim3(a.n_wgs), dim3(kWave), 0, stream, a);
     e = hipGetLastError();
     if (e != hipSuccess) return done(1, e);
     if (ev) (void)hipEventRecord(ev[1], stream);
     hipLaunchKernelGGL(decode_merge_kernel, dim3(kHkv, batch), dim3(kGroup * kWave), 0, stream, a);
     return done(2, hipGetLastError());
+}
+
+hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stream, hipEvent_t* ev) {
+    if (!(a.flags & 2u)) return launch_decode_k<0>(a, batch, stream, ev);
+    // The frequencies are powers of theta: the largest is the first (1) or the last.
+    const double top = a.capacity * std::fmax(a.rope.inv_freq[0], a.rope.inv_freq[kPairs - 1]);
+    return top <= kKRopeMaxAngle ? launch_decode_k<kKRopeShared>(a, batch, stream, ev)
+                                 : launch_decode_k<kKRopePerPair>(a, batch, stream, ev);
 }
 
 }  // namespace gqa

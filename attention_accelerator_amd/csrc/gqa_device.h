@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gqa_rope_math.h"
+
 namespace gqa {
 
 constexpr int kHq = 32;       // Q heads
@@ -230,54 +232,6 @@ __device__ __forceinline__ float bf16x2_sq_acc(uint32_t w, float acc) {
 __device__ __forceinline__ float wave_sum(float x) { return cross_row_sum(row16_sum(x)); }
 __device__ __forceinline__ float wave_max(float x) { return cross_row_max(row16_max(x)); }
 
-
-// sin and cos of an angle in double: reduced to |r| <= pi/4 with a two-part Cody-Waite pi/2
-// and fused multiply-adds, then the Taylor series of both (first omitted terms at pi/4: 9e-20
-// for the sine, 2.1e-18 for the cosine) and the quadrant.  The reduction runs twice: from
-// angles of about 2^46 on the rounding of angle * 2/pi can put k one off, and the second step
-// takes that back (on smaller angles its j is 0, or +-1 where r sits at pi/4).  Against 113-bit
-// values for every frequency of theta = 500000 at positions up to 400,000: largest error
-// 1.2e-16, rms 3.1e-17; over all angles below 2^53 1.9e-16 (the library's sincos of the angle
-// reduced modulo 2 pi: 2.5e-16 and 6.2e-17, in about three times the instructions; the kernels
-// here wait for one sincos after the other at their start).  From 2^54 on the two parts of pi/2
-// are too few bits and the error grows with the angle (1.9e-15 below 2^58); the clamp keeps
-// what is left past about 2^105 bounded.
-__device__ __forceinline__ void sincos_f64(double angle, double& s, double& c) {
-    const double k = rint(angle * 0.63661977236758134308);    // 2 / pi
-    double r = fma(-k, 1.5707963267948965580, angle);          // pi / 2 rounded to double
-    r = fma(-k, 6.1232339957367658e-17, r);                    // pi / 2 - that
-    const double j = rint(r * 0.63661977236758134308);
-    r = fma(-j, 1.5707963267948965580, r);
-    r = fma(-j, 6.1232339957367658e-17, r);
-    r = r > 0.8 ? 0.8 : r;
-    r = r < -0.8 ? -0.8 : r;
-    const double z = r * r;
-    double ps = 1.0 / 355687428096000.0;      // 1/17!
-    double pc = 1.0 / 20922789888000.0;       // 1/16!
-    ps = fma(ps, z, -1.0 / 1307674368000.0);
-    pc = fma(pc, z, -1.0 / 87178291200.0);
-    ps = fma(ps, z, 1.0 / 6227020800.0);
-    pc = fma(pc, z, 1.0 / 479001600.0);
-    ps = fma(ps, z, -1.0 / 39916800.0);
-    pc = fma(pc, z, -1.0 / 3628800.0);
-    ps = fma(ps, z, 1.0 / 362880.0);
-    pc = fma(pc, z, 1.0 / 40320.0);
-    ps = fma(ps, z, -1.0 / 5040.0);
-    pc = fma(pc, z, -1.0 / 720.0);
-    ps = fma(ps, z, 1.0 / 120.0);
-    pc = fma(pc, z, 1.0 / 24.0);
-    ps = fma(ps, z, -1.0 / 6.0);
-    const double sr = fma(r * z, ps, r);
-    const double hz = 0.5 * z;
-    const double w = 1.0 - hz;
-    const double cr = w + fma(z * z, pc, (1.0 - w) - hz);
-    // quadrant (k + j) mod 4 (both may exceed the int range, and their sum's last bit a double)
-    const double q = (k * 0.25 - floor(k * 0.25)) + j * 0.25;
-    const int n = static_cast<int>(4.0 * (q - floor(q)));
-    const double a = (n & 1) ? cr : sr, b = (n & 1) ? sr : cr;
-    s = (n & 2) ? -a : a;
-    c = ((n + 1) & 2) ? -b : b;
-}
 
 // sin and cos of angle = position * inv_freq, rounded to double as the golden forms it
 // (pyfiles/gen_gqa_wrapper_vectors.py:30).

@@ -14,6 +14,7 @@ import attention_accelerator_amd as gqa
 from attention_accelerator_amd import stimulus
 from oracle import oracle as orc
 from _util import assert_within_ulp, to_codes
+from test_gpu_paged import _paginate
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +51,27 @@ def test_rope_k_pieces_off_chunk_starts(dev, stream, length):
     got = to_codes(gqa.gqa_attention(b.q.to(dev), b.k.to(dev), b.v.to(dev), b.query_pos.to(dev), b.seq_len.to(dev),
                                      params=p))
     assert assert_within_ulp(want.reshape(-1, 128), got.reshape(-1, 128), 64, f"L={length}") <= 1
+
+
+# The smallest theta whose angles over 2112 positions stay within 2^26, where a chunk's rotations
+# are shared; below it each pair has a sincos of its own.
+_LINE = (2.0 ** 26 / 2112) ** (-128.0 / 126.0)
+
+
+@pytest.mark.parametrize("path", ["single", "stream", "paged"])
+@pytest.mark.parametrize("theta", [1.001 * _LINE, 0.999 * _LINE, 1e-9, 1e-12])
+def test_rope_k_large_angles(dev, path, theta):
+    """RoPE on K with frequencies above 1: angles about 2^26, 2^41 and 2^50 (where neighbouring
+    doubles lie 1/4 rad apart), each key at its rounded angle."""
+    lengths = [2100, 77, 1000]
+    b = stimulus.decode_batch(3, 2112, lengths=torch.tensor(lengths), seed=17)
+    want = orc.decode(to_codes(b.q), to_codes(b.k), to_codes(b.v), b.seq_len.numpy(), b.query_pos.numpy(),
+                      rope_q=False, rope_k=True, theta=theta)
+    p = gqa.make_params(rope_q=False, rope_k=True, theta=theta, stream_k=path == "stream")
+    pos, n = b.query_pos.to(dev), b.seq_len.to(dev)
+    if path == "paged":
+        kp, vp, table = _paginate(b.k, b.v, b.seq_len, 17)
+        got = to_codes(gqa.gqa_decode_paged(b.q.to(dev), kp.to(dev), vp.to(dev), table.to(dev), pos, n, params=p))
+    else:
+        got = to_codes(gqa.gqa_attention(b.q.to(dev), b.k.to(dev), b.v.to(dev), pos, n, params=p))
+    assert assert_within_ulp(want.reshape(-1, 128), got.reshape(-1, 128), 64, f"{path} theta={theta}") <= 1
