@@ -906,11 +906,13 @@ __device__ __forceinline__ void pf_pv(uint32_t vaddr, const uint32_t (&ph)[2][2]
 // before this kernel runs) and the block's rows up to its own (rs_kpre, rs_dpre).  Q's
 // pair-group norms come from the row as given (rotation leaves them unchanged): this lane
 // reads dims 8g .. 8g+7 and 32 + 8g .. (and their pairs 64 on), pair groups g and 4 + g.
-// y and its square in double, as in the multi-token merge (in fp32 y^2 underflows in every
-// dim of a row whose elements lie ~2^63 below their dims' largest |V|).  ul bounds the error
-// fp16's subnormal quantum added to every element (the attention loop's u over l; infinite for
-// rows that are always rescored): a row with an element below 8 ul, where that error could
-// reach 64 ULP with a margin of 2, is rescored as well.  Returns the decision for the row in every lane of its column.
+// The decision is formed in fp32 first, and where that cannot tell with y and its square in
+// double, as in the multi-token merge (in fp32 y^2 underflows in every dim of a row whose
+// elements lie ~2^63 below their dims' largest |V|).  ul bounds the error fp16's subnormal
+// quantum added to every element (the attention loop's u over l; infinite for rows that are
+// always rescored): a row with an element below 8 ul, where that error could reach 64 ULP with
+// a margin of 2, is rescored as well.  Returns the decision for the row in every lane of its
+// column.
 __device__ __forceinline__ bool pf_flag_row(const PrefillArgs& a, int b, int kvh, int st, int pos, int64_t row,
                                             float m, double ul, const uint2 (&pk)[8], int lane) {
     const int g = lane >> 4;
@@ -956,12 +958,13 @@ __device__ __forceinline__ bool pf_flag_row(const PrefillArgs& a, int b, int kvh
         const uint32_t w = i < 2 ? pk[dt].x : pk[dt].y;
         return __uint_as_float((i & 1) ? w & 0xffff0000u : w << 16);
     };
-    // A first decision in fp32: y and its squares lose range there (an element 2^63 below its
-    // D_j squares to zero, a subnormal D_j has no reciprocal), but only towards "cannot tell"
-    // -- a zero minimum, an infinite or NaN sum -- and its relative error is far below the 1 %
-    // margin, so a row it clears is clear.  About 1 % of the N(0,1) waves hold a row that it
-    // does not clear and form the decision in double below.  (The double version for every
-    // wave cost about 2 us at the end of each workgroup.)
+    // A first decision in fp32.  Where it can tell -- every square at or above kMinY2, so that
+    // none has lost bits to fp32's subnormals (an element 2^59 below its D_j and further), and
+    // no infinite or NaN sum (a zero or subnormal D_j has no reciprocal) -- its relative error
+    // is far below the 1 % margin, so a row it clears is clear.  About 1 % of the N(0,1) waves
+    // hold a row that it does not clear and form the decision in double below.  (The double
+    // version for every wave cost about 2 us at the end of each workgroup.)
+    constexpr float kMinY2 = 3.0092655e-36f;             // 2^-118
     float ss32 = 0.f, mn32 = INFINITY;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
@@ -989,7 +992,8 @@ __device__ __forceinline__ bool pf_flag_row(const PrefillArgs& a, int b, int kvh
     if (d_max >= 0x7f80u && (lane >> 4) == 0) atomicOr(a.rs_hdr + 2, 1u);
     const double ed = static_cast<double>(e) * fabs(a.qk_scale_log2);
     const double md = static_cast<double>(m);
-    bool flagged = bad || rs_flag_decide(-static_cast<double>(mn32), 1.01 * static_cast<double>(ss32), md, ed);
+    bool flagged = bad || !(-mn32 >= kMinY2) ||
+                   rs_flag_decide(-static_cast<double>(mn32), 1.01 * static_cast<double>(ss32), md, ed);
     if (__ballot(flagged && !bad)) {
         double ss = 0.0, mn2 = INFINITY;
 #pragma unroll

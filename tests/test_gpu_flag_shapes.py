@@ -214,3 +214,24 @@ def test_multi_tiny_weight_huge_v(dev):
     q = (q.float() * 2.0 ** 6).to(torch.bfloat16)
     vn = (vn.float() * 2.0 ** 120).to(torch.bfloat16)
     _run_and_check(q, kn, vn, k, v, starts, "multi-token T=16, Q x 2^6, chunk V x 2^120")
+
+
+@pytest.mark.parametrize("n_new", [17, 70])
+@pytest.mark.parametrize("small,flagged", [(1.0625 * 2.0 ** -15, True), (2.0 ** -12, False)])
+def test_prefill_flag_squares_below_fp32(dev, small, flagged, n_new):
+    """64 cached keys of score -155 (log2 units) and V = 2^60 before chunk keys of score 0 and V
+    = 1, in one dim `small`: every output is the chunk keys' V exactly, and in units of its dims'
+    largest |V| (2^60) its smallest square lies at 1.13 * 2^-150 or at 2^-144, its bound
+    (2^-34 F^2 / 128 times the sum of squares, F = 155 / 32) at 1.46 * 2^-150.  The first lies
+    below the bound although fp32 rounds it to 2^-149, above it."""
+    q = torch.ones((1, n_new, 32, 128), device=dev).to(torch.bfloat16)
+    kn = torch.zeros((1, n_new, 8, 128), device=dev).to(torch.bfloat16)
+    vn = torch.ones((1, n_new, 8, 128), device=dev).to(torch.bfloat16)
+    vn[..., 40] = small
+    k = torch.full((1, 8, 64 + n_new, 128), -9.5, device=dev).to(torch.bfloat16)
+    v = torch.full((1, 8, 64 + n_new, 128), 2.0 ** 60, device=dev).to(torch.bfloat16)
+    ws = torch.empty(gqa.prefill_workspace_bytes(1, n_new, 64 + n_new), dtype=torch.uint8, device=dev)
+    out = gqa.gqa_prefill(q, kn, vn, k, v, [64], rope_q=False, rope_k=False, workspace=ws)
+    assert torch.equal(out, vn[:, :, :1].expand_as(out))
+    rows = gqa.prefill_rescored_rows(ws, 1, n_new, 64 + n_new)
+    assert rows == (n_new * 32 if flagged else 0)
