@@ -1230,12 +1230,12 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     tl.u = 0.f;
     // The open group: blocks summed into tl.acc so far and their V scale exponent.  A block
     // whose V scale differs from the group's by more than 3 (its P would leave fp16's range
-    // or its precision) closes the group first.  A block with keys past the wave's first
-    // query is summed alone: its scales depend on rows that later tokens see and this token
-    // does not, and within a group a different scale would change how the other blocks'
-    // terms round, so this token's output would depend on keys its mask hides.  Alone, its
-    // sum only scales by a power of two.  (Blocks of chunk keys that every query of the wave
-    // sees join groups like cached ones.)
+    // or its precision) closes the group first.  A block holding chunk keys is summed alone.
+    // Its scales may depend on rows that later tokens see and this token does not, and within a
+    // group a different scale would change how the other blocks' terms round, so this token's
+    // output would depend on keys its mask hides; alone, its sum only scales by a power of two.
+    // And a prompt's blocks, all of them chunk blocks, meet in fp64: joined in fp32 (those that
+    // every query of the wave sees) two prompts of 1000 tokens took 116.6 us, so 119.1.
     int grp_n = 0, grp_sv = 0;
     int shut_sv = 0;                        // a group to close before the next products, its exponent
     bool shut = false;
@@ -1298,7 +1298,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
     auto p_off = [&](int shift, float m) {
         return static_cast<float>(kPScaleExp + shift) - (m == -INFINITY ? 0.f : m);
     };
-    int vshift = open_group(w_cur, blk_diag(blk0));
+    int vshift = open_group(w_cur, blk_new(blk0));
     float off = p_off(vshift, tl.m_run);
     float lsum = 0.f;
     uint32_t ph[2][2][4];
@@ -1329,7 +1329,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a)
         if (shut) pf_flush(tl, static_cast<double>(pow2f(-shut_sv)));
         const int sv_blk = grp_sv;               // this block's group
         const int l_shift = -vshift;
-        if (next) vshift = open_group(w_next, !kPlain && blk_diag(blk + 1));
+        if (next) vshift = open_group(w_next, !kPlain && blk_new(blk + 1));
 
         f32x4_t snext[4];
         VtPair vt[2];

@@ -13,7 +13,7 @@ import torch
 
 import attention_accelerator_amd as gqa
 from oracle import oracle as orc
-from _util import assert_within_ulp, to_codes, to_dev
+from _util import assert_within_ulp, to_codes, to_dev, ulp_distance
 
 pytestmark = pytest.mark.gpu
 
@@ -283,3 +283,27 @@ def test_kv_append_then_decode(dev):
     got = to_codes(gqa.gqa_attention(qd, kd, vd, starts, seq_len))
     want = orc.decode(to_codes(q[:, 0]), kc, vc, np.asarray(seq_len), np.asarray(starts))
     assert_within_ulp(want, got, 64, "append then decode")
+
+
+def test_prefill_chunk_blocks_meet_in_fp64(dev):
+    """Chunk keys 64..127 repeat keys 0..63 with V negated, the later keys have weights of about
+    2^-16: a row from token 192 on is the later keys' share alone, about 3 * 10^-6 of what the
+    first two blocks add and take back.  Where the blocks meet in fp64, one's fp32 sum is the
+    other's negative, but for a last bit in a few elements of a hundred; where one is summed onto
+    the other in fp32, most elements are left with an error of that bit, 2^-24 / 3 * 10^-6 = 2 %
+    of them or several ULP (53 in 100 measured; 3 with fp64).  Few of these rows go to the
+    rescore: no element is far below its row."""
+    n_new = 224
+    q, kn, vn, k, v = _chunk(1, n_new, n_new + 5, [0], 41)
+    q[:] = q[:, :1, ::4].repeat_interleave(4, dim=2)              # one query vector per KV head
+    kn[:, 64:128] = kn[:, :64]
+    kn[:, 128:] = -q[:, :1, ::4]
+    vn[:, 64:128] = -vn[:, :64]
+    ws = torch.empty(gqa.prefill_workspace_bytes(1, n_new, n_new + 5), dtype=torch.uint8, device=dev)
+    want = _oracle(q, kn, vn, k, v, [0], rope_q=False, rope_k=False)
+    got, _, _ = _run(q, kn, vn, k, v, [0], dev, rope_q=False, rope_k=False, workspace=ws)
+    rows = gqa.prefill_rescored_rows(ws, 1, n_new, n_new + 5)
+    print(f"{rows} of {n_new * 32} rows rescored", flush=True)
+    off = ulp_distance(want[:, 192:], got[:, 192:]) > 1
+    assert off.mean() < 0.15, f"{int(off.sum())} of {off.size} elements more than 1 ULP off"
+    assert rows < 100
