@@ -4,7 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "gqa_rope_math.h"
+#include "gqa_math.h"
 
 namespace gqa {
 

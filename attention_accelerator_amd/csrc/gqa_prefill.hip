@@ -1033,8 +1033,11 @@ __device__ __forceinline__ void pf_finish(const PrefillArgs& a, int b, int kvh, 
     uint2 pk[8];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
-        pk[dt].x = f32x2_to_bf16_out(static_cast<float>(o64[dt][0] * inv_l), static_cast<float>(o64[dt][1] * inv_l));
-        pk[dt].y = f32x2_to_bf16_out(static_cast<float>(o64[dt][2] * inv_l), static_cast<float>(o64[dt][3] * inv_l));
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = static_cast<float>(quotient(o64[dt][i], l, inv_l));
+        pk[dt].x = f32x2_to_bf16_out(x[0], x[1]);
+        pk[dt].y = f32x2_to_bf16_out(x[2], x[3]);
     }
     if (a.rs_hdr && __ballot(q_ok)) {
         if (pf_flag_row(a, b, kvh, st, st + t, row, m, ul, pk, lane) && q_ok && g == 0)

@@ -1,6 +1,8 @@
-"""RoPE's sines and cosines (csrc/gqa_rope_math.h) built for the host, against numpy's long
-double (64-bit mantissa) at the rounded angle, the one the golden rotates at
-(pyfiles/gen_gqa_wrapper_vectors.py:30).
+"""The kernels' double arithmetic (csrc/gqa_math.h) built for the host.
+
+RoPE's sines and cosines against numpy's long double (64-bit mantissa) at the rounded angle, the
+one the golden rotates at (pyfiles/gen_gqa_wrapper_vectors.py:30); the prefill epilogue's quotient
+against division.
 
 Bounds: the library's double sincos of the angle reduced modulo 2 pi, which these replace, has a
 largest error of 2.45e-16 against 113-bit values, over all angles below 2^53; sincos_f64 and a
@@ -21,7 +23,7 @@ _SRC = r"""
 #define __host__
 #define __device__
 #define __forceinline__ inline
-#include "gqa_rope_math.h"
+#include "gqa_math.h"
 extern "C" void sincos_all(const double* a, int n, double* s, double* c) {
     for (int i = 0; i < n; ++i) gqa::sincos_f64(a[i], s[i], c[i]);
 }
@@ -33,13 +35,16 @@ extern "C" void turned(const double* kc, const double* d, const double* f, int n
         gqa::rot_turn(bc, bs, dc, ds, kc[i] + d[i], f[i], c[i], s[i]);
     }
 }
+extern "C" void quotients(const double* a, const double* b, int n, double* q) {
+    for (int i = 0; i < n; ++i) q[i] = gqa::quotient(a[i], b[i], 1.0 / b[i]);
+}
 extern "C" double max_angle() { return gqa::kKRopeMaxAngle; }
 """
 
 
 @pytest.fixture(scope="module")
 def math(tmp_path_factory):
-    tmp = tmp_path_factory.mktemp("rope_math")
+    tmp = tmp_path_factory.mktemp("host_math")
     (tmp / "m.cpp").write_text(_SRC)
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=off",
                     f"-I{ROOT / 'attention_accelerator_amd/csrc'}", "-o", str(tmp / "m.so"), str(tmp / "m.cpp")],
@@ -91,3 +96,16 @@ def test_turned_rotation_error(math, theta, top):
     s, c = np.empty(n), np.empty(n)
     math.turned(_ptr(kc), _ptr(d), _ptr(f), n, _ptr(s), _ptr(c))
     assert _error((kc + d) * f, s, c) <= LIBRARY_ERROR
+
+
+def test_quotient_is_division(math):
+    """Bit for bit over O's and l's ranges (the product with 1 / l differs in about one of four)."""
+    rng = np.random.default_rng(9)
+    n = 1_000_000
+    b = np.ldexp(1.0 + rng.random(n), rng.integers(8, 44, n))
+    a = np.ldexp(1.0 + rng.random(n), rng.integers(-200, 180, n)) * rng.choice([-1.0, 1.0], n)
+    a[:100] = 0.0
+    q = np.empty(n)
+    math.quotients(_ptr(a), _ptr(b), n, _ptr(q))
+    assert (a * (1.0 / b) != a / b).mean() > 0.2
+    assert np.array_equal(q, a / b)
