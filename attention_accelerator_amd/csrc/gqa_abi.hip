@@ -97,14 +97,12 @@ int32_t multi_wgs(const gqa_params_t* p, int32_t n_new) {
     return w > 0 ? w : 1;
 }
 
-// Key runs per query block of the prefill attention kernel: one of its workgroups fills a CU
+// CUs that the prefill attention kernel's key runs may fill: one of its workgroups fills a CU
 // (kWavesPerCu persistent stream workgroups).
-int32_t prefill_splits_of(const gqa_params_t* p, int32_t batch, int32_t n_new) {
-    return prefill_splits(batch, n_new, stream_wgs(p) / kWavesPerCu);
-}
+int32_t prefill_cus(const gqa_params_t* p) { return stream_wgs(p) / kWavesPerCu; }
 
 size_t prefill_attn_bytes(const gqa_params_t* p, int32_t batch, int32_t n_new, int32_t capacity) {
-    return align_up(prefill_stage_bytes(batch, n_new, capacity, prefill_splits_of(p, batch, n_new)), 256);
+    return align_up(prefill_stage_bytes(batch, n_new, capacity, prefill_cus(p)), 256);
 }
 
 bool geometry_ok(const gqa_params_t* p) {
@@ -722,7 +720,7 @@ int gqa_prefill_bf16(const gqa_params_t* params, const uint16_t* q, const uint16
         rescore_layout(a, params, ws + align_up(prefill_multi_bytes(batch, n_new, multi_wgs(params, n_new)), 256), 1,
                        n_new, 0);
     } else {
-        a.n_split = prefill_splits_of(params, batch, n_new);
+        a.n_split = prefill_splits(batch, n_new, prefill_cus(params));
         prefill_stage_layout(a, workspace);
         rescore_layout(a, params, ws + prefill_attn_bytes(params, batch, n_new, kv->capacity),
                        prefill_chunk_blocks(n_new), 64, prefill_cache_blocks(kv->capacity));

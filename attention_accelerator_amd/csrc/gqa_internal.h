@@ -281,8 +281,9 @@ int32_t multi_simd_waves(int32_t n_new);
 
 // Workspace of the prefill attention path (chunks of more than kMultiMaxNew tokens): the
 // fp32 rotated new K rows, then the fp16 staging planes and block scales, then the partials of
-// the attention kernel's key runs (n_split > 1).
-size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity, int32_t n_split);
+// the attention kernel's key runs on a device of `cus` CUs.  No smaller batch, n_new or
+// capacity needs more.
+size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity, int32_t cus);
 void prefill_stage_layout(PrefillArgs& a, void* base);       // a.n_split set
 // Key runs per query block on a device of `cus` CUs.
 int32_t prefill_splits(int32_t batch, int32_t n_new, int32_t cus);

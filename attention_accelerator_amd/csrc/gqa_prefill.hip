@@ -96,8 +96,18 @@ struct SplitMl {
 };
 constexpr size_t kSplitMlB = size_t{kPfWaves} * kWave * sizeof(SplitMl);
 
-size_t split_slots(int32_t batch, int32_t n_new, int32_t n_split) {
-    return n_split > 1 ? static_cast<size_t>(batch) * kHkv * ((n_new + kPfPos - 1) / kPfPos) * n_split : 0;
+// Workgroups of the attention kernel without a split.
+int64_t query_blocks(int32_t batch, int32_t n_new) {
+    return static_cast<int64_t>(batch) * kHkv * ((n_new + kPfPos - 1) / kPfPos);
+}
+
+// Partials a workspace has room for: at least those of this call's split, and of every smaller
+// call's (fewer sequences or tokens may be cut into more runs), so that a workspace made for a
+// program's largest chunk holds its shorter ones too.
+size_t split_slots(int32_t batch, int32_t n_new, int32_t cus) {
+    if (cus < 2 * kHkv) return 0;                        // (the smallest call has kHkv query blocks)
+    const int64_t most = query_blocks(batch, n_new) * kPfMaxSplit;
+    return static_cast<size_t>(most < cus ? most : cus);
 }
 
 // The runs of a query block of n_blk key blocks: `per` blocks each, n of them (1: no partial).
@@ -110,22 +120,21 @@ __device__ __forceinline__ int pf_runs(int n_blk, int n_split, int& per) {
 }  // namespace
 
 int32_t prefill_splits(int32_t batch, int32_t n_new, int32_t cus) {
-    const int64_t wgs = static_cast<int64_t>(batch) * kHkv * ((n_new + kPfPos - 1) / kPfPos);
-    const int64_t n = cus / wgs;
+    const int64_t n = cus / query_blocks(batch, n_new);
     return n < 2 ? 1 : n > kPfMaxSplit ? kPfMaxSplit : static_cast<int32_t>(n);
 }
 
 // ---------------------------------------------------------------------------------
 // Workspace of the prefill attention path: the rotated new K rows in fp32, the fp16 K and
 // V planes, the trailing-part planes of the chunk blocks and the block scale words.
-size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity, int32_t n_split) {
+size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity, int32_t cus) {
     const size_t rows = static_cast<size_t>(batch) * n_new * kHkv;
     const size_t pos = (static_cast<size_t>(capacity) + kPfBlk - 1) / kPfBlk * kPfBlk;
     const size_t cb = static_cast<size_t>(prefill_chunk_blocks(n_new));
     const size_t bh = static_cast<size_t>(batch) * kHkv;
     return al256(rows * kD * sizeof(float)) + 2 * al256(bh * pos * kD * sizeof(uint16_t)) +
            al256(bh * cb * kPfBlk * kD * sizeof(uint16_t)) + al256(bh * (pos / kPfBlk) * sizeof(uint32_t)) +
-           split_slots(batch, n_new, n_split) * (kSplitOB + kSplitMlB);
+           split_slots(batch, n_new, cus) * (kSplitOB + kSplitMlB);
 }
 
 void prefill_stage_layout(PrefillArgs& a, void* base) {
@@ -145,7 +154,7 @@ void prefill_stage_layout(PrefillArgs& a, void* base) {
     a.stg_scale = reinterpret_cast<uint32_t*>(p);
     p += al256(bh * (a.stg_pos / kPfBlk) * sizeof(uint32_t));
     a.sp_o = reinterpret_cast<double2*>(p);
-    a.sp_ml = p + split_slots(a.batch, a.n_new, a.n_split) * kSplitOB;
+    a.sp_ml = p + static_cast<size_t>(query_blocks(a.batch, a.n_new)) * a.n_split * kSplitOB;
 }
 
 // ---------------------------------------------------------------------------------

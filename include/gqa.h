@@ -232,9 +232,11 @@ int gqa_kv_append_paged_bf16(const gqa_params_t* params, const uint16_t* k_new, 
  * with an fp64 recomputation of the output rows its kernels may have computed outside 64
  * BF16 ULP.  GQA_PLAN_NO_MULTI_TOKEN sends short chunks to the attention kernel too.  For
  * longer chunks the workspace grows with capacity (the staging planes hold 512 bytes per
- * position of every (sequence, KV head): 143 MB for batch 4 over 8704 positions); where the
- * query blocks (batch * 8 * ceil(n_new / 32)) fill at most half of the CUs, the attention
- * kernel cuts their keys into runs and the workspace holds up to 136 KB per CU of partials. */
+ * position of every (sequence, KV head): 143 MB for batch 4 over 8704 positions) and holds up
+ * to 136 KB per CU of partials: where the query blocks (batch * 8 * ceil(n_new / 32)) fill at
+ * most half of the CUs, the attention kernel cuts their keys into runs.  Chunks of more than
+ * 16 tokens never need more than a chunk of at least their batch, n_new and capacity, so a
+ * workspace for the longest chunk serves a shorter last one. */
 size_t gqa_prefill_workspace_bytes(const gqa_params_t* params, int32_t batch, int32_t n_new,
                                    int32_t capacity);
 

@@ -174,6 +174,26 @@ def test_prefill_workspace_bytes():
     assert L.gqa_prefill_workspace_bytes(ctypes.byref(p), 4, 512, 511) == 0
 
 
+@pytest.mark.parametrize("wgs", [0, 64, 256])
+def test_prefill_workspace_never_shrinks(wgs):
+    """A longer chunk, a larger batch or capacity never needs less (attention path, 17 tokens and
+    more), so a workspace for the largest call serves every smaller one."""
+    L = _lib.lib()
+    p = _params(flags=3, stream_wgs=wgs)
+
+    def size(b, n, c):
+        return L.gqa_prefill_workspace_bytes(ctypes.byref(p), b, n, c)
+
+    for b, c in ((1, 1024), (1, 8192), (2, 2048), (3, 2048), (4, 8704), (9, 1100)):
+        sizes = [size(b, n, c) for n in range(17, 1025)]
+        assert all(x <= y for x, y in zip(sizes, sizes[1:])), (b, c)
+    for n in (17, 32, 33, 100, 512):
+        sizes = [size(b, n, 1024) for b in range(1, 40)]
+        assert all(x <= y for x, y in zip(sizes, sizes[1:])), n
+        sizes = [size(1, n, c) for c in range(512, 4096, 16)]
+        assert all(x <= y for x, y in zip(sizes, sizes[1:])), n
+
+
 def _prefill(p, *, q=256, kn=256, vn=256, k=256, v=256, layout=None, start=256, batch=1,
              n_new=8, out=256, ws=256, ws_bytes=1 << 30):
     L = _lib.lib()

@@ -66,3 +66,19 @@ def test_runs_follow_stream_wgs(dev):
     a, _, _ = _run(q, kn, vn, k, v, starts, dev, params=one)
     b, _, _ = _run(q, kn, vn, k, v, starts, dev)
     assert_within_ulp(a.reshape(-1, 128), b.reshape(-1, 128), 64, "one run against many")
+
+
+def test_short_chunk_in_a_long_chunks_workspace(dev):
+    """A prompt in chunks of one length and a shorter last one (cut into more runs), in the
+    workspace that the long chunk asks for."""
+    cap, long, short = 1600, 512, 20
+    p = gqa.make_params(rope_k=True)
+    ws = torch.empty(gqa.prefill_workspace_bytes(1, long, cap, p), dtype=torch.uint8, device=dev)
+    for n_new, start in ((long, 0), (short, 1500), (long, 1000)):
+        q, kn, vn, k, v = _chunk(1, n_new, cap, [start], n_new + start)
+        got, _, _ = _run(q, kn, vn, k, v, [start], dev, params=p, workspace=ws)
+        alone, _, _ = _run(q, kn, vn, k, v, [start], dev, params=p)
+        assert np.array_equal(got, alone)
+        if n_new == short:
+            want = _oracle(q, kn, vn, k, v, [start])
+            assert_within_ulp(want.reshape(-1, 128), got.reshape(-1, 128), 64, "short chunk")
