@@ -71,7 +71,7 @@ def test_runs_follow_stream_wgs(dev):
 def test_short_chunk_in_a_long_chunks_workspace(dev):
     """A prompt in chunks of one length and a shorter last one (cut into more runs), in the
     workspace that the long chunk asks for."""
-    cap, long, short = 1600, 512, 20
+    cap, long, short = 2100, 1024, 20
     p = gqa.make_params(rope_k=True)
     ws = torch.empty(gqa.prefill_workspace_bytes(1, long, cap, p), dtype=torch.uint8, device=dev)
     for n_new, start in ((long, 0), (short, 1500), (long, 1000)):
