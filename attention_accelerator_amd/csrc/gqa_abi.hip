@@ -720,7 +720,7 @@ int gqa_prefill_bf16(const gqa_params_t* params, const uint16_t* q, const uint16
         rescore_layout(a, params, ws + align_up(prefill_multi_bytes(batch, n_new, multi_wgs(params, n_new)), 256), 1,
                        n_new, 0);
     } else {
-        a.n_split = prefill_splits(batch, n_new, prefill_cus(params));
+        a.n_split = prefill_splits(batch, n_new, kv->capacity, prefill_cus(params));
         prefill_stage_layout(a, workspace);
         rescore_layout(a, params, ws + prefill_attn_bytes(params, batch, n_new, kv->capacity),
                        prefill_chunk_blocks(n_new), 64, prefill_cache_blocks(kv->capacity));

@@ -286,7 +286,7 @@ int32_t multi_simd_waves(int32_t n_new);
 size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity, int32_t cus);
 void prefill_stage_layout(PrefillArgs& a, void* base);       // a.n_split set
 // Key runs per query block on a device of `cus` CUs.
-int32_t prefill_splits(int32_t batch, int32_t n_new, int32_t cus);
+int32_t prefill_splits(int32_t batch, int32_t n_new, int32_t capacity, int32_t cus);
 hipError_t launch_prefill_stage(const PrefillArgs& a, hipStream_t stream);
 // Workspace of the multi-token path: Q operands, plan, partials, chunk-key scores.
 size_t prefill_multi_bytes(int32_t batch, int32_t n_new, int32_t n_wgs);

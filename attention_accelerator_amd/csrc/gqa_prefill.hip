@@ -101,12 +101,19 @@ int64_t query_blocks(int32_t batch, int32_t n_new) {
     return static_cast<int64_t>(batch) * kHkv * ((n_new + kPfPos - 1) / kPfPos);
 }
 
+// Runs that the keys of `capacity` positions can be cut into: kPfMinRun blocks each, at most
+// kPfMaxSplit.
+int32_t most_runs(int32_t capacity) {
+    const int32_t n = (capacity + kPfBlk - 1) / kPfBlk / kPfMinRun;
+    return n < 2 ? 1 : n > kPfMaxSplit ? kPfMaxSplit : n;
+}
+
 // Partials a workspace has room for: at least those of this call's split, and of every smaller
 // call's (fewer sequences or tokens may be cut into more runs), so that a workspace made for a
 // program's largest chunk holds its shorter ones too.
-size_t split_slots(int32_t batch, int32_t n_new, int32_t cus) {
-    if (cus < 2 * kHkv) return 0;                        // (the smallest call has kHkv query blocks)
-    const int64_t most = query_blocks(batch, n_new) * kPfMaxSplit;
+size_t split_slots(int32_t batch, int32_t n_new, int32_t capacity, int32_t cus) {
+    if (cus < 2 * kHkv || most_runs(capacity) == 1) return 0;      // (the smallest call has kHkv query blocks)
+    const int64_t most = query_blocks(batch, n_new) * most_runs(capacity);
     return static_cast<size_t>(most < cus ? most : cus);
 }
 
@@ -119,9 +126,12 @@ __device__ __forceinline__ int pf_runs(int n_blk, int n_split, int& per) {
 
 }  // namespace
 
-int32_t prefill_splits(int32_t batch, int32_t n_new, int32_t cus) {
+// (The lengths are on the device: the capacity bounds what they can ask for.  A prompt of 200
+// tokens in a cache of 256 has one run per query block: no idle workgroups, no merge launch.)
+int32_t prefill_splits(int32_t batch, int32_t n_new, int32_t capacity, int32_t cus) {
     const int64_t n = cus / query_blocks(batch, n_new);
-    return n < 2 ? 1 : n > kPfMaxSplit ? kPfMaxSplit : static_cast<int32_t>(n);
+    const int64_t most = most_runs(capacity);
+    return n < 2 ? 1 : static_cast<int32_t>(n < most ? n : most);
 }
 
 // ---------------------------------------------------------------------------------
@@ -134,7 +144,7 @@ size_t prefill_stage_bytes(int32_t batch, int32_t n_new, int32_t capacity, int32
     const size_t bh = static_cast<size_t>(batch) * kHkv;
     return al256(rows * kD * sizeof(float)) + 2 * al256(bh * pos * kD * sizeof(uint16_t)) +
            al256(bh * cb * kPfBlk * kD * sizeof(uint16_t)) + al256(bh * (pos / kPfBlk) * sizeof(uint32_t)) +
-           split_slots(batch, n_new, cus) * (kSplitOB + kSplitMlB);
+           split_slots(batch, n_new, capacity, cus) * (kSplitOB + kSplitMlB);
 }
 
 void prefill_stage_layout(PrefillArgs& a, void* base) {

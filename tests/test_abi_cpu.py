@@ -194,6 +194,17 @@ def test_prefill_workspace_never_shrinks(wgs):
         assert all(x <= y for x, y in zip(sizes, sizes[1:])), n
 
 
+def test_prefill_workspace_of_a_short_cache_holds_no_partials():
+    """A cache of fewer than eight 64-position blocks is never cut into runs (a run keeps at least
+    four): no partials (about 34 MB on a whole GPU), whatever the chunk."""
+    L = _lib.lib()
+    p = _params(flags=3, stream_wgs=1024)
+    for n in (17, 200, 400):
+        at = [L.gqa_prefill_workspace_bytes(ctypes.byref(p), 1, n, c) for c in (448, 449)]
+        assert at[0] < 12 << 20
+        assert at[1] - at[0] > 2 * 8 * (128 + 8) * 1024          # at least two runs of eight query blocks
+
+
 def _prefill(p, *, q=256, kn=256, vn=256, k=256, v=256, layout=None, start=256, batch=1,
              n_new=8, out=256, ws=256, ws_bytes=1 << 30):
     L = _lib.lib()
