@@ -307,3 +307,25 @@ def test_prefill_chunk_blocks_meet_in_fp64(dev):
     off = ulp_distance(want[:, 192:], got[:, 192:]) > 1
     assert off.mean() < 0.15, f"{int(off.sum())} of {off.size} elements more than 1 ULP off"
     assert rows < 100
+
+
+def test_prefill_two_byte_aligned_inputs(dev):
+    """Q and the new K/V rows at 2-byte (not 16-byte) aligned addresses: the same bits as aligned
+    inputs, in rows that the attention kernel ends and in rows of the rescore (a Q head 2^100
+    times larger)."""
+    starts = [300, 9]
+    q, kn, vn, k, v = _chunk(2, 40, 345, starts, 48)
+    q[:, :, 6] = (q[:, :, 6].float() * 2.0 ** 100).to(torch.bfloat16)
+    want, _, _ = _run(q, kn, vn, k, v, starts, dev)
+
+    def shifted(x):
+        flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=dev)
+        view = flat[1:].view(x.shape)
+        view.copy_(x.to(dev))
+        return view
+
+    qs, kns, vns = shifted(q), shifted(kn), shifted(vn)
+    assert qs.data_ptr() % 16 != 0 and kns.data_ptr() % 16 != 0
+    got = to_codes(gqa.gqa_prefill(qs, kns, vns, k.to(dev), v.to(dev), starts))
+    torch.cuda.synchronize()
+    assert np.array_equal(got, want)
