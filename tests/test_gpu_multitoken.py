@@ -320,18 +320,24 @@ def test_rescore_pieces(dev, n_wgs, heads):
     (24, False, False),   # no RoPE at all
 ])
 def test_every_row_rescored(dev, n_new, rope_q, rope_k):
-    """V dimension 5 is exactly zero in every row, so every output row holds an exact zero
-    and is flagged for the fp64 rescore (min |x| = 0 < 2^-17 rms): the rescore runs with
-    one piece per row (more flagged rows than workgroups) and must reproduce every row of
-    the oracle, the zero dimension exactly."""
+    """K is zero in RoPE pairs 0..3 and Q 2^20 times larger there: scores of N(0,1) size whose
+    bound |q| |k| passes 10^5, so that every row is flagged for the fp64 rescore, which runs
+    with one piece per tile (at least as many tiles as workgroups) and must reproduce every row of the
+    oracle, V dimension 5, zero in every key, exactly.  (A dimension of zeros flags no row.)"""
     starts = [37, 300, 1000, 8, 513, 64, 2049, 129][: 8 if n_new <= 16 else 3]
     cap = max(starts) + n_new
     q, kn, vn, k, v = _chunk(starts, n_new, cap, 40 + n_new)
     vn[..., 5] = 0.0
+    pairs = [0, 1, 2, 3, 64, 65, 66, 67]
+    q[..., pairs] = (q[..., pairs].float() * 2.0 ** 20).to(torch.bfloat16)
+    kn[..., pairs] = 0.0
     for b, s in enumerate(starts):
         v[b, :, :s, 5] = 0.0
+        k[b, :, :s, pairs] = 0.0
     want = _oracle(q, kn, vn, k, v, starts, rope_q=rope_q, rope_k=rope_k)
-    got, _, _ = _run(q, kn, vn, k, v, starts, dev, rope_q=rope_q, rope_k=rope_k)
+    ws = torch.empty(gqa.prefill_workspace_bytes(len(starts), n_new, cap), dtype=torch.uint8, device=dev)
+    got, _, _ = _run(q, kn, vn, k, v, starts, dev, rope_q=rope_q, rope_k=rope_k, workspace=ws)
+    assert gqa.prefill_rescored_rows(ws, len(starts), n_new, cap) == len(starts) * n_new * 32
     assert np.all(got[..., 5] == 0)
     w = _check(want, got.reshape(-1, 128), f"T={n_new} rope_q={rope_q} rope_k={rope_k}, all rows rescored")
     print("worst ULP", w)
