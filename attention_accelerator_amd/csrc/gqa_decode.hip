@@ -1397,14 +1397,21 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
 // dims {8c + i, 64 + 8c + i : i < 8}, c = l % 8 -- 8 rotate_half pairs, so a chunk key's
 // rotation is lane-local.  A key's score is the sum over its eight lanes; each lane
 // accumulates p * V over its own keys for its 16 dims, and the 8 key slots are summed once
-// per wave, the four waves' sums per piece.  The workgroups take (row, piece) pairs, wave w of
-// piece p of a row taking its chunks 4p + w, 4(p + n_pieces) + w, ..., so that the waves share
-// the costlier chunk keys evenly.  With at most 64 flagged rows (one per lane) every workgroup reads all of them
-// and gives each row pieces in proportion to its chunks (at least kRsMinChunks per piece, at
-// most kRsMaxPieces pieces): the longest row, which sets the kernel's time, gets the most.
-// With more rows each gets gridDim / rows pieces.  A row's result depends on its keys and
-// its piece count only, which follow from the flagged rows' key counts and the grid, never
-// from the order they were flagged in.
+// per wave.  Two plans.
+//
+// Up to 64 flagged rows (one per lane): every workgroup reads all of them and gives each row
+// pieces in proportion to its chunks (at least kRsMinChunks per piece, at most kRsMaxPieces
+// pieces): the longest row, which sets the kernel's time, gets the most.  A workgroup's four
+// waves share a piece -- wave w of piece p takes chunks 4p + w, 4(p + n_pieces) + w, .., so that
+// the waves share the costlier chunk keys evenly -- and their sums meet in LDS: a quarter of
+// the pieces to merge.
+//
+// More rows: each gets waves / rows pieces, and every wave takes (row, piece) pairs by itself.
+// With four waves to a piece 365 rows are 365 pieces for 256 workgroups, two rounds where one and
+// a half would do, and each round pays a piece's start and sums; the step ROWS_TIMES.
+//
+// A row's result depends on its keys and its piece count only, which follow from the flagged
+// rows' key counts and the grid, never from the order they were flagged in.
 
 constexpr int kRsKeys = 8;              // keys per rescore chunk (one per 8 lanes)
 constexpr int kRsWaves = 4;             // waves per rescore workgroup
@@ -1680,13 +1687,16 @@ __device__ __forceinline__ uint32_t rs_out2(double o0, double o1, double l) {
            (static_cast<uint32_t>(f32_to_bf16_out(static_cast<float>(o1 / l))) << 16);
 }
 
+// kTeam: waves that share an item (kRsWaves with the proportional plan, 1 with the uniform one).
+template <int kTeam>
 __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_rows) {
     __shared__ double o_s[kRsWaves][kRsKeys][8][17];      // per wave, key slot and lane group (16, padded)
     __shared__ double2 ow_s[kRsWaves][kWave];             // each wave's O (dims 2i, 2i + 1)
     __shared__ double2 ml_s[kRsWaves];                    // and its (m, l)
     __shared__ int last_s;
     const int T = a.n_new;
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int tw = kTeam > 1 ? wave : 0;                  // this wave's place in its team
     const int lane = threadIdx.x & (kWave - 1);
     const int c = lane & 7;
     // The plan.  Proportional (n_rows <= 64): lane r holds row r, its pieces np_l and its
@@ -1694,7 +1704,9 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
     // slots have the same numbers (the items stay below gridDim.x <= kRsSlots: the piece size
     // is set for gridDim.x - n_rows pieces, and rounding up adds at most one per row).
     // Uniform otherwise: n_pieces per row, row idx at items idx * n_pieces ...
-    const bool prop = n_rows <= static_cast<uint32_t>(kWave);
+    constexpr bool prop = kTeam > 1;
+    const int64_t n_teams = static_cast<int64_t>(gridDim.x) * (kRsWaves / kTeam);
+    const int64_t team = kTeam > 1 ? blockIdx.x : static_cast<int64_t>(wave) * gridDim.x + blockIdx.x;
     uint32_t row_l = 0;
     int np_l = 0, first_l = 0, st_l = 0;
     int64_t n_work;
@@ -1715,11 +1727,11 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
         first_l = incl - np_l;
         n_work = __shfl(incl, kWave - 1);
     } else {
-        n_pieces = gridDim.x / n_rows;      // gridDim.x <= kRsSlots
+        n_pieces = static_cast<uint32_t>(min(n_teams, int64_t{kRsSlots})) / n_rows;
         n_pieces = n_pieces < 1 ? 1 : n_pieces > kRsMaxPieces ? kRsMaxPieces : n_pieces;
         n_work = static_cast<int64_t>(n_rows) * n_pieces;
     }
-    for (int64_t wk = blockIdx.x; wk < n_work; wk += gridDim.x) {
+    for (int64_t wk = team; wk < n_work; wk += n_teams) {
         uint32_t idx, row;
         int piece, np, st = 0;
         int64_t slot0;
@@ -1756,7 +1768,7 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
         const int n_chunks = (it.n_keys + kRsKeys - 1) / kRsKeys;
         // first chunk holding a chunk key (with RoPE on K those are rotated from the new rows)
         const int c_split = (a.flags & 2u) ? it.st / kRsKeys : n_chunks;
-        const int first = kRsWaves * piece + wave, step = kRsWaves * np;     // this wave's chunks
+        const int first = kTeam * piece + tw, step = kTeam * np;     // this wave's chunks
 
         // Q of head h at token t, rotated at start + t (the cos/sin row of token t) and
         // scaled by scale * log2(e): this lane's 8 pairs.  Its loads are issued first, then
@@ -1793,7 +1805,7 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
         rs_new(it, rs_first(first, step, c_split), n_chunks, step, q, stt);
 
         // The wave's O over its 8 key slots (through its part of LDS, summed in slot order)
-        // and l; then the waves' sums, in wave order, by wave 0.
+        // and l; then the team's sums, in wave order, by its first wave.
 #pragma unroll
         for (int i = 0; i < 16; ++i) o_s[wave][lane >> 3][c][i] = stt.o[i];
         double l_tot = stt.l;
@@ -1811,24 +1823,30 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
             o0 += o_s[wave][jj][cd][ii];
             o1 += o_s[wave][jj][cd][ii + 1];
         }
-        ow_s[wave][lane] = make_double2(o0, o1);
-        if (lane == 0) ml_s[wave] = make_double2(stt.m, l_tot);
-        __syncthreads();
+        double m_tot = stt.m;
+        if (kTeam > 1) {
+            ow_s[wave][lane] = make_double2(o0, o1);
+            if (lane == 0) ml_s[wave] = make_double2(stt.m, l_tot);
+            __syncthreads();
+        }
         uint32_t* orow = reinterpret_cast<uint32_t*>(a.out + static_cast<int64_t>(row) * kD);
-        if (wave == 0) {
-            double m_tot = ml_s[0].x;
+        int last = 0;
+        if (tw == 0) {
+            if (kTeam > 1) {
+                m_tot = ml_s[0].x;
 #pragma unroll
-            for (int w = 1; w < kRsWaves; ++w) m_tot = fmax(m_tot, ml_s[w].x);
-            o0 = 0.0;
-            o1 = 0.0;
-            l_tot = 0.0;
+                for (int w = 1; w < kTeam; ++w) m_tot = fmax(m_tot, ml_s[w].x);
+                o0 = 0.0;
+                o1 = 0.0;
+                l_tot = 0.0;
 #pragma unroll
-            for (int w = 0; w < kRsWaves; ++w) {
-                const double2 ml = ml_s[w], ow = ow_s[w][lane];
-                const int ex = ml.x == -INFINITY ? -1100 : max_shift_f64(ml.x, m_tot);   // (no key: weight 0)
-                l_tot += ldexp(ml.y, ex);
-                o0 += ldexp(ow.x, ex);
-                o1 += ldexp(ow.y, ex);
+                for (int w = 0; w < kTeam; ++w) {
+                    const double2 ml = ml_s[w], ow = ow_s[w][lane];
+                    const int ex = ml.x == -INFINITY ? -1100 : max_shift_f64(ml.x, m_tot);   // (no key: weight 0)
+                    l_tot += ldexp(ml.y, ex);
+                    o0 += ldexp(ow.x, ex);
+                    o1 += ldexp(ow.y, ex);
+                }
             }
             if (np == 1) {
                 orow[lane] = rs_out2(o0, o1, l_tot);
@@ -1844,27 +1862,37 @@ __device__ __forceinline__ void rs_rows_path(const PrefillArgs& a, uint32_t n_ro
                 }
                 wait_vmem();                              // the stores have completed ...
                 __atomic_signal_fence(__ATOMIC_SEQ_CST);  // ... and stay before the count
-                if (lane == 0) last_s = atomicAdd(&a.rs_done[row], 1u) == static_cast<uint32_t>(np) - 1u;
+                if (lane == 0) last = atomicAdd(&a.rs_done[row], 1u) == static_cast<uint32_t>(np) - 1u;
+                if (kTeam > 1 && lane == 0) last_s = last;
             }
         }
-        __syncthreads();                // (also: ow_s and ml_s have been read)
-        if (np == 1 || !last_s) continue;
+        if (kTeam > 1) {
+            __syncthreads();            // (also: ow_s and ml_s have been read)
+            last = last_s;
+        } else {
+            last = __shfl(last, 0);
+        }
+        if (np == 1 || !last) continue;
         __atomic_signal_fence(__ATOMIC_SEQ_CST);      // the merge's loads stay after the count
-        // Lane u of each wave reads piece u's (m, l); wave w sums pieces w, w + 4, .., lane i
-        // dims 2i, 2i + 1.
+        // Lane u of each wave reads piece u's (m, l); wave w of a team sums pieces w, w + kTeam,
+        // .., lane i dims 2i, 2i + 1.
         const double2 ml = load_agent_d2(reinterpret_cast<const double*>(a.rs_part_ml + slot0 + min(lane, np - 1)));
         const int my_ex = rs_piece_ex(ml);
         o0 = 0.0;
         o1 = 0.0;
-        rs_sum_pieces(a.rs_part_o + slot0 * kD + 2 * lane, kD, wave, kRsWaves, np, my_ex, o0, o1);
+        rs_sum_pieces(a.rs_part_o + slot0 * kD + 2 * lane, kD, tw, kTeam, np, my_ex, o0, o1);
+        const double lw = rs_piece_l(ml, my_ex, np);
+        if (kTeam == 1) {
+            orow[lane] = rs_out2(o0, o1, lw);
+            continue;
+        }
         ow_s[wave][lane] = make_double2(o0, o1);
         __syncthreads();
         if (wave == 0) {
-            const double lw = rs_piece_l(ml, my_ex, np);
             o0 = 0.0;
             o1 = 0.0;
 #pragma unroll
-            for (int w = 0; w < kRsWaves; ++w) {
+            for (int w = 0; w < kTeam; ++w) {
                 o0 += ow_s[w][lane].x;
                 o1 += ow_s[w][lane].y;
             }
@@ -2224,7 +2252,10 @@ __global__ __launch_bounds__(kRsWaves * kWave) void rescore_kernel(PrefillArgs a
     if (n_rows == 0) return;
     const uint32_t n_pairs = a.rs_hdr[1];
     if (a.rs_hdr[2] != 0u || static_cast<uint64_t>(n_rows) < static_cast<uint64_t>(kRsTileFill) * n_pairs) {
-        rs_rows_path(a, n_rows);
+        if (n_rows <= static_cast<uint32_t>(kWave))
+            rs_rows_path<kRsWaves>(a, n_rows);
+        else
+            rs_rows_path<1>(a, n_rows);
         return;
     }
     const RsPairs pairs = rs_load_pairs(a, 0, 0);

@@ -111,9 +111,9 @@ def test_tiles_of_spread_weights(dev, n_new, starts, wgs):
     (1, [8190], 0, [0]),                          # long rows, shared by the whole grid
     (8, [3000, 40], 64, [2, 7]),                  # two rows per pair; 16 workgroups for 32 rows
     (40, [2000], 0, [0, 39]),                     # the attention kernel's rows
-    (1, [300 + 37 * i for i in range(12)], 0, [0]),       # 96 rows: the same pieces for every row, two each
-    (1, [90, 2500, 800] * 3, 4096, [0]),          # 72 rows on the largest grid: 14 pieces each
-    (2, [30 + 11 * i for i in range(5)], 32, [0, 1]),     # 80 rows on eight workgroups: a piece per row
+    (1, [300 + 37 * i for i in range(12)], 0, [0]),       # 96 rows: the same pieces for every row, a wave each
+    (1, [90, 2500, 800] * 3, 4096, [0]),          # 72 rows on the largest grid: as many pieces as there are slots for
+    (2, [30 + 11 * i for i in range(5)], 32, [0, 1]),     # 80 rows on eight workgroups: a piece per row, three rounds
 ])
 def test_rows_of_spread_weights(dev, n_new, starts, wgs, tokens):
     """One head per KV head: fewer than three rows per pair, each by itself."""
