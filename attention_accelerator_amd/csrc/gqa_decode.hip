@@ -1385,14 +1385,16 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
 // chunks (2.4 + 3.5 us), the chunks, the sums, the count, the merge.  One-wave pieces, four
 // times as many, spent 4 to 6 us on the merge alone and 2 us per chunk of new keys, whose (cos,
 // sin) rows were read when needed (now with the chunk's rows): two prompts of 1000 tokens (148
-// rows) step 132.9 -> 119.8 us, 1000 over 4000 (101 rows) 247 -> 220, four prompts of 1000 with
-// 1300 rows 272 -> 268; rows path: 200 over 5003 (4 rows) 100.9 -> 98.6, 4 x 512 over 8192 (55
-// rows) 653 -> 650, T = 4 / 16 of 64 sequences (6 / 30 rows) 246.6 -> 243.2 / 385 -> 382.
-// Two such workgroups per CU do not fit: at 256 registers per wave the
-// chunks in flight spill (slower by 1 to 8 %).
+// rows) step 132.9 -> 119.8 us, 1000 over 4000 (101 rows) 247 -> 220; rows path: 200 over 5003
+// (4 rows) 100.9 -> 98.6; T = 4 of 64 sequences (9 rows) rescore 23.3 -> 17.5 (the step's gain is
+// within the runs' spread).  With many tiles the time is fp64 issue, and a long piece per wave
+// pays a piece's fixed cost once: Q x 16 over 4 x 512 tokens and 8192 (761 rows) 166 us with
+// one-wave pieces, 182 here; with Q x 64 (3016 rows) the claims balance better, 703 and 582.
+// Two such workgroups per CU do not fit: at 256 registers per wave the chunks in flight spill
+// (slower by 1 to 8 %).
 
-// Rows path (the flagged rows spread thin over their (sequence, KV head) pairs): one row per
-// wave, fp64 VALU (an fp64 MFMA would compute four columns for one and costs more than the
+// Rows path (the flagged rows spread thin over their (sequence, KV head) pairs): one row at a
+// time per wave, fp64 VALU (an fp64 MFMA would compute four columns for one and costs more than the
 // VALU chain for a single row) -- lane l holds key slot l/8 of an 8-key chunk and the 16
 // dims {8c + i, 64 + 8c + i : i < 8}, c = l % 8 -- 8 rotate_half pairs, so a chunk key's
 // rotation is lane-local.  A key's score is the sum over its eight lanes; each lane
@@ -1408,7 +1410,10 @@ __global__ __launch_bounds__(kSingleWaves * kWave) void decode_single_kernel(Dec
 //
 // More rows: each gets waves / rows pieces, and every wave takes (row, piece) pairs by itself.
 // With four waves to a piece 365 rows are 365 pieces for 256 workgroups, two rounds where one and
-// a half would do, and each round pays a piece's start and sums; the step ROWS_TIMES.
+// a half would do, and each round pays a piece's start and sums (steps on a cold cache: 16
+// tokens of 8 sequences over 16000, 178 rows, 396 us, so 364; 8 of 32 over 8000, 368 rows, 523
+// and 477; 16 of 32 over 500, 665 rows, 133 and 124).  With 70 rows, just past the line, the
+// kernel takes 35 us either way.
 //
 // A row's result depends on its keys and its piece count only, which follow from the flagged
 // rows' key counts and the grid, never from the order they were flagged in.

@@ -152,7 +152,8 @@ struct PrefillArgs {
     // fp64 rescore of the output rows the MFMA kernels may have computed outside 64 BF16 ULP
     // (the attention epilogue or the multi-token merge decides, rescore_kernel recomputes); rs_hdr
     // nullptr: off.
-    uint32_t* rs_hdr;         // [2]: flagged rows, (sequence, KV head) pairs with one
+    uint32_t* rs_hdr;         // [64]: flagged rows, (sequence, KV head) pairs with one, whether a flagged
+                              // row sees a V that is not finite; [kRsClaim]: items of the tiles path claimed
     uint32_t* rs_flat;        // [B*T*32] flagged rows (b*T + t)*32 + q_head, in flagging order
     uint32_t* rs_rows;        // [B*8][4T] the same rows by (sequence, KV head)
     uint32_t* rs_gcnt;        // [B*8] flagged rows per (sequence, KV head)

@@ -9,7 +9,8 @@
 // chunk's own K/V rows, rotated at their positions in double and not re-rounded, as
 // the golden rotates K (gen_gqa_wrapper_vectors.py:124-126).
 //
-// Four launches, then the fp64 rescore of flagged rows (gqa_decode.hip):
+// Four launches, or five where few query blocks have their keys cut into runs, then the fp64
+// rescore of flagged rows (gqa_decode.hip):
 //
 // kv_append_kernel writes the chunk's K rows (rotated, rounded double -> f32 -> BF16,
 // pyfiles/gqa_reference.py:15-19) and V rows into the cache, and the rotated K rows in fp32
@@ -48,11 +49,14 @@
 //    The lane already holds P for keys {4g+i} of tiles 2w and 2w+1, which is its B
 //    operand for the 32-key window w if V^T stores each window's keys in that order
 //    (slot 8g+4h+i <-> key 16h+4g+i).  P, scaled by 2^12, is split into two fp16 parts
-//    (rounded to nearest: ~22 bits).  Each block's fp32 product is scaled by the block's
-//    V scale into an fp64 accumulator, so accumulation over thousands of keys adds no fp32
-//    rounding.
+//    (rounded to nearest: ~22 bits).  The fp32 products of a group of up to four cached
+//    blocks, or of one block holding chunk keys, are scaled by the group's V scale into an
+//    fp64 accumulator, so that accumulation over thousands of keys adds no fp32 rounding.
 //  * O / l, rounded double -> f32 -> BF16, written in Q-head order; the row's rescore flag
 //    decided from those BF16 values (pf_flag_row).
+//
+// prefill_merge_kernel: where a query block's keys were cut into runs, a workgroup each, sums
+// the runs' fp64 partials and ends the rows in the attention kernel's stead.
 //
 // Chunks of at most 16 new tokens take the multi-token decode path instead
 // (gqa_multitoken.hip), which shares this file's LDS row layout (gqa_prefill_common.h).
@@ -76,12 +80,13 @@ constexpr int kPScaleExp = 12;             // P is formed as 2^12 * 2^(s - m) <=
 
 // Key splits of the attention kernel.  One workgroup per (sequence, KV head, 32 positions)
 // leaves most of the chip idle for a short chunk of one or a few sequences (200 tokens of one
-// sequence: 56 workgroups on 256 CUs), however long the context is.  When at least two
-// workgroups per CU-slot fit (a workgroup's LDS and registers fill a CU), each query block's
-// keys are cut into n_split runs of whole blocks, one workgroup each, whose fp64 partials
-// prefill_merge_kernel combines: as many as fit in one round of the CUs, so that a split never
-// adds a round.  A run keeps at least kPfMinRun blocks (a workgroup costs about 10 us besides
-// its blocks of 1.8 us each, and a partial is 136 KB to write and read).
+// sequence: 56 workgroups on 256 CUs), however long the context is.  When the CUs hold the
+// query blocks at least twice over (a workgroup's LDS and registers fill a CU), each query
+// block's keys are cut into up to n_split runs of whole blocks, one workgroup each, whose fp64
+// partials prefill_merge_kernel combines: as many as fit in one round of the CUs, so that a
+// split never adds a round.  Every run but the last has at least kPfMinRun blocks (a workgroup
+// costs about 15 us, its launch included, besides its blocks of 1.6 us each, measured with 8
+// to 128 blocks; and a partial is 136 KB to write and read).
 constexpr int kPfMaxSplit = 32;
 constexpr int kPfMinRun = 4;
 

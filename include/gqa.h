@@ -273,12 +273,12 @@ int gqa_rope_rows_bf16(const uint16_t* in, uint16_t* out, int64_t n_rows, int64_
  * call brackets its kernels with HIP events on the call's stream (up to `max_calls`
  * calls are recorded; later ones are not), in up to four stages: decode {stream kernel,
  * merge kernel} (the Q-operand preparation kernel runs before the first event), prefill
- * {KV append, staging and reduce kernels; attention kernel; fp64 rescore}, prefill of at
- * most 16 new tokens {preparation kernel (with the append); stream kernel; merge kernel;
- * fp64 rescore}.  gqa_profile_read waits for the recorded events, returns the summed times
- * of the first two stages and the number of calls recorded, and clears the record;
- * gqa_profile_read_stages does the same for up to four stages (a path's missing stages
- * read 0).  Not for the hot path: enabling creates the events.  No reference counterpart
+ * {KV append, staging and reduce kernels; attention kernel and the merge of its key runs;
+ * fp64 rescore}, prefill of at most 16 new tokens {preparation kernel (with the append);
+ * stream kernel; merge kernel; fp64 rescore}.  gqa_profile_read waits for the recorded events,
+ * returns the summed times of the first two stages and the number of calls recorded, and
+ * clears the record; gqa_profile_read_stages does the same for up to four stages (a path's
+ * missing stages read 0).  Not for the hot path: enabling creates the events.  No reference counterpart
  * (the reference's timing is its simulator's cycle count). */
 typedef struct gqa_profile {
     double kernel_ms[2];  /* summed durations of the call's first and second kernel */
@@ -293,7 +293,9 @@ int gqa_profile_read_stages(double* stage_ms, int32_t n_stages, int32_t* calls);
 /* Human-readable name of a status code. */
 const char* gqa_status_string(int status);
 
-/* ABI version: (major << 16) | minor. */
+/* ABI version: (major << 16) | minor.  It tells callers what of the declarations above they may
+ * rely on, but for gqa_decode_host_bf16 and gqa_decode_host_workspace_bytes: they came after 4.1
+ * without a new minor number, so a caller that may meet an older library looks the symbol up. */
 uint32_t gqa_abi_version(void);
 
 #ifdef __cplusplus
